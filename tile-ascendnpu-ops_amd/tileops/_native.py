@@ -23,6 +23,7 @@ __all__ = [
     "LIB_PATH",
     "check",
     "dtype_code",
+    "eager",
     "lib",
     "require_device",
     "stream_of",
@@ -153,10 +154,13 @@ def dtype_code(dtype: torch.dtype) -> int:
         raise ValueError(f"tileops HIP kernels do not support dtype {dtype}") from None
 
 
+_HIP = torch.version.hip is not None
+
+
 def require_device(*tensors: torch.Tensor) -> None:
     """Every tensor must live in HIP device memory (there is no host path)."""
     for t in tensors:
-        if t is not None and (not t.is_cuda or torch.version.hip is None):
+        if t is not None and not (_HIP and t.is_cuda):
             raise RuntimeError(
                 f"tileops HIP kernels need tensors on a ROCm GPU, got device {t.device}"
             )
@@ -164,4 +168,34 @@ def require_device(*tensors: torch.Tensor) -> None:
 
 def stream_of(t: torch.Tensor) -> int:
     """Raw hipStream_t of the current PyTorch stream on ``t``'s device."""
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
+
+
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def eager(*tensors: torch.Tensor) -> bool:
+    """True when a call on ``tensors`` may run its launch function directly
+    rather than through the ``torch.library`` custom op around it.
+
+    The custom op exists for everything that must see one opaque operator:
+    compilation and tracing, dispatch and function modes (fake tensors among
+    them), tensor subclasses, functorch transforms, forward-mode and
+    reverse-mode autograd.  A plain eager call is none of these and gets the
+    same result from the launch function; the dispatcher's Python round trip
+    costs it about 7 us (Argmax [4, 128]: 17.0 -> 9.8 us per call).
+    """
+    if (
+        torch.compiler.is_compiling()
+        or torch._C._get_tracing_state() is not None
+        or torch._C._len_torch_dispatch_stack()
+        or torch._C._len_torch_function_stack()
+        or torch._C._functorch.peek_interpreter_stack() is not None
+        or torch.autograd.forward_ad._current_level >= 0
+    ):
+        return False
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if type(t) not in _PLAIN or (grad and t.requires_grad):
+            return False
+    return True

@@ -21,8 +21,7 @@ from tileops.kernels.kernel_base import Kernel
 __all__ = ["GQAPrefillFwdKernel"]
 
 
-@torch.library.custom_op("tileops::gqa_prefill_fwd", mutates_args=())
-def _gqa_prefill_fwd(
+def _gqa_prefill_fwd_launch(
     batch: int,
     heads: int,
     heads_kv: int,
@@ -46,6 +45,9 @@ def _gqa_prefill_fwd(
     )
     _native.check(code, "tileops_mha_fwd")
     return o, lse
+
+
+_gqa_prefill_fwd = torch.library.custom_op("tileops::gqa_prefill_fwd", mutates_args=())(_gqa_prefill_fwd_launch)
 
 
 @_gqa_prefill_fwd.register_fake
@@ -127,15 +129,16 @@ class GQAPrefillFwdKernel(Kernel):
         _native.require_device(q, k, v)
         exp_q = (self.batch, self.seq_len_q, self.heads, self.dim)
         exp_kv = (self.batch, self.seq_len_kv, self.heads_kv, self.dim)
-        if tuple(q.shape) != exp_q:
+        if q.shape != exp_q:
             raise ValueError(f"Expected q.shape {exp_q}, got {tuple(q.shape)}")
         for name, t in (("k", k), ("v", v)):
-            if tuple(t.shape) != exp_kv:
+            if t.shape != exp_kv:
                 raise ValueError(f"Expected {name}.shape {exp_kv}, got {tuple(t.shape)}")
         for name, t in (("q", q), ("k", k), ("v", v)):
             if t.dtype != self.dtype:
                 raise ValueError(f"Expected {name}.dtype {self.dtype}, got {t.dtype}")
-        return _gqa_prefill_fwd(
+        fwd = _gqa_prefill_fwd_launch if _native.eager(q, k, v) else _gqa_prefill_fwd
+        return fwd(
             self.batch, self.heads, self.heads_kv, self.seq_len_q, self.seq_len_kv, self.dim,
             self.is_causal, self.sm_scale, self.softcap, q.contiguous(), k.contiguous(),
             v.contiguous(),

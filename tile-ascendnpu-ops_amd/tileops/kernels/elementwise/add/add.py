@@ -22,6 +22,9 @@ __all__ = ["AddFwdKernel", "BroadcastFwdKernel", "broadcast_strides", "MAX_DIMS"
 MAX_DIMS = 8
 
 
+_PLANS_KEPT = 64
+
+
 def broadcast_strides(t: torch.Tensor, out_shape: Sequence[int]) -> list:
     """Element strides of ``t`` over the dims of ``out_shape`` (right-aligned,
     as torch broadcasting aligns them), 0 where ``t`` is broadcast."""
@@ -48,6 +51,7 @@ class BroadcastFwdKernel(Kernel):
         self.N_total = int(N_total)
         self.dtype = dtype
         self.output_dtype = dtype
+        self._plans: dict = {}
         self.init_config(config)
 
     @property
@@ -61,6 +65,20 @@ class BroadcastFwdKernel(Kernel):
         _native.require_device(*tensors)
         for name, t in zip(names, tensors):
             self.check_tensor(name, t, dtype=self.dtype)
+        key = tuple((t.shape, t.stride()) for t in tensors)
+        plan = self._plans.get(key)
+        if plan is None:
+            plan = self._plan(tensors)
+            if len(self._plans) >= _PLANS_KEPT:
+                self._plans.clear()
+            self._plans[key] = plan
+        out_shape, nd, shape, strides = plan
+        y = torch.empty(out_shape, dtype=self.dtype, device=tensors[0].device)
+        return out_shape, y, nd, shape, strides
+
+    def _plan(self, tensors: Sequence[torch.Tensor]):
+        """The output shape and the host arrays of sizes and strides, which
+        depend on the operands' shapes and strides only."""
         out_shape = tuple(torch.broadcast_shapes(*(t.shape for t in tensors)))
         if len(out_shape) > MAX_DIMS:
             raise ValueError(f"{type(self).__name__} supports at most {MAX_DIMS} dims")
@@ -70,11 +88,10 @@ class BroadcastFwdKernel(Kernel):
         if n != self.N_total:
             raise ValueError(f"{type(self).__name__}: expected {self.N_total} output elements, "
                              f"got {n}")
-        y = torch.empty(out_shape, dtype=self.dtype, device=tensors[0].device)
         nd = len(out_shape)
         arr = ctypes.c_int64 * max(nd, 1)
         strides = [arr(*broadcast_strides(t, out_shape)) for t in tensors]
-        return out_shape, y, nd, arr(*out_shape), strides
+        return out_shape, nd, arr(*out_shape), strides
 
 
 class AddFwdKernel(BroadcastFwdKernel):

@@ -71,7 +71,7 @@ class Kernel(ABC):
         cls = self.__class__.__name__
         if dtype is not None and t.dtype != dtype:
             raise ValueError(f"{cls}: expected {name}.dtype {dtype}, got {t.dtype}")
-        if shape is not None and tuple(t.shape) != tuple(shape):
+        if shape is not None and t.shape != shape and tuple(t.shape) != tuple(shape):
             raise ValueError(
                 f"{cls}: expected {name}.shape {tuple(shape)}, got {tuple(t.shape)}")
         if numel is not None and t.numel() != numel:

@@ -21,8 +21,7 @@ from tileops.kernels.kernel_base import Kernel
 __all__ = ["GDNDecodeKernel"]
 
 
-@torch.library.custom_op("tileops::gdn_decode_fwd", mutates_args=())
-def _gdn_decode_fwd(
+def _gdn_decode_fwd_launch(
     B: int, H: int, DK: int, DV: int, scale: float,
     q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor, beta: torch.Tensor,
     state: torch.Tensor,
@@ -38,6 +37,9 @@ def _gdn_decode_fwd(
     )
     _native.check(code, "tileops_gdn_decode_fwd")
     return o, new_state
+
+
+_gdn_decode_fwd = torch.library.custom_op("tileops::gdn_decode_fwd", mutates_args=())(_gdn_decode_fwd_launch)
 
 
 @_gdn_decode_fwd.register_fake
@@ -111,9 +113,11 @@ class GDNDecodeKernel(Kernel):
             ("beta", beta, (B, H), torch.float32),
             ("state", state, (B, H, K, V), torch.float32),
         ):
-            if tuple(t.shape) != shape:
+            if t.shape != shape:
                 raise ValueError(f"Expected {name}.shape {shape}, got {tuple(t.shape)}")
             if t.dtype != dt:
                 raise ValueError(f"Expected {name}.dtype {dt}, got {t.dtype}")
         q, k, v, g, beta, state = (t.contiguous() for t in (q, k, v, g, beta, state))
-        return _gdn_decode_fwd(B, H, K, V, self.scale, q, k, v, g, beta, state)
+        fwd = (_gdn_decode_fwd_launch if _native.eager(q, k, v, g, beta, state)
+               else _gdn_decode_fwd)
+        return fwd(B, H, K, V, self.scale, q, k, v, g, beta, state)

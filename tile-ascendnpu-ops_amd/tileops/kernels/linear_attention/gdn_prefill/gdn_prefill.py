@@ -105,7 +105,7 @@ class GDNPrefillFwdKernel(Kernel):
             ("g", g, (B, T, H), torch.float32),
             ("beta", beta, (B, T, H), torch.float32),
         ):
-            if tuple(t.shape) != shape:
+            if t.shape != shape:
                 raise ValueError(f"Expected {name}.shape {shape}, got {tuple(t.shape)}")
             if t.dtype != dt:
                 raise ValueError(f"Expected {name}.dtype {dt}, got {t.dtype}")

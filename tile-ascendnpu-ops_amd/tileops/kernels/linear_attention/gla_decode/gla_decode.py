@@ -21,8 +21,7 @@ from tileops.kernels.kernel_base import Kernel
 __all__ = ["GLADecodeKernel"]
 
 
-@torch.library.custom_op("tileops::gla_decode_fwd", mutates_args=())
-def _gla_decode_fwd(
+def _gla_decode_fwd_launch(
     B: int, H: int, DK: int, DV: int, scale: float,
     q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gk: torch.Tensor, state: torch.Tensor,
 ) -> Tuple[torch.Tensor, torch.Tensor]:
@@ -35,6 +34,9 @@ def _gla_decode_fwd(
     )
     _native.check(code, "tileops_gla_decode_fwd")
     return o, new_state
+
+
+_gla_decode_fwd = torch.library.custom_op("tileops::gla_decode_fwd", mutates_args=())(_gla_decode_fwd_launch)
 
 
 @_gla_decode_fwd.register_fake
@@ -98,9 +100,10 @@ class GLADecodeKernel(Kernel):
         B, H, DK, DV = self.B, self.H, self.DK, self.DV
         for name, t, shape in (("q", q, (B, H, DK)), ("k", k, (B, H, DK)), ("v", v, (B, H, DV)),
                                ("gk", gk, (B, H, DK)), ("state", state, (B, H, DK, DV))):
-            if tuple(t.shape) != shape:
+            if t.shape != shape:
                 raise ValueError(f"Expected {name}.shape {shape}, got {tuple(t.shape)}")
             if t.dtype != self.dtype:
                 raise ValueError(f"Expected {name}.dtype {self.dtype}, got {t.dtype}")
         q, k, v, gk, state = (t.contiguous() for t in (q, k, v, gk, state))
-        return _gla_decode_fwd(B, H, DK, DV, self.scale, q, k, v, gk, state)
+        fwd = _gla_decode_fwd_launch if _native.eager(q, k, v, gk, state) else _gla_decode_fwd
+        return fwd(B, H, DK, DV, self.scale, q, k, v, gk, state)

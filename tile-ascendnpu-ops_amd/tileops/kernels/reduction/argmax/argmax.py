@@ -19,8 +19,7 @@ __all__ = ["ArgreduceKernel"]
 _ARGREDUCE_KINDS = {"argmax", "argmin"}
 
 
-@torch.library.custom_op("tileops::argreduce_fwd", mutates_args=())
-def _argreduce_fwd(M: int, N: int, op_kind: str, x: torch.Tensor) -> torch.Tensor:
+def _argreduce_fwd_launch(M: int, N: int, op_kind: str, x: torch.Tensor) -> torch.Tensor:
     y = torch.empty((M,), dtype=torch.int64, device=x.device)
     code = _native.lib().tileops_argreduce_fwd(
         x.data_ptr(),
@@ -33,6 +32,9 @@ def _argreduce_fwd(M: int, N: int, op_kind: str, x: torch.Tensor) -> torch.Tenso
     )
     _native.check(code, "tileops_argreduce_fwd")
     return y
+
+
+_argreduce_fwd = torch.library.custom_op("tileops::argreduce_fwd", mutates_args=())(_argreduce_fwd_launch)
 
 
 @_argreduce_fwd.register_fake
@@ -89,4 +91,6 @@ class ArgreduceKernel(Kernel):
         _native.require_device(x)
         self.check_tensor("x", x, dtype=self.dtype, shape=(self.M, self.N))
         x = x.contiguous()
+        if _native.eager(x):
+            return _argreduce_fwd_launch(self.M, self.N, self.op_kind, x)
         return _argreduce_fwd(self.M, self.N, self.op_kind, x)

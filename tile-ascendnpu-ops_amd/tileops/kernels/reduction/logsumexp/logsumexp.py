@@ -19,14 +19,16 @@ from tileops.kernels.kernel_base import Kernel
 __all__ = ["LogSumExpKernel"]
 
 
-@torch.library.custom_op("tileops::logsumexp_fwd", mutates_args=())
-def _logsumexp_fwd(M: int, N: int, x: torch.Tensor) -> torch.Tensor:
+def _logsumexp_fwd_launch(M: int, N: int, x: torch.Tensor) -> torch.Tensor:
     y = torch.empty((M,), dtype=x.dtype, device=x.device)
     code = _native.lib().tileops_logsumexp_fwd(
         x.data_ptr(), y.data_ptr(), M, N, _native.dtype_code(x.dtype), _native.stream_of(x)
     )
     _native.check(code, "tileops_logsumexp_fwd")
     return y
+
+
+_logsumexp_fwd = torch.library.custom_op("tileops::logsumexp_fwd", mutates_args=())(_logsumexp_fwd_launch)
 
 
 @_logsumexp_fwd.register_fake
@@ -79,4 +81,6 @@ class LogSumExpKernel(Kernel):
         _native.require_device(x)
         self.check_tensor("x", x, dtype=self.dtype, shape=(self.M, self.N))
         x = x.contiguous()
+        if _native.eager(x):
+            return _logsumexp_fwd_launch(self.M, self.N, x)
         return _logsumexp_fwd(self.M, self.N, x)

@@ -58,7 +58,7 @@ class GatedActivationOp(Op):
             raise ValueError(f"x must be a {backend.name} tensor, got device {x.device}")
         if x.dtype != self.dtype:
             raise ValueError(f"Expected x.dtype {self.dtype}, got {x.dtype}")
-        if tuple(x.shape) != self.x_shape:
+        if x.shape != self.x_shape:
             raise ValueError(f"Expected x.shape {self.x_shape}, got {tuple(x.shape)}")
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:

@@ -65,7 +65,7 @@ class AddFwdOp(Op):
                                   ("other", other, self.other_shape)):
             if t.dtype != self.dtype:
                 raise ValueError(f"Expected {name}.dtype {self.dtype}, got {t.dtype}")
-            if tuple(t.shape) != expected:
+            if t.shape != expected:
                 raise ValueError(f"Expected {name}.shape {expected}, got {tuple(t.shape)}")
         return self.kernel(input, other)
 

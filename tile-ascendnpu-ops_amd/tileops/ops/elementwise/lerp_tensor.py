@@ -72,7 +72,7 @@ class LerpTensorFwdOp(Op):
                                   ("weight", weight, self.weight_shape)):
             if t.dtype != self.dtype:
                 raise ValueError(f"Expected {name}.dtype {self.dtype}, got {t.dtype}")
-            if tuple(t.shape) != expected:
+            if t.shape != expected:
                 raise ValueError(f"Expected {name}.shape {expected}, got {tuple(t.shape)}")
         return self.kernel(input, end, weight)
 

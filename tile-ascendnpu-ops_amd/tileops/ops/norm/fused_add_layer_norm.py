@@ -105,18 +105,18 @@ class FusedAddLayerNormFwdOp(Op):
         if residual.shape != x.shape:
             raise ValueError(f"Expected residual shape {x.shape}, got {residual.shape}")
         N = x.shape[-1]
-        if tuple(weight.shape) != (N,):
+        if weight.shape != (N,):
             raise ValueError(f"Expected weight shape {(N,)}, got {tuple(weight.shape)}")
-        if tuple(bias.shape) != (N,):
+        if bias.shape != (N,):
             raise ValueError(f"Expected bias shape {(N,)}, got {tuple(bias.shape)}")
         if self._committed_N is not None and self._committed_N != N:
             raise ValueError(f"Expected hidden dim {self._committed_N}, got {N}")
 
         orig_shape = x.shape
-        x = x.contiguous().reshape(-1, N)
-        residual = residual.contiguous().reshape(-1, N)
-        weight = weight.contiguous().reshape(N)
-        bias = bias.contiguous().reshape(N)
+        x, residual = x.contiguous(), residual.contiguous()
+        if x.dim() != 2:
+            x, residual = x.reshape(-1, N), residual.reshape(-1, N)
+        weight, bias = weight.contiguous(), bias.contiguous()
         M_actual = x.shape[0]
         if self._committed_M is not None and M_actual != self._committed_M:
             raise ValueError(
@@ -130,4 +130,6 @@ class FusedAddLayerNormFwdOp(Op):
         y, residual_out = kernel(x, residual, weight, bias)
         self._last_roofline_mn = (M_actual, N)
         self._last_param_bytes = weight.dtype.itemsize
-        return y.reshape(orig_shape), residual_out.reshape(orig_shape)
+        if y.shape != orig_shape:
+            y, residual_out = y.reshape(orig_shape), residual_out.reshape(orig_shape)
+        return y, residual_out

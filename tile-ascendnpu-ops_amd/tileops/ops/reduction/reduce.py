@@ -132,7 +132,9 @@ class _ReduceOpBase(Op):
         self._last_roofline_mn = (M, N)
         if dim != x.ndim - 1:
             x = x.movedim(dim, -1)
-        x = x.contiguous().reshape(M, N)
+        x = x.contiguous()
+        if x.dim() != 2:
+            x = x.reshape(M, N)
         return x, orig_shape, dim, self._get_or_create_kernel(M, N)
 
     def _reshape_output(self, y: torch.Tensor, orig_shape: torch.Size, dim_info) -> torch.Tensor:
@@ -144,4 +146,6 @@ class _ReduceOpBase(Op):
             shape[dim] = 1
             return y.reshape(shape)
         shape = [s for i, s in enumerate(orig_shape) if i != dim]
+        if len(shape) == 1 and y.dim() == 1:
+            return y
         return y.squeeze() if not shape else y.reshape(shape)

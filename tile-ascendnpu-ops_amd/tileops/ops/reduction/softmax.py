@@ -119,7 +119,9 @@ class LogSumExpFwdOp(Op):
         moved = d != x.ndim - 1
         if moved:
             x = x.movedim(d, -1)
-        x = x.contiguous().reshape(M, N)
+        x = x.contiguous()
+        if x.dim() != 2:
+            x = x.reshape(M, N)
         kernel = self._get_or_create_kernel(M, N, x.dtype, x.device.index)
         self.kernel = kernel
         y = kernel(x)
@@ -128,6 +130,8 @@ class LogSumExpFwdOp(Op):
             shape[d] = 1
             return y.reshape(shape)
         shape = [s for i, s in enumerate(orig_shape) if i != d]
+        if len(shape) == 1 and y.dim() == 1:
+            return y
         return y.squeeze() if not shape else y.reshape(shape)
 
     def eval_roofline(self) -> tuple[int, int]:
