@@ -47,6 +47,13 @@ enum tileops_predicate {
   TILEOPS_ISFINITE = 2,
 };
 
+/* Row reduction selector for tileops_reduce_fwd. */
+enum tileops_reduce_op {
+  TILEOPS_LOGSUMEXP = 0,
+  TILEOPS_ARGMAX = 1,
+  TILEOPS_ARGMIN = 2,
+};
+
 /* Flags for tileops_unary_fwd (TILEOPS_CLAMP only). */
 #define TILEOPS_CLAMP_HAS_MIN 1
 #define TILEOPS_CLAMP_HAS_MAX 2
@@ -183,6 +190,19 @@ int tileops_logsumexp_fwd(const void* x, void* y, int64_t M, int64_t N, int dtyp
  */
 int tileops_argreduce_fwd(const void* x, int64_t* y, int64_t M, int64_t N, int dtype,
                           int is_min, void* stream);
+
+/*
+ * The reductions of tileops_logsumexp_fwd / tileops_argreduce_fwd (`op`:
+ * enum tileops_reduce_op) with caller scratch: long rows that are too few to
+ * fill the device are split over workgroups, whose partial results
+ * (tileops_reduce_workspace_bytes, 0 where no split is planned) go to `ws`
+ * (16-byte aligned) and are merged by a second launch.  With `ws` NULL or
+ * smaller than that the rows run unsplit, as in the two functions above; the
+ * result is the same up to the order of the fp32 sums.
+ */
+size_t tileops_reduce_workspace_bytes(int64_t M, int64_t N, int dtype);
+int tileops_reduce_fwd(int op, const void* x, void* y, int64_t M, int64_t N, int dtype, void* ws,
+                       size_t ws_bytes, void* stream);
 
 /*
  * Flash attention forward, BSHD layout.

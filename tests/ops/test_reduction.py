@@ -254,3 +254,38 @@ def test_argreduce_kernel_contract():
         ArgreduceKernel(4, 4, "argsort", torch.float32)
     with pytest.raises(ValueError, match="empty"):
         ArgreduceKernel(4, 0, "argmax", torch.float32)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M, N, dtype", [
+    (1, 600000, torch.float32),    # several workgroups per row, merged
+    (128, 131073, torch.float16),  # the most rows that split, odd length
+    (129, 131073, torch.float16),  # one 16-wavefront workgroup per row
+    (512, 16384, torch.float32),   # sixteen wavefronts per row
+    (513, 16381, torch.bfloat16),  # four
+    (3072, 1027, torch.bfloat16),  # one
+    (5, 3, torch.float16),         # short rows: elements, 4 lanes each
+    (1001, 13, torch.bfloat16),    # 16
+    (70, 64, torch.float32),       # packs, 16 lanes
+    (9, 17, torch.float16),        # ragged packs, 16 lanes
+    (600, 131, torch.float32),     # 32
+    (77, 519, torch.float16),      # 64 packs and both edges
+    (5000, 512, torch.float16),    # packs, 64 lanes
+    (6, 521, torch.bfloat16),      # the shortest ragged row past them
+])
+def test_row_split_and_ragged_rows(M, N, dtype):
+    # extremes at the row's first and last elements and around the first and
+    # last aligned pack: each must be seen exactly once by the plan
+    x = torch.randn(M, N, device="cuda").to(dtype)
+    rows = torch.arange(M, device="cuda")
+    where = torch.tensor([0, N - 1, min(7, N - 1), max(0, N - 8), N // 2], device="cuda")
+    x[rows, where[rows % 5]] = 30.0
+    x[0, N // 3] = float("nan")
+    got = ArgmaxFwdOp(dtype=dtype, dim=-1)(x)
+    assert torch.equal(got.cpu(), torch.argmax(x.cpu(), dim=-1))
+    # fp32 sums of N positive terms: N eps relative in the sum, far below
+    # atol on its logarithm
+    x[0, N // 3] = 0.0
+    y = LogSumExpFwdOp(dtype=dtype)(x)
+    atol, rtol = ref_tolerance(dtype)
+    assert_close_np(to_np(y), torch.logsumexp(x.double(), -1).cpu().numpy(), atol, rtol, "lse")

@@ -1,12 +1,15 @@
 // Row reductions for gfx950: LogSumExp and Argmax / Argmin over the last
 // dimension of a row-major [M, N] tensor.
 //
-// Work split: a wavefront owns a row (WPR = 1, four rows per 256-thread
-// workgroup) when there are enough rows to fill the chip; otherwise the four
-// wavefronts of a workgroup share one row (WPR = 4) and meet in LDS.  Inside
-// a wavefront every lane streams 16-byte packs (64 lanes x one pack = one
-// contiguous "chunk" of the row), keeps UNROLL packs in flight, folds them
-// into a per-lane partial, and the 64 partials meet in a shuffle butterfly.
+// A wavefront streams its share of a row in 16-byte packs, UNROLL packs per
+// lane in flight, folds them into a per-lane partial, and the 64 partials meet
+// in a shuffle butterfly.  What bounds the kernel is HBM where the rows fill
+// the chip, and the latency of one wavefront's chain of loads where they do
+// not, so the number of wavefronts per row follows the row count (plan_rows):
+// 1 (four rows per workgroup), 4, 16 (a 1024-thread workgroup), or several
+// 16-wavefront workgroups per row whose partials a second launch merges.
+#include <algorithm>
+
 #include <float.h>
 
 #include "common.h"
@@ -68,9 +71,11 @@ __device__ __forceinline__ void lse_fold(LseState& st, const float (&v)[CNT]) {
   st.s = acc;
 }
 
+// Merged over aligned groups of G lanes.
+template <int G>
 __device__ __forceinline__ LseState lse_wave(LseState st) {
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
+  for (int o = G / 2; o > 0; o >>= 1) {
     LseState other{__shfl_xor(st.m, o, 64), __shfl_xor(st.s, o, 64)};
     st = lse_merge(st, other);
   }
@@ -111,10 +116,10 @@ __device__ __forceinline__ void arg_step(ArgState& st, float a, int i) {
   st.i = take ? i : st.i;
 }
 
-template <bool IS_MIN>
+template <bool IS_MIN, int G>
 __device__ __forceinline__ ArgState arg_wave(ArgState st) {
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
+  for (int o = G / 2; o > 0; o >>= 1) {
     ArgState other{__shfl_xor(st.v, o, 64), __shfl_xor(st.i, o, 64)};
     if (arg_better<IS_MIN>(other.v, other.i, st.v, st.i)) st = other;
   }
@@ -122,9 +127,7 @@ __device__ __forceinline__ ArgState arg_wave(ArgState st) {
 }
 
 // ---------------------------------------------------------------------------
-// Shared row driver.  OP 0 = logsumexp, 1 = argmax, 2 = argmin.
-// VEC: the row base is 16-byte aligned and N % kVec == 0, so packs are used;
-// otherwise every lane reads one element per chunk.
+// OP 0 = logsumexp, 1 = argmax, 2 = argmin.
 // ---------------------------------------------------------------------------
 template <int OP> struct RowState;
 template <> struct RowState<0> { typedef LseState S; };
@@ -144,63 +147,97 @@ __device__ __forceinline__ typename RowState<OP>::S row_merge(typename RowState<
   else return arg_better<OP == 2>(b.v, b.i, a.v, a.i) ? b : a;
 }
 
-template <int OP>
+template <int OP, int G = 64>
 __device__ __forceinline__ typename RowState<OP>::S row_wave(typename RowState<OP>::S st) {
-  if constexpr (OP == 0) return lse_wave(st);
-  else return arg_wave<OP == 2>(st);
+  if constexpr (OP == 0) return lse_wave<G>(st);
+  else return arg_wave<OP == 2, G>(st);
 }
 
-template <typename T, int OP, int WPR, int UNROLL, bool VEC>
-__global__ __launch_bounds__(256) void row_reduce_kernel(const T* __restrict__ x,
-                                                         void* __restrict__ out, int64_t M,
-                                                         int64_t N) {
+template <typename T, int OP>
+__device__ __forceinline__ void row_store(void* out, int64_t row, typename RowState<OP>::S st) {
+  if constexpr (OP == 0) static_cast<T*>(out)[row] = Elem<T>::from_f32(lse_final(st));
+  else static_cast<int64_t*>(out)[row] = st.i < 0 ? 0 : (int64_t)st.i;
+}
+
+// WPR wavefronts of one workgroup share a row, and `nsplit` workgroups; a
+// wavefront takes every (WPR * nsplit)-th chunk of 64 packs, U of them in
+// flight per step.  ALIGNED: every row starts on a 16-byte boundary and holds
+// whole packs.  Otherwise the row's packs start at its first aligned element;
+// the row's first wavefront folds the elements before them in its first step
+// and those after them in its last, one per lane,
+// so that an odd row length costs no more loads than an even one (LogSumExp
+// bf16 16384 x 4097: 73.9 us with one element per lane and load, 34.8 so).
+// With nsplit > 1 `out` holds nsplit partials per row.
+template <typename T, int OP, int WPR, int U, bool ALIGNED>
+__global__ __launch_bounds__(WPR > 4 ? 64 * WPR : 256) void row_reduce_kernel(
+    const T* __restrict__ x, void* __restrict__ out, int64_t M, int64_t N, int nstep, int nsplit) {
   typedef typename RowState<OP>::S S;
-  constexpr int V = VEC ? Elem<T>::kVec : 1;
-  constexpr int ROWS_PER_BLOCK = 4 / WPR;
+  constexpr int V = Elem<T>::kVec;
+  constexpr int WPB = WPR > 4 ? WPR : 4;  // wavefronts per workgroup
+  constexpr int ROWS_PER_BLOCK = WPB / WPR;
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wave_in_row = wave % WPR;
-  const int row_in_block = wave / WPR;
-  const int64_t chunk = 64 * V;                 // elements per wave step
-  const int64_t nchunk = (N + chunk - 1) / chunk;
+  const int64_t ngroup = (M + ROWS_PER_BLOCK - 1) / ROWS_PER_BLOCK * nsplit;
 
-  __shared__ S part[4];
+  __shared__ S part[WPB];
 
-  for (int64_t row0 = (int64_t)blockIdx.x * ROWS_PER_BLOCK; row0 < M;
-       row0 += (int64_t)gridDim.x * ROWS_PER_BLOCK) {
-    const int64_t row = row0 + row_in_block;
+  for (int64_t group = blockIdx.x; group < ngroup; group += gridDim.x) {
+    const int split = nsplit == 1 ? 0 : (int)(group % nsplit);
+    const int64_t row = (nsplit == 1 ? group : group / nsplit) * ROWS_PER_BLOCK + wave / WPR;
     S st = row_init<OP>();
     if (row < M) {
       const T* xr = x + row * N;
-      for (int64_t c0 = wave_in_row; c0 < nchunk; c0 += (int64_t)WPR * UNROLL) {
-        float vals[UNROLL][V];
-        int64_t base[UNROLL];
+      int64_t head = 0;
+      if constexpr (!ALIGNED) {
+        const uint32_t mis = (uint32_t)(reinterpret_cast<uintptr_t>(xr) & 15u);
+        head = min((int64_t)((16u - mis) & 15u) / (int64_t)sizeof(T), N);
+      }
+      const int64_t np = (N - head) / V;
+      const T* xb = xr + head;
+      const int gw = split * WPR + wave_in_row, nw = nsplit * WPR;
+      for (int k = 0; k < nstep; ++k) {
+        // Slots past the row read as -inf: they add exp(-inf) = 0 to a sum
+        // and are skipped by the arg-reduction below.
+        constexpr int EDGE = ALIGNED ? 0 : 2;
+        float vals[U * V + EDGE];
+        int64_t base[U];
 #pragma unroll
-        for (int u = 0; u < UNROLL; ++u) {
-          base[u] = (c0 + (int64_t)u * WPR) * chunk + (int64_t)lane * V;
-          // Out-of-row slots read as -inf: they add exp(-inf) = 0 to a sum
-          // and are skipped by the arg-reduction below.
+        for (int u = 0; u < U; ++u) {
+          base[u] = ((int64_t)(k * U + u) * nw + gw) * 64 + lane;
 #pragma unroll
-          for (int e = 0; e < V; ++e) vals[u][e] = -INFINITY;
-          if constexpr (VEC) {
-            if (base[u] < N) {
-              Pack<T> p = load_pack_nt(xr + base[u]);
+          for (int e = 0; e < V; ++e) vals[u * V + e] = -INFINITY;
+          if (base[u] < np) {
+            const Pack<T> p = load_pack_nt(xb + base[u] * V);
 #pragma unroll
-              for (int e = 0; e < V; ++e) vals[u][e] = Elem<T>::to_f32(p.v[e]);
-            }
-          } else {
-            if (base[u] < N) vals[u][0] = Elem<T>::to_f32(xr[base[u]]);
+            for (int e = 0; e < V; ++e) vals[u * V + e] = Elem<T>::to_f32(p.v[e]);
           }
         }
+        bool first = false, last = false;
+        const int64_t t = head + np * V + lane;
+        if constexpr (!ALIGNED) {
+          first = gw == 0 && k == 0 && lane < (int)head;
+          last = gw == 0 && k == nstep - 1 && t < N;
+          vals[U * V] = vals[U * V + 1] = -INFINITY;
+          if (first) vals[U * V] = Elem<T>::to_f32(xr[lane]);
+          if (last) vals[U * V + 1] = Elem<T>::to_f32(xr[t]);
+        }
         if constexpr (OP == 0) {
-          lse_fold<UNROLL * V>(st, reinterpret_cast<const float(&)[UNROLL * V]>(vals));
+          lse_fold<U * V + EDGE>(st, vals);
         } else {
+          if constexpr (!ALIGNED) {
+            if (first) arg_step<OP == 2>(st, vals[U * V], lane);
+          }
 #pragma unroll
-          for (int u = 0; u < UNROLL; ++u) {
-            if (base[u] < N) {
+          for (int u = 0; u < U; ++u) {
+            if (base[u] < np) {
 #pragma unroll
-              for (int e = 0; e < V; ++e) arg_step<OP == 2>(st, vals[u][e], (int)(base[u] + e));
+              for (int e = 0; e < V; ++e)
+                arg_step<OP == 2>(st, vals[u * V + e], (int)(head + base[u] * V + e));
             }
+          }
+          if constexpr (!ALIGNED) {
+            if (last) arg_step<OP == 2>(st, vals[U * V + 1], (int)t);
           }
         }
       }
@@ -209,50 +246,217 @@ __global__ __launch_bounds__(256) void row_reduce_kernel(const T* __restrict__ x
     if constexpr (WPR > 1) {
       if (lane == 0) part[wave] = st;
       __syncthreads();
-      if (wave == 0) {
-        st = part[0];
+      if constexpr (WPR > 4) {
+        if (wave == 0) st = row_wave<OP, WPR>(part[lane % WPR]);
+      } else {
+        if (wave == 0) {
+          st = part[0];
 #pragma unroll
-        for (int w = 1; w < WPR; ++w) st = row_merge<OP>(st, part[w]);
+          for (int w = 1; w < WPR; ++w) st = row_merge<OP>(st, part[w]);
+        }
       }
       __syncthreads();
     }
     if (lane == 0 && wave_in_row == 0 && row < M) {
-      if constexpr (OP == 0) {
-        static_cast<T*>(out)[row] = Elem<T>::from_f32(lse_final(st));
-      } else {
-        static_cast<int64_t*>(out)[row] = st.i < 0 ? 0 : (int64_t)st.i;
-      }
+      if (nsplit > 1) static_cast<S*>(out)[row * nsplit + split] = st;
+      else row_store<T, OP>(out, row, st);
     }
   }
 }
 
+// Short rows: G lanes per row, one load per lane, 64 / G rows per wavefront, so
+// that a row costs log2 G merges instead of six and no lane group idles (one
+// wavefront per row and this, us: Argmax fp16 524288 x 4: 120 -> 6.8,
+// LogSumExp bf16 88000 x 128: 50 -> 8.9).  PACKS: a lane takes one pack;
+// ragged rows as in row_reduce_kernel (G >= 16 lanes hold the elements before
+// and after the packs).  Otherwise a lane takes one element.
+template <typename T, int OP, int G, bool PACKS, bool ALIGNED>
+__global__ __launch_bounds__(256) void short_row_kernel(const T* __restrict__ x,
+                                                        void* __restrict__ out, int64_t M, int N) {
+  constexpr int V = PACKS ? Elem<T>::kVec : 1, EDGE = PACKS && !ALIGNED ? 2 : 0;
+  static_assert(EDGE == 0 || G >= Elem<T>::kVec, "a lane per edge element");
+  const int64_t row = (int64_t)blockIdx.x * (256 / G) + threadIdx.x / G;
+  const int lane = threadIdx.x % G;
+  typename RowState<OP>::S st = row_init<OP>();
+  if (row < M) {
+    const T* xr = x + row * N;
+    int head = 0;
+    if constexpr (EDGE > 0) {
+      const uint32_t mis = (uint32_t)(reinterpret_cast<uintptr_t>(xr) & 15u);
+      head = min((int)(((16u - mis) & 15u) / sizeof(T)), N);
+    }
+    const int np = (N - head) / V, t = head + np * V + lane;
+    float vals[V + EDGE];
+#pragma unroll
+    for (int e = 0; e < V + EDGE; ++e) vals[e] = -INFINITY;
+    if (lane < np) {
+      if constexpr (PACKS) {
+        const Pack<T> p = load_pack_nt(xr + head + lane * V);
+#pragma unroll
+        for (int e = 0; e < V; ++e) vals[e] = Elem<T>::to_f32(p.v[e]);
+      } else {
+        vals[0] = Elem<T>::to_f32(xr[lane]);
+      }
+    }
+    if constexpr (EDGE > 0) {
+      if (lane < head) vals[V] = Elem<T>::to_f32(xr[lane]);
+      if (t < N) vals[V + 1] = Elem<T>::to_f32(xr[t]);
+    }
+    if constexpr (OP == 0) {
+      lse_fold<V + EDGE>(st, vals);
+    } else {
+      if constexpr (EDGE > 0) {
+        if (lane < head) arg_step<OP == 2>(st, vals[V], lane);
+      }
+      if (lane < np) {
+#pragma unroll
+        for (int e = 0; e < V; ++e) arg_step<OP == 2>(st, vals[e], head + lane * V + e);
+      }
+      if constexpr (EDGE > 0) {
+        if (t < N) arg_step<OP == 2>(st, vals[V + 1], t);
+      }
+    }
+  }
+  st = row_wave<OP, G>(st);
+  if (row < M && lane == 0) row_store<T, OP>(out, row, st);
+}
+
+// The nsplit partials of each output, one wavefront per output.
 template <typename T, int OP>
-static int launch_row_reduce(const void* xv, void* out, int64_t M, int64_t N, hipStream_t s) {
-  const T* x = static_cast<const T*>(xv);
-  const bool vec = host_aligned16(x) && (N % Elem<T>::kVec) == 0;
-  // Enough rows to give every CU a dozen wavefronts: one row per wavefront.
-  const bool wide = M < 256 * 12;
-  const int rows_per_block = wide ? 1 : 4;
-  int64_t blocks = (M + rows_per_block - 1) / rows_per_block;
-  if (blocks > 256 * 32) blocks = 256 * 32;
-  dim3 grid((unsigned)blocks), block(256);
-  if (vec) {
-    if (wide) row_reduce_kernel<T, OP, 4, 4, true><<<grid, block, 0, s>>>(x, out, M, N);
-    else row_reduce_kernel<T, OP, 1, 4, true><<<grid, block, 0, s>>>(x, out, M, N);
+__global__ __launch_bounds__(256) void merge_partials_kernel(
+    const typename RowState<OP>::S* __restrict__ part, void* __restrict__ out, int64_t M,
+    int nsplit) {
+  const int lane = threadIdx.x & 63;
+  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= M) return;
+  typename RowState<OP>::S st = row_init<OP>();
+  for (int i = lane; i < nsplit; i += 64) st = row_merge<OP>(st, part[row * nsplit + i]);
+  st = row_wave<OP>(st);
+  if (lane == 0) row_store<T, OP>(out, row, st);
+}
+
+// How a [M, N] row reduction is laid out.  One wavefront per row from 3072
+// rows up (a dozen wavefronts per CU), four below, sixteen where at most 512
+// rows leave each of those work (LogSumExp bf16 512 x 32768: 14.2 us with
+// four, 11.1 with sixteen; 1024 rows: 18.6 and 19.5).  At most 128 rows (two
+// CUs each) of 256 chunks or more (sixteen wavefronts would take four steps
+// and more, ~2 us each) are split over workgroups of four wavefronts, one
+// step each up to 1024 workgroups; the merge launch and its scratch cost ~2.5
+// us on the GPU and ~4 us of an eager call's host time, so shorter rows stay
+// whole (LogSumExp bf16 4 x 102400: 17.5 us with four wavefronts per row, 9.8
+// with sixteen, 6.3 split, but 10.4 and 14.6 us per eager call; Argmax of 2^21
+// fp16 elements 682 -> 9.7 us, of 2^25 fp32 9222 -> 32).
+// A wavefront keeps 4 packs per lane in flight, fewer where its whole share of
+// the row is less (slots past the row still cost their exponentials).
+struct RowPlan {
+  int wpr, u, nsplit, nstep;
+};
+static RowPlan plan_rows(int64_t M, int64_t N, int vec) {
+  const int64_t chunks = std::max<int64_t>((N / vec + 63) / 64, 1);
+  RowPlan p{4, 4, 1, 0};
+  if (M >= 256 * 12) p.wpr = 1;
+  else if (M <= 512 && chunks >= 16 * 4) p.wpr = 16;
+  if (M <= 128 && chunks >= 16 * 16) {
+    p.wpr = 4;
+    p.nsplit = (int)std::min<int64_t>((chunks + 15) / 16, 1024 / M);
+  }
+  if (p.wpr <= 4 && p.nsplit == 1) p.u = (int)std::min<int64_t>((chunks + p.wpr - 1) / p.wpr, 4);
+  const int64_t per_step = (int64_t)p.u * p.wpr * p.nsplit;
+  p.nstep = (int)((chunks + per_step - 1) / per_step);
+  return p;
+}
+
+template <typename T, int OP, int WPR, int U>
+static void launch_rows(const T* x, void* out, int64_t M, int64_t N, const RowPlan& p,
+                        hipStream_t s) {
+  const bool aligned = host_aligned16(x) && (N % Elem<T>::kVec) == 0;
+  const int rows_per_block = WPR > 4 ? 1 : 4 / WPR;
+  const int64_t blocks = (M + rows_per_block - 1) / rows_per_block * p.nsplit;
+  const dim3 grid((unsigned)std::min<int64_t>(blocks, 256 * 32)), block(WPR > 4 ? 64 * WPR : 256);
+  if (aligned)
+    row_reduce_kernel<T, OP, WPR, U, true><<<grid, block, 0, s>>>(x, out, M, N, p.nstep, p.nsplit);
+  else
+    row_reduce_kernel<T, OP, WPR, U, false><<<grid, block, 0, s>>>(x, out, M, N, p.nstep, p.nsplit);
+}
+
+template <typename T, int OP, int WPR>
+static void launch_rows_u(const T* x, void* out, int64_t M, int64_t N, const RowPlan& p,
+                          hipStream_t s) {
+  if (p.u == 1) launch_rows<T, OP, WPR, 1>(x, out, M, N, p, s);
+  else if (p.u == 2) launch_rows<T, OP, WPR, 2>(x, out, M, N, p, s);
+  else if (p.u == 3) launch_rows<T, OP, WPR, 3>(x, out, M, N, p, s);
+  else launch_rows<T, OP, WPR, 4>(x, out, M, N, p, s);
+}
+
+// The short-row kernel where it applies: rows of at most 64 packs.  Ragged
+// rows of up to 16 elements go element by element.
+template <typename T, int OP>
+static bool try_short(const T* x, void* out, int64_t M, int64_t N, hipStream_t s) {
+  constexpr int V = Elem<T>::kVec;
+  if (N / V > 64 || M > (int64_t)INT32_MAX) return false;  // four rows per workgroup at worst
+  const int n = (int)N, np = n / V;
+  const dim3 block(256);
+  auto grid = [&](int G) { return dim3((unsigned)((M + 256 / G - 1) / (256 / G))); };
+  if (host_aligned16(x) && n % V == 0) {
+    if (np <= 4) short_row_kernel<T, OP, 4, true, true><<<grid(4), block, 0, s>>>(x, out, M, n);
+    else if (np <= 16) short_row_kernel<T, OP, 16, true, true><<<grid(16), block, 0, s>>>(x, out, M, n);
+    else if (np <= 32) short_row_kernel<T, OP, 32, true, true><<<grid(32), block, 0, s>>>(x, out, M, n);
+    else short_row_kernel<T, OP, 64, true, true><<<grid(64), block, 0, s>>>(x, out, M, n);
+  } else if (n <= 16) {
+    if (n <= 4) short_row_kernel<T, OP, 4, false, false><<<grid(4), block, 0, s>>>(x, out, M, n);
+    else short_row_kernel<T, OP, 16, false, false><<<grid(16), block, 0, s>>>(x, out, M, n);
   } else {
-    if (wide) row_reduce_kernel<T, OP, 4, 8, false><<<grid, block, 0, s>>>(x, out, M, N);
-    else row_reduce_kernel<T, OP, 1, 8, false><<<grid, block, 0, s>>>(x, out, M, N);
+    if (np <= 16) short_row_kernel<T, OP, 16, true, false><<<grid(16), block, 0, s>>>(x, out, M, n);
+    else if (np <= 32) short_row_kernel<T, OP, 32, true, false><<<grid(32), block, 0, s>>>(x, out, M, n);
+    else short_row_kernel<T, OP, 64, true, false><<<grid(64), block, 0, s>>>(x, out, M, n);
+  }
+  return true;
+}
+
+template <typename T, int OP>
+static int launch_row_reduce(const void* xv, void* out, int64_t M, int64_t N, void* ws,
+                             size_t ws_bytes, hipStream_t s) {
+  typedef typename RowState<OP>::S S;
+  const T* x = static_cast<const T*>(xv);
+  if (try_short<T, OP>(x, out, M, N, s)) return launch_status();
+  RowPlan p = plan_rows(M, N, Elem<T>::kVec);
+  if (p.nsplit > 1 && ws_bytes < (size_t)M * p.nsplit * sizeof(S)) p.nsplit = 1;  // no scratch
+  void* dst = p.nsplit > 1 ? ws : out;
+  if (p.wpr == 1) launch_rows_u<T, OP, 1>(x, dst, M, N, p, s);
+  else if (p.wpr == 4) launch_rows_u<T, OP, 4>(x, dst, M, N, p, s);
+  else launch_rows<T, OP, 16, 4>(x, dst, M, N, p, s);
+  if (p.nsplit > 1) {
+    if (int e = launch_status()) return e;
+    merge_partials_kernel<T, OP><<<dim3((unsigned)((M + 3) / 4)), dim3(256), 0, s>>>(
+        static_cast<const S*>(ws), out, M, p.nsplit);
   }
   return launch_status();
 }
 
 template <int OP>
-static int dispatch_row_reduce(const void* x, void* out, int64_t M, int64_t N, int dtype,
-                               hipStream_t s) {
+static int dispatch_row_reduce(const void* x, void* out, int64_t M, int64_t N, int dtype, void* ws,
+                               size_t ws_bytes, hipStream_t s) {
   switch (dtype) {
-    case TILEOPS_F32: return launch_row_reduce<float, OP>(x, out, M, N, s);
-    case TILEOPS_F16: return launch_row_reduce<f16, OP>(x, out, M, N, s);
-    case TILEOPS_BF16: return launch_row_reduce<bf16, OP>(x, out, M, N, s);
+    case TILEOPS_F32: return launch_row_reduce<float, OP>(x, out, M, N, ws, ws_bytes, s);
+    case TILEOPS_F16: return launch_row_reduce<f16, OP>(x, out, M, N, ws, ws_bytes, s);
+    case TILEOPS_BF16: return launch_row_reduce<bf16, OP>(x, out, M, N, ws, ws_bytes, s);
+  }
+  return TILEOPS_EINVAL;
+}
+
+// Checks and dispatch shared by the entry points.
+static int reduce_rows(int op, const void* x, void* y, int64_t M, int64_t N, int dtype, void* ws,
+                       size_t ws_bytes, hipStream_t s) {
+  if (M < 0 || N <= 0 || N > INT32_MAX) return TILEOPS_ESHAPE;
+  if (dtype < TILEOPS_F32 || dtype > TILEOPS_BF16) return TILEOPS_EINVAL;
+  if (M == 0) return 0;
+  if (!x || !y) return TILEOPS_ENULL;
+  if (ws && !host_aligned16(ws)) return TILEOPS_EINVAL;
+  if (!ws) ws_bytes = 0;
+  switch (op) {
+    case TILEOPS_LOGSUMEXP: return dispatch_row_reduce<0>(x, y, M, N, dtype, ws, ws_bytes, s);
+    case TILEOPS_ARGMAX: return dispatch_row_reduce<1>(x, y, M, N, dtype, ws, ws_bytes, s);
+    case TILEOPS_ARGMIN: return dispatch_row_reduce<2>(x, y, M, N, dtype, ws, ws_bytes, s);
   }
   return TILEOPS_EINVAL;
 }
@@ -263,20 +467,24 @@ using namespace tileops;
 
 extern "C" int tileops_logsumexp_fwd(const void* x, void* y, int64_t M, int64_t N, int dtype,
                                      void* stream) {
-  if (M < 0 || N <= 0 || N > INT32_MAX) return TILEOPS_ESHAPE;
-  if (dtype < TILEOPS_F32 || dtype > TILEOPS_BF16) return TILEOPS_EINVAL;
-  if (M == 0) return 0;
-  if (!x || !y) return TILEOPS_ENULL;
-  return dispatch_row_reduce<0>(x, y, M, N, dtype, static_cast<hipStream_t>(stream));
+  return reduce_rows(TILEOPS_LOGSUMEXP, x, y, M, N, dtype, nullptr, 0,
+                     static_cast<hipStream_t>(stream));
 }
 
 extern "C" int tileops_argreduce_fwd(const void* x, int64_t* y, int64_t M, int64_t N, int dtype,
                                      int is_min, void* stream) {
-  if (M < 0 || N <= 0 || N > INT32_MAX) return TILEOPS_ESHAPE;
-  if (dtype < TILEOPS_F32 || dtype > TILEOPS_BF16) return TILEOPS_EINVAL;
-  if (M == 0) return 0;
-  if (!x || !y) return TILEOPS_ENULL;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  return is_min ? dispatch_row_reduce<2>(x, y, M, N, dtype, s)
-                : dispatch_row_reduce<1>(x, y, M, N, dtype, s);
+  return reduce_rows(is_min ? TILEOPS_ARGMIN : TILEOPS_ARGMAX, x, y, M, N, dtype, nullptr, 0,
+                     static_cast<hipStream_t>(stream));
+}
+
+extern "C" size_t tileops_reduce_workspace_bytes(int64_t M, int64_t N, int dtype) {
+  if (M <= 0 || N <= 0 || N > INT32_MAX || dtype < TILEOPS_F32 || dtype > TILEOPS_BF16) return 0;
+  const RowPlan p = plan_rows(M, N, dtype == TILEOPS_F32 ? 4 : 8);
+  static_assert(sizeof(LseState) == 8 && sizeof(ArgState) == 8, "partials of 8 bytes");
+  return p.nsplit > 1 ? (size_t)M * p.nsplit * 8 : 0;
+}
+
+extern "C" int tileops_reduce_fwd(int op, const void* x, void* y, int64_t M, int64_t N, int dtype,
+                                  void* ws, size_t ws_bytes, void* stream) {
+  return reduce_rows(op, x, y, M, N, dtype, ws, ws_bytes, static_cast<hipStream_t>(stream));
 }

@@ -12,6 +12,7 @@ device, the call raises.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 import threading
 from pathlib import Path
@@ -34,6 +35,9 @@ LIB_PATH = Path(
         "TILEOPS_HIP_LIB", str(Path(__file__).resolve().parent / "_native" / "libtileops_hip.so")
     )
 )
+
+# enum tileops_reduce_op (include/tileops_hip.h)
+LOGSUMEXP, ARGMAX, ARGMIN = 0, 1, 2
 
 DTYPE_CODES = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 
@@ -58,6 +62,11 @@ SIGNATURES = {
     ),
     "tileops_logsumexp_fwd": (_c_int, [_c_p, _c_p, _c_i64, _c_i64, _c_int, _c_p]),
     "tileops_argreduce_fwd": (_c_int, [_c_p, _c_p, _c_i64, _c_i64, _c_int, _c_int, _c_p]),
+    "tileops_reduce_workspace_bytes": (ctypes.c_size_t, [_c_i64, _c_i64, _c_int]),
+    "tileops_reduce_fwd": (
+        _c_int,
+        [_c_int, _c_p, _c_p, _c_i64, _c_i64, _c_int, _c_p, ctypes.c_size_t, _c_p],
+    ),
     "tileops_mha_fwd": (
         _c_int,
         [
@@ -199,3 +208,19 @@ def eager(*tensors: torch.Tensor) -> bool:
         if type(t) not in _PLAIN or (grad and t.requires_grad):
             return False
     return True
+
+
+@functools.lru_cache(maxsize=1024)
+def _reduce_scratch(M: int, N: int, code: int) -> int:
+    return lib().tileops_reduce_workspace_bytes(M, N, code)
+
+
+def reduce_rows(op: int, x: torch.Tensor, y: torch.Tensor, M: int, N: int) -> int:
+    """``tileops_reduce_fwd`` of ``x[M, N]`` into ``y[M]``, with the scratch its
+    launch plan asks for taken from torch's allocator (none for most shapes)."""
+    code = dtype_code(x.dtype)
+    need = _reduce_scratch(M, N, code)
+    ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
+    return lib().tileops_reduce_fwd(
+        op, x.data_ptr(), y.data_ptr(), M, N, code, ws.data_ptr() if need else None, need,
+        stream_of(x))

@@ -21,16 +21,8 @@ _ARGREDUCE_KINDS = {"argmax", "argmin"}
 
 def _argreduce_fwd_launch(M: int, N: int, op_kind: str, x: torch.Tensor) -> torch.Tensor:
     y = torch.empty((M,), dtype=torch.int64, device=x.device)
-    code = _native.lib().tileops_argreduce_fwd(
-        x.data_ptr(),
-        y.data_ptr(),
-        M,
-        N,
-        _native.dtype_code(x.dtype),
-        1 if op_kind == "argmin" else 0,
-        _native.stream_of(x),
-    )
-    _native.check(code, "tileops_argreduce_fwd")
+    op = _native.ARGMIN if op_kind == "argmin" else _native.ARGMAX
+    _native.check(_native.reduce_rows(op, x, y, M, N), "tileops_reduce_fwd")
     return y
 
 
@@ -54,7 +46,7 @@ class ArgreduceKernel(Kernel):
         device_index: Accepted for API compatibility.
     """
 
-    profile_kernel_name = r"tileops(?:::|\d+)row_reduce_kernel"
+    profile_kernel_name = r"tileops(?:::|\d+)(row_reduce|short_row|merge_partials)_kernel"
 
     def __init__(
         self,

@@ -21,10 +21,7 @@ __all__ = ["LogSumExpKernel"]
 
 def _logsumexp_fwd_launch(M: int, N: int, x: torch.Tensor) -> torch.Tensor:
     y = torch.empty((M,), dtype=x.dtype, device=x.device)
-    code = _native.lib().tileops_logsumexp_fwd(
-        x.data_ptr(), y.data_ptr(), M, N, _native.dtype_code(x.dtype), _native.stream_of(x)
-    )
-    _native.check(code, "tileops_logsumexp_fwd")
+    _native.check(_native.reduce_rows(_native.LOGSUMEXP, x, y, M, N), "tileops_reduce_fwd")
     return y
 
 
@@ -49,7 +46,7 @@ class LogSumExpKernel(Kernel):
             per-device sizing).
     """
 
-    profile_kernel_name = r"tileops(?:::|\d+)row_reduce_kernel"
+    profile_kernel_name = r"tileops(?:::|\d+)(row_reduce|short_row|merge_partials)_kernel"
 
     def __init__(
         self,
@@ -72,9 +69,9 @@ class LogSumExpKernel(Kernel):
 
     @property
     def default_config(self) -> dict:
-        # row_reduce_kernel: 256-thread workgroups; one wavefront per row
-        # (four rows per workgroup) from 3072 rows up, else the four
-        # wavefronts of a workgroup share a row; 4 packs in flight per lane
+        # row_reduce_kernel: one wavefront per row (four rows per workgroup)
+        # from 3072 rows up, else at least four wavefronts per row (few long
+        # rows: sixteen, or several workgroups); 4 packs in flight per lane
         return {"wavefronts_per_row": 1 if self.M >= 3072 else 4, "packs_in_flight": 4}
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
