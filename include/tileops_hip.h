@@ -224,6 +224,21 @@ int tileops_mha_fwd(const void* q, const void* k, const void* v, void* o, float*
                     void* stream);
 
 /*
+ * tileops_mha_fwd with caller scratch: few query rows against many keys (a
+ * decode step, a short chunk appended to a cache) are split over the keys, and
+ * the fp32 partial outputs and row statistics of the splits
+ * (tileops_mha_workspace_bytes, 0 where no split is planned) go to `ws`
+ * (16-byte aligned) and are combined by a second launch.  With `ws` NULL or
+ * smaller than that no call is split.
+ */
+size_t tileops_mha_workspace_bytes(int64_t B, int64_t Sq, int64_t Skv, int64_t H, int64_t Hkv,
+                                   int64_t D, int causal, float scale);
+int tileops_mha_fwd_ws(const void* q, const void* k, const void* v, void* o, float* lse, int64_t B,
+                       int64_t Sq, int64_t Skv, int64_t H, int64_t Hkv, int64_t D, int causal,
+                       float scale, float softcap, int dtype, void* ws, size_t ws_bytes,
+                       void* stream);
+
+/*
  * Chunked gated delta rule (gated DeltaNet) prefill, per (b, h):
  *   S_t = exp(g_t) S_{t-1} + beta_t k_t (v_t - k_t^T exp(g_t) S_{t-1})^T
  *   o_t = scale * q_t^T S_t

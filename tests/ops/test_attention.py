@@ -104,6 +104,32 @@ def test_gqa_prefill_kernel(causal, sq, skv):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("D, dtype, B, H, Hkv, sq, skv, softcap", [
+    (128, torch.bfloat16, 2, 8, 2, 1, 8191, 0.0),   # a decode step, ragged cache
+    (128, torch.bfloat16, 3, 4, 2, 1, 33, 0.0),     # one 32-key block and one key
+    (128, torch.float16, 1, 8, 8, 1, 31, 0.0),      # less than a block, one wavefront has work
+    (64, torch.float16, 1, 12, 4, 3, 4097, 0.0),    # group of 3: rows of a token straddle nothing
+    (128, torch.bfloat16, 1, 8, 1, 41, 2111, 0.0),  # 328 rows: a ragged last row tile
+    (96, torch.bfloat16, 1, 4, 4, 33, 2049, 0.0),   # padded LDS rows
+    (192, torch.float16, 1, 4, 1, 1, 5000, 0.0),
+    (256, torch.bfloat16, 2, 6, 2, 9, 3001, 0.0),   # two wavefronts per workgroup
+    (128, torch.bfloat16, 1, 8, 2, 2, 3000, 2.0),   # soft-capped scores
+])
+def test_gqa_few_queries_many_keys(causal, D, dtype, B, H, Hkv, sq, skv, softcap):
+    # the key-split kernel: tiles of 32 rows of one K / V head, splits of
+    # 32-key blocks over workgroups and wavefronts, combined in fp32
+    q = torch.randn(B, sq, H, D, device="cuda", dtype=dtype) * (2 if softcap else 1)
+    k = torch.randn(B, skv, Hkv, D, device="cuda", dtype=dtype)
+    v = torch.randn(B, skv, Hkv, D, device="cuda", dtype=dtype)
+    q[0, 0, 0] = 0  # a uniform row
+    k[-1, skv // 2, -1] *= 8  # a late new maximum in some rows
+    kern = GQAPrefillFwdKernel(B, H, Hkv, sq, skv, D, causal, dtype, softcap=softcap)
+    o, lse = kern(q, k, v)
+    _check(q, k, v, o, lse, causal, softcap=softcap, rtol=CAUSAL_RTOL)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("softcap, dtype, D, sq, skv", [
     (30.0, torch.bfloat16, 128, 256, 256),   # cap above every score: near the uncapped result
     (2.0, torch.bfloat16, 128, 200, 333),    # tight cap: most scores saturate

@@ -30,54 +30,20 @@
 // next power of two (rows of 128 or 256 elements, the same swizzles): the
 // padding chunks are filled with a copy of a real chunk of the row and never
 // read, and the MFMA steps cover the real dims only.
-#include <float.h>
 #include <stdlib.h>
 
 #include <type_traits>
 
-#include "common.h"
+#include "attention.h"
 
 namespace tileops {
 namespace mha {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-template <typename T> struct Mfma;
-template <> struct Mfma<bf16> {
-  typedef bf16x8 V8;
-  __device__ __forceinline__ static f32x16 run(V8 a, V8 b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-  }
-};
-template <> struct Mfma<f16> {
-  typedef f16x8 V8;
-  __device__ __forceinline__ static f32x16 run(V8 a, V8 b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-  }
-};
 
 // Lazy rescaling: the running max only moves when a tile's max exceeds it by
 // more than 2^kLazyLog2 in the exp2 domain, so P <= 2^kLazyLog2 (exact in
 // fp32 / bf16) and the O accumulator is rescaled rarely.
 constexpr float kLazyLog2 = 8.0f;
 constexpr float kLazyBound = 256.0f;  // 2^kLazyLog2
-
-typedef __attribute__((address_space(3))) void* lds_void_ptr;
-typedef short v4i16 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-
-// K and V tiles live in LDS unpadded, rows of D / 8 16-byte chunks, chunks
-// XOR-swizzled by row: K so that an MFMA operand read (16 consecutive key
-// rows, one chunk each) hits 16 distinct 16-byte bank groups, V so that the
-// transpose reads of a half-wavefront (4 consecutive key rows x 64 bytes)
-// cover all 64 banks once.
-template <int D> struct Swz {
-  static constexpr int CPR = D / 8;  // chunks per row
-  __host__ __device__ static constexpr int k_key(int r) { return CPR >= 16 ? (r & 15) : ((r >> 1) & 7); }
-  __host__ __device__ static constexpr int v_key(int r) { return CPR == 16 ? 4 * (r & 3) : 4 * ((r >> 1) & 1); }
-};
 
 // Workgroup barrier that waits only for this wavefront's LDS accesses, so
 // that direct-to-LDS loads issued before it stay in flight across it.  The
@@ -91,38 +57,6 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
-}
-
-// One 16-byte direct-to-LDS load per lane: lane l reads 16 bytes at
-// `base + off` (base uniform, in SGPRs; off a per-lane byte offset) and they
-// land at LDS byte address lds + 16 l.  Issued as inline assembly so that the
-// compiler does not track the LDS write: every wait for these loads is
-// explicit (vmcnt) and followed by a workgroup barrier before any wavefront
-// reads the data.  The compiler's hazard checks do not look into inline
-// assembly: the load starts with the one wait state the ISA requires after
-// the SALU write of M0 that precedes it (its base comes from SALU
-// arithmetic, so no VALU-to-SGPR wait is involved).
-__device__ __forceinline__ void lds_dma16(const void* base, uint32_t off, uint32_t lds) {
-  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "{m0}"(lds)
-               : "memory");
-}
-
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-  return (uint32_t)(uintptr_t)(lds_void_ptr)p;
-}
-
-// Combine a value with the one held by the partner lane l ^ 32 (VALU lane
-// swap between the two wavefront halves, no LDS round trip): the two
-// outputs of v_permlane32_swap on (x, x) are x's low and high halves.
-__device__ __forceinline__ float pair_max(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, x),
-                                                  __builtin_bit_cast(unsigned, x), false, false);
-  return fmaxf(__builtin_bit_cast(float, (unsigned)r[0]), __builtin_bit_cast(float, (unsigned)r[1]));
-}
-__device__ __forceinline__ float pair_sum(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, x),
-                                                  __builtin_bit_cast(unsigned, x), false, false);
-  return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
 }
 
 // Ping-pong schedule.  The 8 wavefronts form two groups, A = waves 0-3 and
@@ -142,13 +76,6 @@ __device__ __forceinline__ float pair_sum(float x) {
 // (phases 2t - 5 and 2t - 3), and each group ends every MFMA phase waiting
 // for everything but the windows it just issued (vmcnt(WPW)), so a tile has
 // landed two phases before its first reader.
-// tanh(y) = 1 - 2 / (1 + e^{2y}), saturating to +-1 through the
-// exponential's overflow / underflow (no branch)
-__device__ __forceinline__ float tanh_sat(float y) {
-  const float e = __builtin_amdgcn_exp2f(y * (2.0f * 1.4426950408889634f));
-  return 1.0f - 2.0f * __builtin_amdgcn_rcpf(1.0f + e);
-}
-
 // SOFTCAP: scores are capped, softcap * tanh(scale q.k / softcap) (the
 // reference's order: scale, cap, then the causal mask), and carried in log2
 // units from the start of the softmax: the caller passes scale_log2 = 1,
@@ -842,27 +769,64 @@ static int dispatch_d(int D, const void* q, const void* k, const void* v, void* 
 
 using namespace tileops;
 
-extern "C" int tileops_mha_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
-                               int64_t B, int64_t Sq, int64_t Skv, int64_t H, int64_t Hkv,
-                               int64_t D, int causal, float scale, float softcap, int dtype,
-                               void* stream) {
+namespace tileops {
+namespace mha {
+
+static int check(const Problem& p, int64_t B, int64_t Sq, int64_t Skv, int64_t H, int64_t Hkv,
+                 int64_t D, int causal, float softcap, int dtype) {
   if (B < 0 || Sq < 0 || Skv < 0 || H <= 0 || Hkv <= 0 || H % Hkv != 0) return TILEOPS_ESHAPE;
   if (D != 64 && D != 96 && D != 128 && D != 192 && D != 256) return TILEOPS_ESHAPE;
   if (B > INT32_MAX || Sq > INT32_MAX || Skv > INT32_MAX || H > 65535) return TILEOPS_ESHAPE;
   if (causal && Sq > Skv) return TILEOPS_ESHAPE;
   if (dtype != TILEOPS_F16 && dtype != TILEOPS_BF16) return TILEOPS_EINVAL;
   if (!(softcap >= 0.0f) || !(softcap < INFINITY)) return TILEOPS_EINVAL;  // NaN, < 0, inf
-  if (B == 0 || Sq == 0) return 0;
-  if (Skv == 0) return TILEOPS_ESHAPE;
-  if (!q || !k || !v || !o || !lse) return TILEOPS_ENULL;
-  if (!host_aligned16(q) || !host_aligned16(k) || !host_aligned16(v) || !host_aligned16(o))
+  return 0;
+}
+
+static int run(const Problem& p, void* ws, size_t ws_bytes, hipStream_t s) {
+  if (p.B == 0 || p.Sq == 0) return 0;
+  if (p.Skv == 0) return TILEOPS_ESHAPE;
+  if (!p.q || !p.k || !p.v || !p.o || !p.lse) return TILEOPS_ENULL;
+  if (!host_aligned16(p.q) || !host_aligned16(p.k) || !host_aligned16(p.v) || !host_aligned16(p.o))
     return TILEOPS_EINVAL;
+  if (ws && !host_aligned16(ws)) return TILEOPS_EINVAL;
   // grid: (Sq / 256) query blocks x H x B (x 2 for D = 192, 256), indexed in int
-  if (((Sq + 255) / 256) * H * B * (D >= 192 ? 2 : 1) > (int64_t)INT32_MAX) return TILEOPS_ESHAPE;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  if (dtype == TILEOPS_BF16)
-    return mha::dispatch_d<bf16>((int)D, q, k, v, o, lse, (int)B, (int)Sq, (int)Skv, (int)H,
-                                 (int)Hkv, causal != 0, scale, softcap, s);
-  return mha::dispatch_d<f16>((int)D, q, k, v, o, lse, (int)B, (int)Sq, (int)Skv, (int)H,
-                              (int)Hkv, causal != 0, scale, softcap, s);
+  if (((p.Sq + 255LL) / 256) * p.H * p.B * (p.D >= 192 ? 2 : 1) > (int64_t)INT32_MAX)
+    return TILEOPS_ESHAPE;
+  if (split_planned(p, ws ? ws_bytes : 0)) return split_launch(p, ws, ws ? ws_bytes : 0, s);
+  if (p.dtype == TILEOPS_BF16)
+    return dispatch_d<bf16>(p.D, p.q, p.k, p.v, p.o, p.lse, p.B, p.Sq, p.Skv, p.H, p.Hkv,
+                            p.causal, p.scale, p.softcap, s);
+  return dispatch_d<f16>(p.D, p.q, p.k, p.v, p.o, p.lse, p.B, p.Sq, p.Skv, p.H, p.Hkv, p.causal,
+                         p.scale, p.softcap, s);
+}
+
+}  // namespace mha
+}  // namespace tileops
+
+extern "C" size_t tileops_mha_workspace_bytes(int64_t B, int64_t Sq, int64_t Skv, int64_t H,
+                                              int64_t Hkv, int64_t D, int causal, float scale) {
+  const mha::Problem p{nullptr, nullptr, nullptr, nullptr, nullptr, (int)B, (int)Sq, (int)Skv,
+                       (int)H, (int)Hkv, (int)D, causal != 0, scale, 0.0f, TILEOPS_BF16};
+  if (mha::check(p, B, Sq, Skv, H, Hkv, D, causal, 0.0f, TILEOPS_BF16)) return 0;
+  if (B == 0 || Sq == 0 || Skv == 0) return 0;
+  return mha::split_workspace_bytes(p);
+}
+
+extern "C" int tileops_mha_fwd_ws(const void* q, const void* k, const void* v, void* o, float* lse,
+                                  int64_t B, int64_t Sq, int64_t Skv, int64_t H, int64_t Hkv,
+                                  int64_t D, int causal, float scale, float softcap, int dtype,
+                                  void* ws, size_t ws_bytes, void* stream) {
+  const mha::Problem p{q, k, v, o, lse, (int)B, (int)Sq, (int)Skv, (int)H, (int)Hkv, (int)D,
+                       causal != 0, scale, softcap, dtype};
+  if (int e = mha::check(p, B, Sq, Skv, H, Hkv, D, causal, softcap, dtype)) return e;
+  return mha::run(p, ws, ws_bytes, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int tileops_mha_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
+                               int64_t B, int64_t Sq, int64_t Skv, int64_t H, int64_t Hkv,
+                               int64_t D, int causal, float scale, float softcap, int dtype,
+                               void* stream) {
+  return tileops_mha_fwd_ws(q, k, v, o, lse, B, Sq, Skv, H, Hkv, D, causal, scale, softcap, dtype,
+                            nullptr, 0, stream);
 }

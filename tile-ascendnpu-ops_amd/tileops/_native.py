@@ -75,6 +75,18 @@ SIGNATURES = {
             _c_int, _c_float, _c_float, _c_int, _c_p,
         ],
     ),
+    "tileops_mha_workspace_bytes": (
+        ctypes.c_size_t,
+        [_c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_float],
+    ),
+    "tileops_mha_fwd_ws": (
+        _c_int,
+        [
+            _c_p, _c_p, _c_p, _c_p, _c_p,
+            _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
+            _c_int, _c_float, _c_float, _c_int, _c_p, ctypes.c_size_t, _c_p,
+        ],
+    ),
     "tileops_gdn_prefill_fwd": (
         _c_int,
         [

@@ -8,9 +8,11 @@ log-sum-exp in the log2 domain (``logsumexp / ln 2``, shape
 causal mask is right-aligned (query i sees keys j <= i + Skv - Sq).  The
 launch is wrapped in the ``tileops::gqa_prefill_fwd`` custom op (reference:
 ``npub::gqa_prefill_fwd_wrapped_kernel``).
-Device code: mha_fwd_kernel in csrc/attention.hip.
+Device code: mha_fwd_kernel in csrc/attention.hip; few query rows against
+many keys: mha_split_kernel and mha_combine_kernel in csrc/attention_split.hip.
 """
 
+import functools
 from typing import Optional, Tuple
 
 import torch
@@ -19,6 +21,11 @@ from tileops import _native
 from tileops.kernels.kernel_base import Kernel
 
 __all__ = ["GQAPrefillFwdKernel"]
+
+
+@functools.lru_cache(maxsize=1024)
+def _scratch(B: int, Sq: int, Skv: int, H: int, Hkv: int, D: int, causal: int, scale: float) -> int:
+    return _native.lib().tileops_mha_workspace_bytes(B, Sq, Skv, H, Hkv, D, causal, scale)
 
 
 def _gqa_prefill_fwd_launch(
@@ -37,13 +44,16 @@ def _gqa_prefill_fwd_launch(
 ) -> Tuple[torch.Tensor, torch.Tensor]:
     o = torch.empty_like(q)
     lse = torch.empty((batch, heads, seq_len_q), dtype=torch.float32, device=q.device)
-    code = _native.lib().tileops_mha_fwd(
+    need = _scratch(batch, seq_len_q, seq_len_kv, heads, heads_kv, dim, 1 if is_causal else 0,
+                    float(sm_scale))
+    ws = torch.empty(need, dtype=torch.uint8, device=q.device) if need else None
+    code = _native.lib().tileops_mha_fwd_ws(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(),
         batch, seq_len_q, seq_len_kv, heads, heads_kv, dim,
         1 if is_causal else 0, float(sm_scale), float(softcap), _native.dtype_code(q.dtype),
-        _native.stream_of(q),
+        ws.data_ptr() if need else None, need, _native.stream_of(q),
     )
-    _native.check(code, "tileops_mha_fwd")
+    _native.check(code, "tileops_mha_fwd_ws")
     return o, lse
 
 
@@ -70,7 +80,7 @@ class GQAPrefillFwdKernel(Kernel):
     """
 
     SUPPORTED_DTYPES = (torch.float16, torch.bfloat16)
-    profile_kernel_name = r"mha(?:::|\d+)mha_fwd_kernel"
+    profile_kernel_name = r"mha(?:::|\d+)mha_(fwd|split|combine)_kernel"
 
     def __init__(
         self,
