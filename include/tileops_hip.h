@@ -205,6 +205,18 @@ int tileops_reduce_fwd(int op, const void* x, void* y, int64_t M, int64_t N, int
                        size_t ws_bytes, void* stream);
 
 /*
+ * The same reductions of a contiguous x[outer, n, inner] read as it lies:
+ * over n (ends == 0, y[outer, inner]), or over outer and inner (ends != 0,
+ * y[n], TILEOPS_LOGSUMEXP only).  `ws` (16-byte aligned) must hold
+ * tileops_reduce_axis_workspace_bytes (0 for most shapes with ends == 0).
+ */
+size_t tileops_reduce_axis_workspace_bytes(int op, int64_t outer, int64_t n, int64_t inner,
+                                           int ends, int dtype);
+int tileops_reduce_axis_fwd(int op, const void* x, void* y, int64_t outer, int64_t n,
+                            int64_t inner, int ends, int dtype, void* ws, size_t ws_bytes,
+                            void* stream);
+
+/*
  * Flash attention forward, BSHD layout.
  *   q:    [B, Sq,  H,   D]    k, v: [B, Skv, Hkv, D]   (dtype F16 or BF16)
  *   o:    [B, Sq,  H,   D]    lse:  [B, H, Sq] float32 (log2 domain:

@@ -289,3 +289,82 @@ def test_row_split_and_ragged_rows(M, N, dtype):
     y = LogSumExpFwdOp(dtype=dtype)(x)
     atol, rtol = ref_tolerance(dtype)
     assert_close_np(to_np(y), torch.logsumexp(x.double(), -1).cpu().numpy(), atol, rtol, "lse")
+
+
+# -- reductions over other dims, read as they lie -----------------------------------------
+def test_strided_form_matches_the_general_path():
+    # every dim set of shapes with size-1 dims: the view reduces to what the
+    # permuted copy reduces to; views that are not contiguous are refused
+    import itertools
+
+    from tileops.ops._multidim import flatten_for_multidim, strided_form
+
+    seen = {False: 0, True: 0}
+    for shape in ((5, 64), (3, 4, 70), (2, 3, 4, 66), (3, 1, 64), (1, 7, 64, 1), (2, 65, 1, 3),
+                  (64, 2, 3, 64)):
+        x = torch.randn(shape, dtype=torch.float64)
+        for k in range(1, len(shape) + 1):
+            for dims in itertools.combinations(range(len(shape)), k):
+                form = strided_form(x, list(dims))
+                if form is None:
+                    continue
+                outer, n, inner, ends = form
+                seen[ends] += 1
+                v = x.view(outer, n, inner)
+                y = torch.logsumexp(v, (0, 2) if ends else (1,)).reshape(-1)
+                flat, _, _ = flatten_for_multidim(x, list(dims))
+                ref = torch.logsumexp(flat, -1).reshape(-1)
+                torch.testing.assert_close(y, ref, rtol=1e-12, atol=1e-12)
+                if not ends and len(dims) == 1:
+                    assert torch.equal(v.argmax(1).reshape(-1), flat.argmax(-1).reshape(-1))
+    assert seen[False] >= 8 and seen[True] >= 3
+    x = torch.randn(4, 128, 64)
+    assert strided_form(x.transpose(0, 1), [0]) is None
+    assert strided_form(x[:, ::2], [0]) is None
+    assert strided_form(x[:, :, :63].contiguous(), [1]) is None  # too few columns
+    assert strided_form(torch.empty(0, 4, 64), [0]) is None
+    assert strided_form(torch.empty(20000, 2, 64), [0, 2]) is None  # too many partials
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape, dim, dtype", [
+    ((4, 128, 4096), 0, torch.float16),    # 256 threads across the columns, 4 rows
+    ((3, 5, 67), 1, torch.bfloat16),       # one column per thread, ragged tile
+    ((2, 33, 200), 1, torch.float32),      # 50 packs, 16 across
+    ((2, 1000, 1024), 1, torch.float16),   # 16 row groups per column
+    ((9, 40, 70, 64), 1, torch.float32),   # 64 across, several tiles
+    ((20000, 64), 0, torch.float32),       # split over workgroups
+    ((20001, 65), 0, torch.bfloat16),      # split, one column per thread
+    ((1, 1, 64), 1, torch.float16),        # one row
+])
+def test_reductions_over_an_inner_dim(shape, dim, dtype):
+    x = torch.randn(shape, device="cuda").to(dtype)
+    n = shape[dim]
+    x.select(dim, n - 1)[..., ::3] = 9.0  # extremes in the last and first rows
+    x.select(dim, 0)[..., 1::3] = 9.0
+    x.view(-1)[5] = float("nan")
+    assert torch.equal(ArgmaxFwdOp(dtype=dtype, dim=dim)(x).cpu(), torch.argmax(x.cpu(), dim=dim))
+    x.view(-1)[5] = float("-inf")
+    y = LogSumExpFwdOp(dtype=dtype, dim=dim, keepdim=True)(x)
+    atol, rtol = ref_tolerance(dtype)
+    ref = torch.logsumexp(x.double(), dim, keepdim=True).cpu().numpy()
+    assert_close_np(to_np(y), ref, atol, rtol, "lse over an inner dim")
+    # a contiguous view whose base is off the 16-byte grid
+    off = torch.empty(x.numel() + 1, device="cuda", dtype=dtype)[1:].view(shape).copy_(x)
+    assert torch.equal(ArgmaxFwdOp(dtype=dtype, dim=dim)(off), ArgmaxFwdOp(dtype=dtype, dim=dim)(x))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape, dims, dtype", [
+    ((4, 128, 4096), [0, 2], torch.float16),  # rows of several wavefronts
+    ((33, 3, 100), [0, 2], torch.float32),    # short rows
+    ((70, 2, 203), [0, 2], torch.bfloat16),   # ragged rows
+    ((2, 1, 600000), [0, 2], torch.float32),  # rows split over workgroups too
+    ((6, 5, 4, 64), [0, 1, 3], torch.float32),
+    ((6, 5, 4, 64), [0, 1], torch.float16),
+])
+def test_logsumexp_over_several_dims(shape, dims, dtype):
+    x = (torch.randn(shape, device="cuda") * 2).to(dtype)
+    y = LogSumExpFwdOp(dtype=dtype, dim=dims)(x)
+    atol, rtol = ref_tolerance(dtype)
+    assert_close_np(to_np(y), torch.logsumexp(x.double(), dims).cpu().numpy(), atol, rtol, "lse")

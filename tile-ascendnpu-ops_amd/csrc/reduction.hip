@@ -1,7 +1,8 @@
-// Row reductions for gfx950: LogSumExp and Argmax / Argmin over the last
-// dimension of a row-major [M, N] tensor.
+// Reductions for gfx950: LogSumExp and Argmax / Argmin over the last dimension
+// of a row-major [M, N] tensor, over the middle dimension of [outer, N, inner]
+// (column kernel, below) or over the outer two of [R, M, L].
 //
-// A wavefront streams its share of a row in 16-byte packs, UNROLL packs per
+// Rows.// A wavefront streams its share of a row in 16-byte packs, UNROLL packs per
 // lane in flight, folds them into a per-lane partial, and the 64 partials meet
 // in a shuffle butterfly.  What bounds the kernel is HBM where the rows fill
 // the chip, and the latency of one wavefront's chain of loads where they do
@@ -167,10 +168,16 @@ __device__ __forceinline__ void row_store(void* out, int64_t row, typename RowSt
 // and those after them in its last, one per lane,
 // so that an odd row length costs no more loads than an even one (LogSumExp
 // bf16 16384 x 4097: 73.9 us with one element per lane and load, 34.8 so).
-// With nsplit > 1 `out` holds nsplit partials per row.
+// With PartMap::per > 0 `out` holds partials: `per` for each of the `keep`
+// outputs, of which rows r, r + keep, .. give nsplit each.
+struct PartMap {
+  int64_t keep;
+  int per;
+};
 template <typename T, int OP, int WPR, int U, bool ALIGNED>
 __global__ __launch_bounds__(WPR > 4 ? 64 * WPR : 256) void row_reduce_kernel(
-    const T* __restrict__ x, void* __restrict__ out, int64_t M, int64_t N, int nstep, int nsplit) {
+    const T* __restrict__ x, void* __restrict__ out, int64_t M, int64_t N, int nstep, int nsplit,
+    PartMap pm) {
   typedef typename RowState<OP>::S S;
   constexpr int V = Elem<T>::kVec;
   constexpr int WPB = WPR > 4 ? WPR : 4;  // wavefronts per workgroup
@@ -258,8 +265,10 @@ __global__ __launch_bounds__(WPR > 4 ? 64 * WPR : 256) void row_reduce_kernel(
       __syncthreads();
     }
     if (lane == 0 && wave_in_row == 0 && row < M) {
-      if (nsplit > 1) static_cast<S*>(out)[row * nsplit + split] = st;
-      else row_store<T, OP>(out, row, st);
+      if (pm.per > 0)
+        static_cast<S*>(out)[row % pm.keep * pm.per + row / pm.keep * nsplit + split] = st;
+      else
+        row_store<T, OP>(out, row, st);
     }
   }
 }
@@ -272,7 +281,8 @@ __global__ __launch_bounds__(WPR > 4 ? 64 * WPR : 256) void row_reduce_kernel(
 // and after the packs).  Otherwise a lane takes one element.
 template <typename T, int OP, int G, bool PACKS, bool ALIGNED>
 __global__ __launch_bounds__(256) void short_row_kernel(const T* __restrict__ x,
-                                                        void* __restrict__ out, int64_t M, int N) {
+                                                        void* __restrict__ out, int64_t M, int N,
+                                                        PartMap pm) {
   constexpr int V = PACKS ? Elem<T>::kVec : 1, EDGE = PACKS && !ALIGNED ? 2 : 0;
   static_assert(EDGE == 0 || G >= Elem<T>::kVec, "a lane per edge element");
   const int64_t row = (int64_t)blockIdx.x * (256 / G) + threadIdx.x / G;
@@ -318,7 +328,12 @@ __global__ __launch_bounds__(256) void short_row_kernel(const T* __restrict__ x,
     }
   }
   st = row_wave<OP, G>(st);
-  if (row < M && lane == 0) row_store<T, OP>(out, row, st);
+  if (row < M && lane == 0) {
+    if (pm.per > 0)
+      static_cast<typename RowState<OP>::S*>(out)[row % pm.keep * pm.per + row / pm.keep] = st;
+    else
+      row_store<T, OP>(out, row, st);
+  }
 }
 
 // The nsplit partials of each output, one wavefront per output.
@@ -343,20 +358,20 @@ __global__ __launch_bounds__(256) void merge_partials_kernel(
 // and more, ~2 us each) are split over workgroups of four wavefronts, one
 // step each up to 1024 workgroups; the merge launch and its scratch cost ~2.5
 // us on the GPU and ~4 us of an eager call's host time, so shorter rows stay
-// whole (LogSumExp bf16 4 x 102400: 17.5 us with four wavefronts per row, 9.8
-// with sixteen, 6.3 split, but 10.4 and 14.6 us per eager call; Argmax of 2^21
+// whole (LogSumExp bf16 4 x 102400: 17.5 us with four wavefronts per row,
+// 10.7 with sixteen, 6.3 split, but 10.7 and 14.6 us per eager call; Argmax of 2^21
 // fp16 elements 682 -> 9.7 us, of 2^25 fp32 9222 -> 32).
 // A wavefront keeps 4 packs per lane in flight, fewer where its whole share of
 // the row is less (slots past the row still cost their exponentials).
 struct RowPlan {
   int wpr, u, nsplit, nstep;
 };
-static RowPlan plan_rows(int64_t M, int64_t N, int vec) {
+static RowPlan plan_rows(int64_t M, int64_t N, int vec, bool split = true) {
   const int64_t chunks = std::max<int64_t>((N / vec + 63) / 64, 1);
   RowPlan p{4, 4, 1, 0};
   if (M >= 256 * 12) p.wpr = 1;
   else if (M <= 512 && chunks >= 16 * 4) p.wpr = 16;
-  if (M <= 128 && chunks >= 16 * 16) {
+  if (split && M <= 128 && chunks >= 16 * 16) {
     p.wpr = 4;
     p.nsplit = (int)std::min<int64_t>((chunks + 15) / 16, 1024 / M);
   }
@@ -368,97 +383,285 @@ static RowPlan plan_rows(int64_t M, int64_t N, int vec) {
 
 template <typename T, int OP, int WPR, int U>
 static void launch_rows(const T* x, void* out, int64_t M, int64_t N, const RowPlan& p,
-                        hipStream_t s) {
+                        PartMap pm, hipStream_t s) {
   const bool aligned = host_aligned16(x) && (N % Elem<T>::kVec) == 0;
   const int rows_per_block = WPR > 4 ? 1 : 4 / WPR;
   const int64_t blocks = (M + rows_per_block - 1) / rows_per_block * p.nsplit;
   const dim3 grid((unsigned)std::min<int64_t>(blocks, 256 * 32)), block(WPR > 4 ? 64 * WPR : 256);
   if (aligned)
-    row_reduce_kernel<T, OP, WPR, U, true><<<grid, block, 0, s>>>(x, out, M, N, p.nstep, p.nsplit);
+    row_reduce_kernel<T, OP, WPR, U, true><<<grid, block, 0, s>>>(x, out, M, N, p.nstep, p.nsplit, pm);
   else
-    row_reduce_kernel<T, OP, WPR, U, false><<<grid, block, 0, s>>>(x, out, M, N, p.nstep, p.nsplit);
+    row_reduce_kernel<T, OP, WPR, U, false><<<grid, block, 0, s>>>(x, out, M, N, p.nstep, p.nsplit, pm);
 }
 
 template <typename T, int OP, int WPR>
 static void launch_rows_u(const T* x, void* out, int64_t M, int64_t N, const RowPlan& p,
-                          hipStream_t s) {
-  if (p.u == 1) launch_rows<T, OP, WPR, 1>(x, out, M, N, p, s);
-  else if (p.u == 2) launch_rows<T, OP, WPR, 2>(x, out, M, N, p, s);
-  else if (p.u == 3) launch_rows<T, OP, WPR, 3>(x, out, M, N, p, s);
-  else launch_rows<T, OP, WPR, 4>(x, out, M, N, p, s);
+                          PartMap pm, hipStream_t s) {
+  if (p.u == 1) launch_rows<T, OP, WPR, 1>(x, out, M, N, p, pm, s);
+  else if (p.u == 2) launch_rows<T, OP, WPR, 2>(x, out, M, N, p, pm, s);
+  else if (p.u == 3) launch_rows<T, OP, WPR, 3>(x, out, M, N, p, pm, s);
+  else launch_rows<T, OP, WPR, 4>(x, out, M, N, p, pm, s);
 }
 
 // The short-row kernel where it applies: rows of at most 64 packs.  Ragged
 // rows of up to 16 elements go element by element.
 template <typename T, int OP>
-static bool try_short(const T* x, void* out, int64_t M, int64_t N, hipStream_t s) {
+static bool try_short(const T* x, void* out, int64_t M, int64_t N, PartMap pm, hipStream_t s) {
   constexpr int V = Elem<T>::kVec;
   if (N / V > 64 || M > (int64_t)INT32_MAX) return false;  // four rows per workgroup at worst
   const int n = (int)N, np = n / V;
   const dim3 block(256);
   auto grid = [&](int G) { return dim3((unsigned)((M + 256 / G - 1) / (256 / G))); };
   if (host_aligned16(x) && n % V == 0) {
-    if (np <= 4) short_row_kernel<T, OP, 4, true, true><<<grid(4), block, 0, s>>>(x, out, M, n);
-    else if (np <= 16) short_row_kernel<T, OP, 16, true, true><<<grid(16), block, 0, s>>>(x, out, M, n);
-    else if (np <= 32) short_row_kernel<T, OP, 32, true, true><<<grid(32), block, 0, s>>>(x, out, M, n);
-    else short_row_kernel<T, OP, 64, true, true><<<grid(64), block, 0, s>>>(x, out, M, n);
+    if (np <= 4) short_row_kernel<T, OP, 4, true, true><<<grid(4), block, 0, s>>>(x, out, M, n, pm);
+    else if (np <= 16) short_row_kernel<T, OP, 16, true, true><<<grid(16), block, 0, s>>>(x, out, M, n, pm);
+    else if (np <= 32) short_row_kernel<T, OP, 32, true, true><<<grid(32), block, 0, s>>>(x, out, M, n, pm);
+    else short_row_kernel<T, OP, 64, true, true><<<grid(64), block, 0, s>>>(x, out, M, n, pm);
   } else if (n <= 16) {
-    if (n <= 4) short_row_kernel<T, OP, 4, false, false><<<grid(4), block, 0, s>>>(x, out, M, n);
-    else short_row_kernel<T, OP, 16, false, false><<<grid(16), block, 0, s>>>(x, out, M, n);
+    if (n <= 4) short_row_kernel<T, OP, 4, false, false><<<grid(4), block, 0, s>>>(x, out, M, n, pm);
+    else short_row_kernel<T, OP, 16, false, false><<<grid(16), block, 0, s>>>(x, out, M, n, pm);
   } else {
-    if (np <= 16) short_row_kernel<T, OP, 16, true, false><<<grid(16), block, 0, s>>>(x, out, M, n);
-    else if (np <= 32) short_row_kernel<T, OP, 32, true, false><<<grid(32), block, 0, s>>>(x, out, M, n);
-    else short_row_kernel<T, OP, 64, true, false><<<grid(64), block, 0, s>>>(x, out, M, n);
+    if (np <= 16) short_row_kernel<T, OP, 16, true, false><<<grid(16), block, 0, s>>>(x, out, M, n, pm);
+    else if (np <= 32) short_row_kernel<T, OP, 32, true, false><<<grid(32), block, 0, s>>>(x, out, M, n, pm);
+    else short_row_kernel<T, OP, 64, true, false><<<grid(64), block, 0, s>>>(x, out, M, n, pm);
   }
   return true;
 }
 
+// Rows of x[M, N]; with keep > 0 rows r, r + keep, .. belong to output r
+// (x[M / keep, keep, N] reduced over its outer two dimensions), merged from
+// partials.
 template <typename T, int OP>
-static int launch_row_reduce(const void* xv, void* out, int64_t M, int64_t N, void* ws,
-                             size_t ws_bytes, hipStream_t s) {
+static int launch_row_reduce(const void* xv, void* out, int64_t M, int64_t N, int64_t keep,
+                             void* ws, size_t ws_bytes, hipStream_t s) {
   typedef typename RowState<OP>::S S;
   const T* x = static_cast<const T*>(xv);
-  if (try_short<T, OP>(x, out, M, N, s)) return launch_status();
   RowPlan p = plan_rows(M, N, Elem<T>::kVec);
-  if (p.nsplit > 1 && ws_bytes < (size_t)M * p.nsplit * sizeof(S)) p.nsplit = 1;  // no scratch
-  void* dst = p.nsplit > 1 ? ws : out;
-  if (p.wpr == 1) launch_rows_u<T, OP, 1>(x, dst, M, N, p, s);
-  else if (p.wpr == 4) launch_rows_u<T, OP, 4>(x, dst, M, N, p, s);
-  else launch_rows<T, OP, 16, 4>(x, dst, M, N, p, s);
-  if (p.nsplit > 1) {
+  const int64_t folds = keep > 0 ? M / keep : 1, nout = M / folds;
+  if (folds == 1 && p.nsplit > 1 && ws_bytes < (size_t)M * p.nsplit * sizeof(S))
+    p = plan_rows(M, N, Elem<T>::kVec, false);  // no scratch
+  PartMap pm{nout, 0};
+  const bool is_short = N / Elem<T>::kVec <= 64 && M <= (int64_t)INT32_MAX;
+  if (folds > 1 || (p.nsplit > 1 && !is_short)) pm.per = (int)folds * (is_short ? 1 : p.nsplit);
+  void* dst = pm.per > 0 ? ws : out;
+  if (!try_short<T, OP>(x, dst, M, N, pm, s)) {
+    if (p.wpr == 1) launch_rows_u<T, OP, 1>(x, dst, M, N, p, pm, s);
+    else if (p.wpr == 4) launch_rows_u<T, OP, 4>(x, dst, M, N, p, pm, s);
+    else launch_rows<T, OP, 16, 4>(x, dst, M, N, p, pm, s);
+  }
+  if (pm.per > 0) {
     if (int e = launch_status()) return e;
-    merge_partials_kernel<T, OP><<<dim3((unsigned)((M + 3) / 4)), dim3(256), 0, s>>>(
-        static_cast<const S*>(ws), out, M, p.nsplit);
+    merge_partials_kernel<T, OP><<<dim3((unsigned)((nout + 3) / 4)), dim3(256), 0, s>>>(
+        static_cast<const S*>(ws), out, nout, pm.per);
   }
   return launch_status();
 }
 
+// ---------------------------------------------------------------------------
+// Columns: x[outer, N, inner] reduced over N, read as it lies (the copy that
+// moves the reduced dimension last costs a read and a write of the tensor, and
+// short columns then made one wavefront per column: Argmax fp16 [4, 128, 4096]
+// over dimension 0 126.6 us, 6.6 so).  A thread owns the V columns of one pack (one
+// column where packs do not fit); TX threads cover neighbouring packs and 256
+// / TX share a column's rows, U = 4 in flight each, and meet in LDS.  Bound by
+// HBM where the columns fill the chip; `nsplit` workgroups share a column
+// where they do not.
+// ---------------------------------------------------------------------------
+template <typename T, int OP, int V, int TX>
+__global__ __launch_bounds__(256) void col_reduce_kernel(const T* __restrict__ x,
+                                                         void* __restrict__ out, int64_t N,
+                                                         int64_t inner, int64_t ntile, int nsplit) {
+  typedef typename RowState<OP>::S S;
+  constexpr int TY = 256 / TX, U = 4;
+  const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
+  const int64_t tile = blockIdx.x % ntile;
+  const int64_t rest = blockIdx.x / ntile;
+  const int split = (int)(rest % nsplit);
+  const int64_t o = rest / nsplit;
+  const int64_t c0 = (tile * TX + tx) * V;
+  const int64_t per = (N + nsplit - 1) / nsplit;
+  const int64_t n0 = split * per, n1 = min(N, n0 + per);
+
+  S st[V];
+#pragma unroll
+  for (int e = 0; e < V; ++e) st[e] = row_init<OP>();
+  if (c0 < inner) {
+    const T* xc = x + o * N * inner + c0;
+    for (int64_t n = n0 + ty; n < n1; n += TY * U) {
+      // All U loads, then their uses: rows past the end repeat the last one
+      // (a load under a branch of its own would be waited for there) and
+      // read as -inf.
+      Pack<T> p[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const T* at = xc + min(n + u * TY, n1 - 1) * inner;
+        if constexpr (V > 1) p[u] = load_pack_nt(at);
+        else p[u].v[0] = *at;
+      }
+      float vals[V][U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+#pragma unroll
+        for (int e = 0; e < V; ++e)
+          vals[e][u] = n + u * TY < n1 ? Elem<T>::to_f32(p[u].v[e]) : -INFINITY;
+      }
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+        if constexpr (OP == 0) {
+          lse_fold<U>(st[e], vals[e]);
+        } else {
+#pragma unroll
+          for (int u = 0; u < U; ++u)
+            if (n + u * TY < n1) arg_step<OP == 2>(st[e], vals[e][u], (int)(n + u * TY));
+        }
+      }
+    }
+  }
+  auto put = [&](int64_t col, S v) {
+    const int64_t i = o * inner + col;
+    if (nsplit > 1) static_cast<S*>(out)[i * nsplit + split] = v;
+    else row_store<T, OP>(out, i, v);
+  };
+  if constexpr (TY == 1) {
+    if (c0 < inner) {
+#pragma unroll
+      for (int e = 0; e < V; ++e) put(c0 + e, st[e]);
+    }
+  } else {
+    __shared__ S part[TY][TX * V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) part[ty][tx * V + e] = st[e];
+    __syncthreads();
+    for (int c = threadIdx.x; c < TX * V; c += 256) {
+      const int64_t col = tile * TX * V + c;
+      if (col >= inner) break;
+      S v = part[0][c];
+#pragma unroll 4
+      for (int y = 1; y < TY; ++y) v = row_merge<OP>(v, part[y][c]);
+      put(col, v);
+    }
+  }
+}
+
+// Threads across the columns: 256 where that alone fills the chip, and for a
+// few rows from half a workgroup per CU on (LogSumExp bf16 [4, 128, 4096] over
+// dimension 0: 5.3 us with 256, 6.7 with 64 and their merge) except where a
+// thread would store eight scattered indices (Argmax fp16 of that shape: 7.8
+// and 6.6); else 64, else 16.  With less than a workgroup per CU and six steps
+// of ~2 us or more the rows are split, one step each up to two workgroups per
+// CU (Argmax bf16 [3, 1000, 64]: 32 us whole, 9.7 split; 300 rows: 9.4 either
+// way, and whole is one launch).  Rows past the end of a thread's last step
+// repeat the last one, so that its loads are all in flight (Argmax bf16 [46,
+// 276, 2113]: 38.5 us with a branch per load, 28.6 so).
+struct ColPlan {
+  int v, tx, nsplit;
+  int64_t ntile;
+};
+static ColPlan plan_cols(int64_t outer, int64_t N, int64_t inner, int vec, bool arg) {
+  ColPlan p{inner % vec == 0 ? vec : 1, 16, 1, 0};
+  const int64_t packs = inner / p.v;
+  auto blocks = [&](int tx) { return outer * ((packs + tx - 1) / tx); };
+  if (packs > 64 && blocks(256) >= (N <= 8 && !(arg && p.v == 8) ? 128 : 1024)) p.tx = 256;
+  else if (packs > 16 && (N <= 32 || blocks(64) >= 512)) p.tx = 64;
+  p.ntile = (packs + p.tx - 1) / p.tx;
+  const int64_t wg = blocks(p.tx), steps = N / (256 / p.tx * 4);
+  if (wg < 256 && steps >= 6) p.nsplit = (int)std::min<int64_t>(steps, 512 / wg);
+  return p;
+}
+
+template <typename T, int OP, int V>
+static void launch_cols(const T* x, void* out, int64_t outer, int64_t N, int64_t inner,
+                        const ColPlan& p, hipStream_t s) {
+  const dim3 grid((unsigned)(p.ntile * p.nsplit * outer)), block(256);
+  if (p.tx == 256)
+    col_reduce_kernel<T, OP, V, 256><<<grid, block, 0, s>>>(x, out, N, inner, p.ntile, p.nsplit);
+  else if (p.tx == 64)
+    col_reduce_kernel<T, OP, V, 64><<<grid, block, 0, s>>>(x, out, N, inner, p.ntile, p.nsplit);
+  else
+    col_reduce_kernel<T, OP, V, 16><<<grid, block, 0, s>>>(x, out, N, inner, p.ntile, p.nsplit);
+}
+
+template <typename T, int OP>
+static int launch_col_reduce(const void* xv, void* out, int64_t outer, int64_t N, int64_t inner,
+                             void* ws, hipStream_t s) {
+  typedef typename RowState<OP>::S S;
+  const T* x = static_cast<const T*>(xv);
+  ColPlan p = plan_cols(outer, N, inner, Elem<T>::kVec, OP != 0);
+  if (p.ntile * p.nsplit * outer > (int64_t)INT32_MAX) return TILEOPS_ESHAPE;
+  if (p.v > 1 && !host_aligned16(x)) {  // same grid, one column per thread
+    p.v = 1;
+    p.ntile = (inner + p.tx - 1) / p.tx;
+    if (p.ntile * p.nsplit * outer > (int64_t)INT32_MAX) return TILEOPS_ESHAPE;
+  }
+  void* dst = p.nsplit > 1 ? ws : out;
+  if (p.v > 1) launch_cols<T, OP, Elem<T>::kVec>(x, dst, outer, N, inner, p, s);
+  else launch_cols<T, OP, 1>(x, dst, outer, N, inner, p, s);
+  if (p.nsplit > 1) {
+    if (int e = launch_status()) return e;
+    const int64_t nout = outer * inner;
+    merge_partials_kernel<T, OP><<<dim3((unsigned)((nout + 3) / 4)), dim3(256), 0, s>>>(
+        static_cast<const S*>(ws), out, nout, p.nsplit);
+  }
+  return launch_status();
+}
+
+// One call: x[outer, n, inner].  kRows: rows of `inner` (outer 1); kAxis: over
+// n; kEnds: over outer and inner.
+enum Form { kRows, kAxis, kEnds };
+struct Call {
+  Form form;
+  const void* x;
+  void* y;
+  int64_t outer, n, inner;
+  void* ws;
+  size_t ws_bytes;
+  hipStream_t s;
+};
+
+template <typename T, int OP>
+static int launch_call(const Call& c) {
+  if (c.form == kAxis)
+    return launch_col_reduce<T, OP>(c.x, c.y, c.outer, c.n, c.inner, c.ws, c.s);
+  return launch_row_reduce<T, OP>(c.x, c.y, c.outer * c.n, c.inner, c.form == kEnds ? c.n : 0,
+                                  c.ws, c.ws_bytes, c.s);
+}
+
 template <int OP>
-static int dispatch_row_reduce(const void* x, void* out, int64_t M, int64_t N, int dtype, void* ws,
-                               size_t ws_bytes, hipStream_t s) {
+static int dispatch_call(const Call& c, int dtype) {
   switch (dtype) {
-    case TILEOPS_F32: return launch_row_reduce<float, OP>(x, out, M, N, ws, ws_bytes, s);
-    case TILEOPS_F16: return launch_row_reduce<f16, OP>(x, out, M, N, ws, ws_bytes, s);
-    case TILEOPS_BF16: return launch_row_reduce<bf16, OP>(x, out, M, N, ws, ws_bytes, s);
+    case TILEOPS_F32: return launch_call<float, OP>(c);
+    case TILEOPS_F16: return launch_call<f16, OP>(c);
+    case TILEOPS_BF16: return launch_call<bf16, OP>(c);
   }
   return TILEOPS_EINVAL;
 }
 
-// Checks and dispatch shared by the entry points.
+static int run_call(int op, Call c, int dtype) {
+  if (c.ws && !host_aligned16(c.ws)) return TILEOPS_EINVAL;
+  if (!c.ws) c.ws_bytes = 0;
+  switch (op) {
+    case TILEOPS_LOGSUMEXP: return dispatch_call<0>(c, dtype);
+    case TILEOPS_ARGMAX: return dispatch_call<1>(c, dtype);
+    case TILEOPS_ARGMIN: return dispatch_call<2>(c, dtype);
+  }
+  return TILEOPS_EINVAL;
+}
+
+// Checks and dispatch shared by the row entry points.
 static int reduce_rows(int op, const void* x, void* y, int64_t M, int64_t N, int dtype, void* ws,
                        size_t ws_bytes, hipStream_t s) {
   if (M < 0 || N <= 0 || N > INT32_MAX) return TILEOPS_ESHAPE;
   if (dtype < TILEOPS_F32 || dtype > TILEOPS_BF16) return TILEOPS_EINVAL;
   if (M == 0) return 0;
   if (!x || !y) return TILEOPS_ENULL;
-  if (ws && !host_aligned16(ws)) return TILEOPS_EINVAL;
-  if (!ws) ws_bytes = 0;
-  switch (op) {
-    case TILEOPS_LOGSUMEXP: return dispatch_row_reduce<0>(x, y, M, N, dtype, ws, ws_bytes, s);
-    case TILEOPS_ARGMAX: return dispatch_row_reduce<1>(x, y, M, N, dtype, ws, ws_bytes, s);
-    case TILEOPS_ARGMIN: return dispatch_row_reduce<2>(x, y, M, N, dtype, ws, ws_bytes, s);
-  }
-  return TILEOPS_EINVAL;
+  return run_call(op, Call{kRows, x, y, 1, M, N, ws, ws_bytes, s}, dtype);
+}
+
+static size_t rows_bytes(int64_t M, int64_t N, int vec, int64_t folds) {
+  static_assert(sizeof(LseState) == 8 && sizeof(ArgState) == 8, "partials of 8 bytes");
+  const bool is_short = N / vec <= 64 && M <= (int64_t)INT32_MAX;
+  const int nsplit = is_short ? 1 : plan_rows(M, N, vec).nsplit;
+  return folds > 1 || nsplit > 1 ? (size_t)M * nsplit * 8 : 0;
 }
 
 }  // namespace tileops
@@ -479,12 +682,36 @@ extern "C" int tileops_argreduce_fwd(const void* x, int64_t* y, int64_t M, int64
 
 extern "C" size_t tileops_reduce_workspace_bytes(int64_t M, int64_t N, int dtype) {
   if (M <= 0 || N <= 0 || N > INT32_MAX || dtype < TILEOPS_F32 || dtype > TILEOPS_BF16) return 0;
-  const RowPlan p = plan_rows(M, N, dtype == TILEOPS_F32 ? 4 : 8);
-  static_assert(sizeof(LseState) == 8 && sizeof(ArgState) == 8, "partials of 8 bytes");
-  return p.nsplit > 1 ? (size_t)M * p.nsplit * 8 : 0;
+  return rows_bytes(M, N, dtype == TILEOPS_F32 ? 4 : 8, 1);
 }
 
 extern "C" int tileops_reduce_fwd(int op, const void* x, void* y, int64_t M, int64_t N, int dtype,
                                   void* ws, size_t ws_bytes, void* stream) {
   return reduce_rows(op, x, y, M, N, dtype, ws, ws_bytes, static_cast<hipStream_t>(stream));
+}
+
+extern "C" size_t tileops_reduce_axis_workspace_bytes(int op, int64_t outer, int64_t n,
+                                                      int64_t inner, int ends, int dtype) {
+  if (outer <= 0 || n <= 0 || inner <= 0 || dtype < TILEOPS_F32 || dtype > TILEOPS_BF16) return 0;
+  const int vec = dtype == TILEOPS_F32 ? 4 : 8;
+  if (ends) return rows_bytes(outer * n, inner, vec, outer);
+  const int64_t nsplit = plan_cols(outer, n, inner, vec, op != TILEOPS_LOGSUMEXP).nsplit;
+  return nsplit > 1 ? (size_t)(outer * inner * nsplit) * 8 : 0;
+}
+
+extern "C" int tileops_reduce_axis_fwd(int op, const void* x, void* y, int64_t outer, int64_t n,
+                                       int64_t inner, int ends, int dtype, void* ws,
+                                       size_t ws_bytes, void* stream) {
+  if (outer < 0 || n < 0 || inner < 0) return TILEOPS_ESHAPE;
+  if (n > INT32_MAX || inner > INT32_MAX || outer > INT32_MAX) return TILEOPS_ESHAPE;
+  if (dtype < TILEOPS_F32 || dtype > TILEOPS_BF16) return TILEOPS_EINVAL;
+  if (ends && op != TILEOPS_LOGSUMEXP) return TILEOPS_EINVAL;  // an index has no order there
+  if (outer == 0 || n == 0 || inner == 0) return TILEOPS_ESHAPE;
+  if (outer > INT64_MAX / n / inner) return TILEOPS_ESHAPE;
+  if (!x || !y) return TILEOPS_ENULL;
+  if (ws_bytes < tileops_reduce_axis_workspace_bytes(op, outer, n, inner, ends, dtype) ||
+      (!ws && ws_bytes > 0))
+    return TILEOPS_EWORKSPACE;
+  return run_call(op, Call{ends ? kEnds : kAxis, x, y, outer, n, inner, ws, ws_bytes,
+                           static_cast<hipStream_t>(stream)}, dtype);
 }

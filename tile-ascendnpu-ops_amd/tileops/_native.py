@@ -67,6 +67,14 @@ SIGNATURES = {
         _c_int,
         [_c_int, _c_p, _c_p, _c_i64, _c_i64, _c_int, _c_p, ctypes.c_size_t, _c_p],
     ),
+    "tileops_reduce_axis_workspace_bytes": (
+        ctypes.c_size_t,
+        [_c_int, _c_i64, _c_i64, _c_i64, _c_int, _c_int],
+    ),
+    "tileops_reduce_axis_fwd": (
+        _c_int,
+        [_c_int, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_p, ctypes.c_size_t, _c_p],
+    ),
     "tileops_mha_fwd": (
         _c_int,
         [
@@ -236,3 +244,20 @@ def reduce_rows(op: int, x: torch.Tensor, y: torch.Tensor, M: int, N: int) -> in
     return lib().tileops_reduce_fwd(
         op, x.data_ptr(), y.data_ptr(), M, N, code, ws.data_ptr() if need else None, need,
         stream_of(x))
+
+
+@functools.lru_cache(maxsize=1024)
+def _reduce_axis_scratch(op: int, outer: int, n: int, inner: int, ends: int, code: int) -> int:
+    return lib().tileops_reduce_axis_workspace_bytes(op, outer, n, inner, ends, code)
+
+
+def reduce_axis(op: int, x: torch.Tensor, y: torch.Tensor, outer: int, n: int, inner: int,
+                ends: bool) -> int:
+    """``tileops_reduce_axis_fwd`` of contiguous ``x[outer, n, inner]`` over n
+    (into ``y[outer, inner]``) or over outer and inner (into ``y[n]``)."""
+    code, ends = dtype_code(x.dtype), int(ends)
+    need = _reduce_axis_scratch(op, outer, n, inner, ends, code)
+    ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
+    return lib().tileops_reduce_axis_fwd(
+        op, x.data_ptr(), y.data_ptr(), outer, n, inner, ends, code,
+        ws.data_ptr() if need else None, need, stream_of(x))

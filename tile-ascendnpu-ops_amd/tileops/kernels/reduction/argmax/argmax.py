@@ -34,6 +34,24 @@ def _(M: int, N: int, op_kind: str, x: torch.Tensor) -> torch.Tensor:
     return torch.empty((M,), dtype=torch.int64, device=x.device)
 
 
+def _argreduce_axis_launch(
+    outer: int, n: int, inner: int, ends: bool, op_kind: str, x: torch.Tensor
+) -> torch.Tensor:
+    y = torch.empty((n if ends else outer * inner,), dtype=torch.int64, device=x.device)
+    op = _native.ARGMIN if op_kind == "argmin" else _native.ARGMAX
+    _native.check(
+        _native.reduce_axis(op, x, y, outer, n, inner, ends), "tileops_reduce_axis_fwd")
+    return y
+
+
+_argreduce_axis = torch.library.custom_op("tileops::argreduce_axis_fwd", mutates_args=())(_argreduce_axis_launch)
+
+
+@_argreduce_axis.register_fake
+def _(outer, n, inner, ends, op_kind, x):
+    return torch.empty((n if ends else outer * inner,), dtype=torch.int64, device=x.device)
+
+
 class ArgreduceKernel(Kernel):
     """Argmax / argmin forward kernel; output is always int64.
 
@@ -46,7 +64,7 @@ class ArgreduceKernel(Kernel):
         device_index: Accepted for API compatibility.
     """
 
-    profile_kernel_name = r"tileops(?:::|\d+)(row_reduce|short_row|merge_partials)_kernel"
+    profile_kernel_name = r"tileops(?:::|\d+)(row_reduce|short_row|col_reduce|merge_partials)_kernel"
 
     def __init__(
         self,
@@ -86,3 +104,15 @@ class ArgreduceKernel(Kernel):
         if _native.eager(x):
             return _argreduce_fwd_launch(self.M, self.N, self.op_kind, x)
         return _argreduce_fwd(self.M, self.N, self.op_kind, x)
+
+    def reduce_axis(
+        self, x: torch.Tensor, outer: int, n: int, inner: int, ends: bool
+    ) -> torch.Tensor:
+        """The reduction of contiguous ``x.view(outer, n, inner)`` over n (or, with
+        ``ends``, over outer and inner), flat like ``forward``'s result."""
+        _native.require_device(x)
+        self.check_tensor("x", x, dtype=self.dtype, numel=self.M * self.N)
+        if outer * n * inner != self.M * self.N or not x.is_contiguous():
+            raise ValueError(f"{type(self).__name__}: expected a contiguous [{outer}, {n}, {inner}]")
+        fwd = _argreduce_axis_launch if _native.eager(x) else _argreduce_axis
+        return fwd(outer, n, inner, ends, self.op_kind, x)

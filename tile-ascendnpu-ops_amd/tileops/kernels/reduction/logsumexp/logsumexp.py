@@ -33,6 +33,23 @@ def _(M: int, N: int, x: torch.Tensor) -> torch.Tensor:
     return torch.empty((M,), dtype=x.dtype, device=x.device)
 
 
+def _logsumexp_axis_launch(
+    outer: int, n: int, inner: int, ends: bool, x: torch.Tensor
+) -> torch.Tensor:
+    y = torch.empty((n if ends else outer * inner,), dtype=x.dtype, device=x.device)
+    _native.check(
+        _native.reduce_axis(_native.LOGSUMEXP, x, y, outer, n, inner, ends), "tileops_reduce_axis_fwd")
+    return y
+
+
+_logsumexp_axis = torch.library.custom_op("tileops::logsumexp_axis_fwd", mutates_args=())(_logsumexp_axis_launch)
+
+
+@_logsumexp_axis.register_fake
+def _(outer, n, inner, ends, x):
+    return torch.empty((n if ends else outer * inner,), dtype=x.dtype, device=x.device)
+
+
 class LogSumExpKernel(Kernel):
     """LogSumExp forward kernel.
 
@@ -46,7 +63,7 @@ class LogSumExpKernel(Kernel):
             per-device sizing).
     """
 
-    profile_kernel_name = r"tileops(?:::|\d+)(row_reduce|short_row|merge_partials)_kernel"
+    profile_kernel_name = r"tileops(?:::|\d+)(row_reduce|short_row|col_reduce|merge_partials)_kernel"
 
     def __init__(
         self,
@@ -81,3 +98,15 @@ class LogSumExpKernel(Kernel):
         if _native.eager(x):
             return _logsumexp_fwd_launch(self.M, self.N, x)
         return _logsumexp_fwd(self.M, self.N, x)
+
+    def reduce_axis(
+        self, x: torch.Tensor, outer: int, n: int, inner: int, ends: bool
+    ) -> torch.Tensor:
+        """The reduction of contiguous ``x.view(outer, n, inner)`` over n (or, with
+        ``ends``, over outer and inner), flat like ``forward``'s result."""
+        _native.require_device(x)
+        self.check_tensor("x", x, dtype=self.dtype, numel=self.M * self.N)
+        if outer * n * inner != self.M * self.N or not x.is_contiguous():
+            raise ValueError(f"{type(self).__name__}: expected a contiguous [{outer}, {n}, {inner}]")
+        fwd = _logsumexp_axis_launch if _native.eager(x) else _logsumexp_axis
+        return fwd(outer, n, inner, ends, x)

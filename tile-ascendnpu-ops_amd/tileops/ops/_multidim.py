@@ -8,11 +8,18 @@ moves the reduced dims last and flattens to ``[*kept, reduced]``, and
 
 from __future__ import annotations
 
+from math import prod
 from typing import Literal, Union
 
 import torch
 
-__all__ = ["EmptyDimPolicy", "flatten_for_multidim", "normalize_dim", "restore_multidim_shape"]
+__all__ = [
+    "EmptyDimPolicy",
+    "flatten_for_multidim",
+    "normalize_dim",
+    "restore_multidim_shape",
+    "strided_form",
+]
 
 EmptyDimPolicy = Literal["reject", "full", "noop"]
 
@@ -47,6 +54,33 @@ def normalize_dim(
     if len(set(out)) != len(out):
         raise ValueError(f"Duplicate dims in reduction: {dims}")
     return sorted(out)
+
+
+def strided_form(x: torch.Tensor, dims: list[int]) -> "tuple[int, int, int, bool] | None":
+    """``(outer, n, inner, ends)`` when the reduction of ``x`` over ``dims`` (sorted)
+    is one over the middle (``ends`` False) or the two outer dims (``ends`` True) of
+    ``x.view(outer, n, inner)`` that the kernels read without a copy; None otherwise.
+
+    Below 64 neighbouring columns (or, for ``ends``, rows of 64 elements) the
+    strided reads leave most of a wavefront idle and the copy is kept; ``ends``
+    merges ``outer`` partials per output on one wavefront, which bounds it.
+    """
+    if not x.is_contiguous() or x.numel() == 0 or not dims:
+        return None
+    shape, lo, hi = x.shape, dims[0], dims[-1]
+    if hi - lo + 1 == len(dims):  # one run of reduced dims
+        outer, n, inner = prod(shape[:lo]), prod(shape[lo:hi + 1]), prod(shape[hi + 1:])
+        if inner < 64 or n >= 2**31 or outer * ((inner + 15) // 16) >= 2**31:
+            return None
+        return outer, n, inner, False
+    kept = [i for i in range(lo, hi + 1) if i not in dims]
+    if lo == 0 and hi == x.ndim - 1 and kept[-1] - kept[0] + 1 == len(kept):
+        outer, n = prod(shape[:kept[0]]), prod(shape[kept[0]:kept[-1] + 1])
+        inner = prod(shape[kept[-1] + 1:])
+        if inner < 64 or inner >= 2**31 or outer > 16384:
+            return None
+        return outer, n, inner, True
+    return None
 
 
 def flatten_for_multidim(

@@ -21,6 +21,7 @@ from tileops.ops._multidim import (
     flatten_for_multidim,
     normalize_dim,
     restore_multidim_shape,
+    strided_form,
 )
 from tileops.ops.op_base import Op
 
@@ -78,9 +79,32 @@ class _ReduceOpBase(Op):
         return {}
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        y = self._reduce_strided(x)
+        if y is not None:
+            return y
         x2d, orig_shape, dim_info, kernel = self._prepare_input(x)
         y = kernel(x2d)
         return self._reshape_output(y, orig_shape, dim_info)
+
+    def _reduce_strided(self, x: torch.Tensor) -> Optional[torch.Tensor]:
+        """A reduction over one dim that is not the last, read as it lies, when
+        the kernel is this library's; None otherwise."""
+        self._validate_input_tensor(x)
+        dim = self.dim
+        if not isinstance(dim, int) or not (-x.ndim <= dim < x.ndim):
+            return None
+        dim %= x.ndim
+        form = strided_form(x, [dim]) if dim != x.ndim - 1 else None
+        if form is None:
+            return None
+        N = x.shape[dim]
+        M = x.numel() // N
+        kernel = self._get_or_create_kernel(M, N)
+        if type(kernel) is not self._kernel_cls:
+            return None
+        self._last_roofline_mn = (M, N)
+        y = kernel.reduce_axis(x, *form)
+        return self._reshape_output(y, x.shape, dim)
 
     def _validate_input_tensor(self, x: torch.Tensor) -> None:
         backend = get_device_backend()

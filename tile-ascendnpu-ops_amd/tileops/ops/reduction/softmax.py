@@ -20,6 +20,7 @@ from tileops.ops._multidim import (
     flatten_for_multidim,
     normalize_dim,
     restore_multidim_shape,
+    strided_form,
 )
 from tileops.ops.op_base import Op
 
@@ -92,6 +93,16 @@ class LogSumExpFwdOp(Op):
         if isinstance(dim, (list, tuple)) or dim is None:
             dims = normalize_dim(dim, x.ndim, empty_dim_policy=self._empty_dim_policy)
             self._static_axes = frozenset([(0, d) for d in dims])
+            form = strided_form(x, dims)
+            if form is not None:
+                N = prod(x.shape[i] for i in dims)
+                M = x.numel() // N
+                kernel = self._get_or_create_kernel(M, N, x.dtype, x.device.index)
+                if type(kernel) is self._kernel_class:
+                    self._last_roofline_spec = (M, N, x.dtype)
+                    self.kernel = kernel
+                    y = kernel.reduce_axis(x, *form)
+                    return restore_multidim_shape(y, orig_shape, dims, self.keepdim)
             x, orig_shape, _ = flatten_for_multidim(x, dims)
             N = x.shape[-1]
             M = prod(x.shape[:-1])
@@ -116,15 +127,18 @@ class LogSumExpFwdOp(Op):
         self._static_axes = frozenset({(0, d)})
         M = prod([s for i, s in enumerate(x.shape) if i != d])
         self._last_roofline_spec = (M, N, x.dtype)
-        moved = d != x.ndim - 1
-        if moved:
-            x = x.movedim(d, -1)
-        x = x.contiguous()
-        if x.dim() != 2:
-            x = x.reshape(M, N)
         kernel = self._get_or_create_kernel(M, N, x.dtype, x.device.index)
         self.kernel = kernel
-        y = kernel(x)
+        form = strided_form(x, [d]) if d != x.ndim - 1 else None
+        if form is not None and type(kernel) is self._kernel_class:
+            y = kernel.reduce_axis(x, *form)
+        else:
+            if d != x.ndim - 1:
+                x = x.movedim(d, -1)
+            x = x.contiguous()
+            if x.dim() != 2:
+                x = x.reshape(M, N)
+            y = kernel(x)
         if self.keepdim:
             shape = list(orig_shape)
             shape[d] = 1
