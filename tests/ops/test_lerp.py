@@ -171,3 +171,27 @@ def test_lerp_eval_roofline_and_init_args():
     assert opt.eval_roofline() == (96, 4 * 32 * 4)
     assert _extract_op_init_args(opt) == {"input": (8, 4), "end": (8, 4), "weight": (1, 4),
                                           "dtype": torch.float32}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("sa, sb, sw", [
+    ((3, 16, 7, 7), (16, 1, 1), (1, 1, 7)),   # packs across rows and channels
+    ((2, 9, 14, 14), (9, 1, 1), (2, 1, 1, 1)),
+    ((5, 1001), (1, 1001), (5, 1)),           # odd rows, a ragged tail
+    ((1, 333), (4, 333), (4, 333)),           # only the later operands are laid out like y
+    ((4, 3, 1), (4, 3, 5), (1, 3, 5)),        # rows shorter than a pack
+])
+def test_broadcast_ragged_rows_match_the_materialised_broadcast(dtype, sa, sb, sw):
+    # same arithmetic on another path: equal bit for bit
+    a, b, w = (torch.randn(s, device="cuda").to(dtype) for s in (sa, sb, sw))
+    shape = torch.broadcast_shapes(sa, sb, sw)
+    full = [t.expand(shape).contiguous() for t in (a, b, w)]
+    y = LerpTensorFwdOp(input=sa, end=sb, weight=sw, dtype=dtype)(a, b, w)
+    ref = LerpTensorFwdOp(input=shape, end=shape, weight=shape, dtype=dtype)(*full)
+    assert torch.equal(y, ref)
+    # an operand off the 16-byte grid, the others flat
+    off = torch.empty(full[1].numel() + 1, device="cuda", dtype=dtype)[1:].view(shape)
+    off.copy_(full[1])
+    y = LerpTensorFwdOp(input=shape, end=shape, weight=shape, dtype=dtype)(full[0], off, full[2])
+    assert torch.equal(y, ref)

@@ -5,7 +5,7 @@ Reference class: examples/TileOPs/tileops/kernels/elementwise/add
 reference Ops materialised the broadcast with ``expand().contiguous()`` and
 ran a flat kernel; here the kernel reads each operand through per-dimension
 strides (0 on a broadcast dimension), so no copy is made.  Device code:
-bcast_vec_kernel / bcast_inner_kernel / bcast_any_kernel with BC_ADD in
+bcast_vec_kernel / bcast_inner_kernel / bcast_flat_kernel / bcast_any_kernel with BC_ADD in
 csrc/elementwise.hip.
 """
 
@@ -42,7 +42,7 @@ class BroadcastFwdKernel(Kernel):
     and hand them to the C ABI as host arrays."""
 
     SUPPORTED_DTYPES = (torch.float16, torch.bfloat16, torch.float32)
-    profile_kernel_name = r"tileops(?:::|\d+)bcast_(vec|inner|any)_kernel"
+    profile_kernel_name = r"tileops(?:::|\d+)bcast_(vec|inner|flat|any)_kernel"
 
     def _init_common(self, N_total: int, dtype: torch.dtype, config: Optional[dict]) -> None:
         if dtype not in self.SUPPORTED_DTYPES:
