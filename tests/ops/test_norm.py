@@ -10,7 +10,14 @@ import pytest
 import torch
 
 from oracle import tileops_oracle as orc
-from tests._util import NAMES, from_np, ref_tolerance, to_np
+from tests._util import (
+    NAMES,
+    assert_bits_equal,
+    assert_close_np,
+    from_np,
+    ref_tolerance,
+    to_np,
+)
 from tileops.kernels.norm.fused_add_layer_norm import FusedAddLayerNormKernel
 from tileops.ops.norm.fused_add_layer_norm import FusedAddLayerNormFwdOp
 from tileops.testing.test_base import TestBase
@@ -137,3 +144,26 @@ def test_fused_add_layer_norm_kernel_rejects_dtype():
 def test_fused_add_layer_norm_roofline_needs_forward():
     with pytest.raises(RuntimeError, match="requires a prior"):
         FusedAddLayerNormFwdOp(dtype=torch.float16).eval_roofline()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("param_dtype", [None, torch.float32])
+@pytest.mark.parametrize("m, n, dtype", [
+    (9, 17, torch.float16),       # one pack and every split of the elements around it
+    (9, 15, torch.float16),       # less than two packs: the three-pass kernel
+    (5, 9, torch.float32),
+    (33, 2049, torch.bfloat16),   # the last pack in a pass of its own
+    (3, 4097, torch.float32),
+    (4, 16383, torch.bfloat16),   # the longest row in registers
+    (1500, 517, torch.bfloat16),  # many rows
+])
+def test_fused_add_layer_norm_ragged_rows(m, n, dtype, param_dtype):
+    test = FusedAddLayerNormTest(m, n, dtype, param_dtype=param_dtype)
+    x, r, w, b = test.gen_inputs()
+    y, r_out = FusedAddLayerNormFwdOp(dtype=dtype)(x, r, w, b)
+    y_ref, added = orc.fused_add_layer_norm(to_np(x), to_np(r), to_np(w), to_np(b), 1e-5,
+                                            NAMES[dtype])
+    assert_bits_equal(to_np(r_out), added, "residual_out")
+    # the bound of the test above: one rounding of y, fp32 statistics
+    atol, rtol = ref_tolerance(dtype)
+    assert_close_np(to_np(y), y_ref, atol, rtol, "y")

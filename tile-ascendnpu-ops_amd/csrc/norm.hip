@@ -6,14 +6,14 @@
 //   y     = round_T((r_out - mean) * rstd * w + b)  mean/var of the *rounded* sum,
 //                                                   biased variance, fp32 math
 //
-// Fast path (N % pack == 0, 16-byte aligned rows, a row fits in 16 packs per
-// lane): one wavefront per row, the two row statistics are wavefront
-// butterflies, w / b are staged once per workgroup into LDS as fp32 so that
-// the HBM stream is only x, residual in and y, r_out out.
-// Long rows (up to 32 packs per lane of a wavefront): one 256-lane
+// Many rows (N % pack == 0, up to 16 packs per lane of a wavefront): one
+// wavefront per row, the two row statistics are wavefront butterflies, w / b
+// are staged once per workgroup into LDS as fp32 so that the HBM stream is
+// only x, residual in and y, r_out out.
+// Few or long rows (up to 2048 packs), whole packs or ragged: one 256-lane
 // workgroup per row, the row in registers, workgroup reductions.
-// Fallback (any N or alignment): grid-stride workgroups, three passes over
-// global memory.
+// Fallback (longer rows, any alignment): grid-stride workgroups, three passes
+// over global memory.
 #include "common.h"
 
 namespace tileops {
@@ -216,35 +216,55 @@ __device__ __forceinline__ float block_sum4(float v, float* part) {
   return t;
 }
 
-// Long rows (1024 < packs <= 2048: fp32 N <= 8192, 16-bit N <= 16384): one
-// 256-lane workgroup per row, KP packs per lane held in registers, so the
+// One 256-lane workgroup per row, KP packs per lane held in registers, so the
 // rounded sum is never re-read from memory (the three-pass kernel re-reads
 // r_out twice, and at thousands of rows in flight those re-reads miss L2).
 // w / b come straight from global memory (L2-resident across rows).
-template <typename T, typename W, int KP>
+// RAGGED: N is not a whole number of packs, so rows start off the 16-byte
+// grid, all four by the same amount (their bases are on it): the packs start
+// at the row's first aligned element, and the elements before and after them
+// (at most 2 V - 2) go one to a lane.
+template <typename T, typename W, int KP, bool RAGGED>
 __global__ __launch_bounds__(256) void fused_add_ln_block_kernel(
     const T* __restrict__ x, const T* __restrict__ res, const W* __restrict__ w,
     const W* __restrict__ b, T* __restrict__ y, T* __restrict__ rout, int N, float eps,
     bool vec_params) {
   constexpr int V = Elem<T>::kVec;
   __shared__ float part[4];
-  const int npack = N / V;
-  const int64_t row = blockIdx.x;
-  const T* xr = x + row * N;
-  const T* rr = res + row * N;
+  const int tid = threadIdx.x;
+  const int64_t row0 = (int64_t)blockIdx.x * N;
+  const int head = RAGGED ? min((int)(-row0 & (V - 1)), N) : 0;
+  const int npack = (N - head) / V;
+  const T* xr = x + row0 + head;
+  const T* rr = res + row0 + head;
+  T* yr = y + row0 + head;
+  T* sr = rout + row0 + head;
+  // this lane's edge element, relative to the first pack (a lane without one
+  // takes element 0 of the row and masks it out)
+  const int tail = N - head - npack * V;
+  const bool edge = RAGGED && tid < head + tail;
+  const int ei = edge && tid >= head ? npack * V + (tid - head) : edge ? tid - head : -head;
+  T es{};
   // every lane loads all KP packs, past-the-end ones clamped onto the row's
   // last pack (one uniform load sequence); they are masked out below
   Pack<T> xs[KP], rs[KP];
 #pragma unroll
   for (int k = 0; k < KP; ++k) {
-    const int p = min(k * 256 + (int)threadIdx.x, npack - 1);
+    const int p = min(k * 256 + tid, npack - 1);
     xs[k] = load_pack_nt(xr + (int64_t)p * V);
     rs[k] = load_pack_nt(rr + (int64_t)p * V);
   }
   float sum = 0.0f;
+  if constexpr (RAGGED) {
+    es = Elem<T>::from_f32(Elem<T>::to_f32(xr[ei]) + Elem<T>::to_f32(rr[ei]));
+    if (edge) {
+      sum = Elem<T>::to_f32(es);
+      sr[ei] = es;
+    }
+  }
 #pragma unroll
   for (int k = 0; k < KP; ++k) {
-    const int p = k * 256 + threadIdx.x;
+    const int p = k * 256 + tid;
     float s_part = 0.0f;
 #pragma unroll
     for (int e = 0; e < V; ++e) {
@@ -254,12 +274,16 @@ __global__ __launch_bounds__(256) void fused_add_ln_block_kernel(
     }
     if (p < npack) {
       sum += s_part;
-      store_pack_nt(rout + row * N + (int64_t)p * V, xs[k]);
+      store_pack_nt(sr + (int64_t)p * V, xs[k]);
     }
   }
   const float inv_n = 1.0f / (float)N;
   const float mean = block_sum4(sum, part) * inv_n;
   float sq = 0.0f;
+  if constexpr (RAGGED) {
+    const float d = Elem<T>::to_f32(es) - mean;
+    if (edge) sq = d * d;
+  }
 #pragma unroll
   for (int k = 0; k < KP; ++k) {
     float q_part = 0.0f;
@@ -268,22 +292,28 @@ __global__ __launch_bounds__(256) void fused_add_ln_block_kernel(
       const float d = Elem<T>::to_f32(xs[k].v[e]) - mean;
       q_part = fmaf(d, d, q_part);
     }
-    if (k * 256 + (int)threadIdx.x < npack) sq += q_part;
+    if (k * 256 + tid < npack) sq += q_part;
   }
   const float rstd = 1.0f / sqrtf(block_sum4(sq, part) * inv_n + eps);
+  if constexpr (RAGGED) {
+    if (edge) {
+      const float d = Elem<T>::to_f32(es) - mean;
+      yr[ei] = Elem<T>::from_f32(fmaf(d * rstd, wload(w, head + ei), wload(b, head + ei)));
+    }
+  }
 #pragma unroll
   for (int k = 0; k < KP; ++k) {
-    const int p = k * 256 + threadIdx.x;
+    const int p = k * 256 + tid;
     if (p < npack) {
       float wv[V], bv[V];
-      load_params<T, W>(w, b, (int64_t)p * V, vec_params, wv, bv);
+      load_params<T, W>(w, b, head + (int64_t)p * V, vec_params, wv, bv);
       Pack<T> o;
 #pragma unroll
       for (int e = 0; e < V; ++e) {
         const float d = Elem<T>::to_f32(xs[k].v[e]) - mean;
         o.v[e] = Elem<T>::from_f32(fmaf(d * rstd, wv[e], bv[e]));
       }
-      store_pack_nt(y + row * N + (int64_t)p * V, o);
+      store_pack_nt(yr + (int64_t)p * V, o);
     }
   }
 }
@@ -344,6 +374,27 @@ static void launch_wave(const T* x, const T* r, const W* w, const W* b, T* y, T*
       x, r, w, b, y, ro, M, N, eps, vec);
 }
 
+template <typename T, typename W, bool RAGGED>
+static void launch_block(const T* x, const T* r, const W* w, const W* b, T* y, T* ro, int64_t M,
+                         int n, float eps, hipStream_t s) {
+  constexpr int V = Elem<T>::kVec, PV = 16 / (int)sizeof(W);
+  const bool vec = n % PV == 0 && host_aligned16(w) && host_aligned16(b) && !RAGGED;
+  const dim3 grid((unsigned)M), block(256);
+#define TILEOPS_LN_BLOCK(KP) \
+  fused_add_ln_block_kernel<T, W, KP, RAGGED><<<grid, block, 0, s>>>(x, r, w, b, y, ro, n, eps, vec)
+  switch ((n / V + 255) / 256) {
+    case 1: TILEOPS_LN_BLOCK(1); break;
+    case 2: TILEOPS_LN_BLOCK(2); break;
+    case 3: TILEOPS_LN_BLOCK(3); break;
+    case 4: TILEOPS_LN_BLOCK(4); break;
+    case 5: TILEOPS_LN_BLOCK(5); break;
+    case 6: TILEOPS_LN_BLOCK(6); break;
+    case 7: TILEOPS_LN_BLOCK(7); break;
+    default: TILEOPS_LN_BLOCK(8); break;
+  }
+#undef TILEOPS_LN_BLOCK
+}
+
 template <typename T, typename W>
 static int launch_fused_add_ln(const void* xv, const void* rv, const void* wv, const void* bv,
                                void* yv, void* rov, int64_t M, int64_t N, float eps,
@@ -355,28 +406,28 @@ static int launch_fused_add_ln(const void* xv, const void* rv, const void* wv, c
   const W* b = static_cast<const W*>(bv);
   T* y = static_cast<T*>(yv);
   T* ro = static_cast<T*>(rov);
-  const bool packable = N % V == 0 && host_aligned16(x) && host_aligned16(r) &&
-                        host_aligned16(y) && host_aligned16(ro);
+  const bool aligned = host_aligned16(x) && host_aligned16(r) && host_aligned16(y) &&
+                       host_aligned16(ro);
+  const bool packable = aligned && N % V == 0;
   const int64_t lane_packs = (N / V + 63) / 64;
+  const int n = (int)N;
+  // One wavefront per row where rows are short and many; a workgroup per row
+  // else (1 x 8192 bf16: 7.8 -> 4.3 us, 64 x 4096 5.5 -> 4.0, 1000 x 2048 5.3
+  // -> 4.7, 4096 x 5120 34.1 -> 32.3; the wavefront stays where it is the
+  // faster: 16384 x 768 21.3 against 27.1, 32768 x 4096 181 against 183, and at
+  // 13 to 16 packs per lane 2048 x 8192 23.7 against 27.3).  Ragged rows of two packs and more have at least one aligned pack
+  // (2048 x 4097 bf16: 26.0 us three-pass, 17.4 so).
   // grid x dimension times block size stays within 32 bits on both fast paths
-  if (packable && lane_packs <= 16 && M <= (int64_t)(UINT32_MAX / 64)) {
-    const int n = (int)N;
+  const bool wave = M > 1024 && (lane_packs <= 8 || (lane_packs > 12 && lane_packs <= 16));
+  if (packable && wave && M <= (int64_t)(UINT32_MAX / 64)) {
     if (lane_packs <= 1) launch_wave<T, W, 1>(x, r, w, b, y, ro, M, n, eps, s);
     else if (lane_packs <= 2) launch_wave<T, W, 2>(x, r, w, b, y, ro, M, n, eps, s);
     else if (lane_packs <= 4) launch_wave<T, W, 4>(x, r, w, b, y, ro, M, n, eps, s);
     else if (lane_packs <= 8) launch_wave<T, W, 8>(x, r, w, b, y, ro, M, n, eps, s);
     else launch_wave<T, W, 16>(x, r, w, b, y, ro, M, n, eps, s);
-  } else if (packable && lane_packs <= 32 && M <= (int64_t)(UINT32_MAX / 256)) {
-    // 1024 < N / V <= 2048: KP = ceil(packs / 256) in 5..8
-    const int n = (int)N;
-    const int kp = (int)((N / V + 255) / 256);
-    constexpr int PV = 16 / (int)sizeof(W);
-    const bool vec = N % PV == 0 && host_aligned16(w) && host_aligned16(b);
-    const dim3 grid((unsigned)M), block(256);
-    if (kp <= 5) fused_add_ln_block_kernel<T, W, 5><<<grid, block, 0, s>>>(x, r, w, b, y, ro, n, eps, vec);
-    else if (kp == 6) fused_add_ln_block_kernel<T, W, 6><<<grid, block, 0, s>>>(x, r, w, b, y, ro, n, eps, vec);
-    else if (kp == 7) fused_add_ln_block_kernel<T, W, 7><<<grid, block, 0, s>>>(x, r, w, b, y, ro, n, eps, vec);
-    else fused_add_ln_block_kernel<T, W, 8><<<grid, block, 0, s>>>(x, r, w, b, y, ro, n, eps, vec);
+  } else if (aligned && (packable || N >= 2 * V) && lane_packs <= 32 && M <= (int64_t)(UINT32_MAX / 256)) {
+    if (packable) launch_block<T, W, false>(x, r, w, b, y, ro, M, n, eps, s);
+    else launch_block<T, W, true>(x, r, w, b, y, ro, M, n, eps, s);
   } else {
     int64_t blocks = M < 256 * 16 ? M : 256 * 16;
     fused_add_ln_generic_kernel<T, W><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(x, r, w, b, y,

@@ -10,10 +10,11 @@ Per row of N elements::
 with mean / biased variance of the rounded sum in fp32.  ``forward`` returns a
 list ``[y, residual_out]`` shaped like ``x``.  ``weight`` / ``bias`` may be the
 input dtype (the reference contract) or float32.
-Device code (csrc/norm.hip): fused_add_ln_wave_kernel (up to 1024 16-byte
-packs per row: one wavefront per row), fused_add_ln_block_kernel (1025 to
-2048 packs: one 256-lane workgroup per row, the row in registers) and
-fused_add_ln_generic_kernel (any other N or alignment).
+Device code (csrc/norm.hip): fused_add_ln_wave_kernel (many rows of up to 1024
+16-byte packs: one wavefront per row), fused_add_ln_block_kernel (few rows, and
+rows of up to 2048 packs, ragged ones included: one 256-lane workgroup per row,
+the row in registers) and fused_add_ln_generic_kernel (longer rows and other
+alignments).
 """
 
 from typing import Optional
