@@ -83,6 +83,8 @@ def _slow_inputs(B, T, H, seed):
         pytest.param(2, 320, 1, False, marks=pytest.mark.full),  # 5 chunks
         pytest.param(1, 128, 5, True, marks=pytest.mark.full),   # 2 chunks, 5 heads
         pytest.param(3, 1500, 11, True, marks=pytest.mark.full),  # 33 heads, several segments
+        pytest.param(1, 577, 2, True, marks=pytest.mark.full),    # 10 chunks: the fewest that split
+        pytest.param(1, 1000, 16, True, marks=pytest.mark.full),  # two chunks per segment
     ],
 )
 def test_gdn_prefill_small(B, T, H, with_h0):

@@ -1100,24 +1100,33 @@ __global__ __launch_bounds__(256) void gdn_copy_state_kernel(const float* h0, fl
   if (i < n) hT[i] = h0 ? h0[i] : 0.0f;
 }
 
-// Segment count: enough (head, segment) workgroups for the device's compute
-// units in each launch (one workgroup per CU: its LDS images fill one), at
-// least 4 chunks per segment, and none when the heads alone fill the device.
+// Segment count.  At most one (head, segment) workgroup per compute unit in
+// each launch (its LDS images fill one), and none where the heads alone fill
+// the device.  Within that, the two launches cost ~11 us per chunk of a
+// segment and every segment ~4.2 us more (the composition is a chain over
+// them), fitted to 16 shapes of 2 to 64 heads and 8 to 64 chunks; the mean of
+// the exact and the rounded-up segment length stands for the longest one.
+// (At least 4 chunks per segment before, us: 16 heads x 16 chunks 59.2 with 4
+// segments, 48.7 with 8; x 12 chunks 56.2 with 3, 43.5 with 6; 8 heads x 64
+// chunks 89.2 with 16, 87.5 with 12.)  Short sequences run as one segment:
+// below 10 chunks (9: 40.6 us as one, 39.7 as 5), below 16 where segments
+// multiply the parallelism by at most 4 (64 heads x 12: 55.1 as one, 61.8 as
+// 3), below 32 where at most by 2 (128 x 16: 68 and 76).
 static int plan_segments(int64_t BH, int64_t nc, int requested) {
-  int ns;
-  if (requested > 0) {
-    ns = (int)std::min<int64_t>(std::min<int64_t>(requested, kMaxSeg), std::max<int64_t>(nc, 1));
-  } else {
-    const int cus = device_cu_count();
-    if (nc < 8 || 2 * BH > cus) return 1;
-    // at most twice the parallelism of one segment: the maps' extra work
-    // and the launches' fixed costs only pay off over long sequences
-    // (128 heads x 16 chunks: 68 us as one segment, 76 us as three)
-    if (cus / BH <= 2 && nc < 32) return 1;
-    ns = (int)std::min<int64_t>(std::min<int64_t>(cus / BH + 1, nc / 4), kMaxSeg);
-    if (ns < 3) ns = 1;
+  if (requested > 0)
+    return (int)std::min<int64_t>(std::min<int64_t>(requested, kMaxSeg), std::max<int64_t>(nc, 1));
+  const int64_t room = device_cu_count() / BH;
+  if (room < 2 || nc < 10) return 1;
+  if ((room <= 4 && nc < 16) || (room <= 2 && nc < 32)) return 1;
+  int best = 1;
+  double cost = 0.0;
+  const int64_t most = std::min<int64_t>(std::min<int64_t>(room + 1, nc / 2), kMaxSeg);
+  for (int64_t ns = 3; ns <= most; ++ns) {
+    const double len = 0.5 * ((double)((nc + ns - 1) / ns) + (double)nc / (double)ns);
+    const double c = 11.0 * len + 4.2 * (double)ns;
+    if (best == 1 || c < cost) best = (int)ns, cost = c;
   }
-  return std::max(ns, 1);
+  return best;
 }
 
 inline size_t ws_bytes_for(int64_t BH, int nseg) {
