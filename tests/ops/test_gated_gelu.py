@@ -53,6 +53,7 @@ class GatedTest(GeluAndMulWorkload, TestBase):
         pytest.param(2048, 14336, torch.bfloat16, marks=pytest.mark.full),
         pytest.param(1, 14336, torch.bfloat16, marks=pytest.mark.full),
         pytest.param(7, 1001, torch.bfloat16, marks=pytest.mark.full),  # odd N: scalar path
+        pytest.param(300, 1025, torch.float16, marks=pytest.mark.full),  # four per thread, one past
         pytest.param(5, 36, torch.float32, marks=pytest.mark.full),
     ],
 )
