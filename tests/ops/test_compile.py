@@ -62,6 +62,41 @@ def test_argmax_compiles_to_one_graph(dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dim", [0, 1, [0, 2]])
+def test_reductions_over_inner_dims_compile_to_one_graph(dim):
+    x = torch.randn(6, 20, 192, generator=torch.Generator().manual_seed(15)).bfloat16().cuda()
+    ops = [LogSumExpFwdOp(dtype=torch.bfloat16, dim=dim)]
+    if isinstance(dim, int):
+        ops.append(ArgmaxFwdOp(dtype=torch.bfloat16, dim=dim))
+    for op in ops:
+        y = op(x)  # the first call builds (and announces) the kernel
+        assert torch.equal(_compiled(op)(x), y)
+
+
+@pytest.mark.gpu
+def test_decode_attention_captured_into_a_graph():
+    # the key-split launch and its scratch under capture: every replay equals
+    # the eager call, with eager work between the replays
+    from tileops.kernels.attention.multi_head_attention import GQAPrefillFwdKernel
+
+    B, H, Hkv, Skv, D = 2, 8, 2, 4095, 128
+    q, k, v = (torch.randn(B, s, h, D, device="cuda", dtype=torch.bfloat16)
+               for s, h in ((1, H), (Skv, Hkv), (Skv, Hkv)))
+    kern = GQAPrefillFwdKernel(B, H, Hkv, 1, Skv, D, True, torch.bfloat16)
+    kern(q, k, v)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        o, lse = kern(q, k, v)
+    for _ in range(3):
+        q.normal_()
+        o_e, lse_e = kern(q, k, v)
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(o, o_e) and torch.equal(lse, lse_e)
+
+
+@pytest.mark.gpu
 def test_gdn_decode_compiles_to_one_graph():
     B, H, K, V = 2, 4, 128, 64
     gen = torch.Generator().manual_seed(14)

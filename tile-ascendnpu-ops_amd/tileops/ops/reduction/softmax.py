@@ -95,7 +95,7 @@ class LogSumExpFwdOp(Op):
             self._static_axes = frozenset([(0, d) for d in dims])
             form = strided_form(x, dims)
             if form is not None:
-                N = prod(x.shape[i] for i in dims)
+                N = prod([x.shape[i] for i in dims])
                 M = x.numel() // N
                 kernel = self._get_or_create_kernel(M, N, x.dtype, x.device.index)
                 if type(kernel) is self._kernel_class:
