@@ -160,9 +160,30 @@ def test_gdn_prefill_beta_zero_only_decays(segments):
                                config={"segments": segments})
     o, hT = kern(q, k, v, g, beta, h0)
     expect = torch.exp(g.sum(1))[:, :, None, None] * h0
-    # the segmented run composes the decay through bf16-split map products
     tol = 1e-5 if segments == 1 else 1e-4
     torch.testing.assert_close(hT, expect, rtol=tol, atol=tol)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize(
+    "T, H, segments",
+    [(640, 16, 0), (704, 4, 0), (1000, 16, 0), (1024, 1, 3), (1100, 2, 16), (4096, 2, 0)],
+)
+def test_gdn_prefill_decay_is_fp32_in_any_number_of_segments(T, H, segments):
+    # The state of a sequence that writes nothing is one fp32 product per
+    # chunk: at most 64 roundings of 2^-24 and the exponentials' few ulps, so
+    # 1e-5; a 16-bit pass anywhere is off by up to 2^-17 = 8e-6 each time.
+    gen = torch.Generator().manual_seed(T + H)
+    q, k, v, g, beta = _slow_inputs(1, T, H, T + H)
+    g = g * 0.1
+    beta.zero_()
+    h0 = torch.randn(1, H, 128, 128, generator=gen).cuda()
+    kern = GDNPrefillFwdKernel(1, T, H, 128, 128, 64, torch.bfloat16,
+                               config={"segments": segments})
+    _, hT = kern(q, k, v, g, beta, h0)
+    expect = (torch.exp(g.double().sum(1))[:, :, None, None] * h0.double()).float()
+    assert (hT - expect).norm() <= 1e-6 * expect.norm()
+    torch.testing.assert_close(hT, expect, rtol=1e-5, atol=0)
 
 
 @pytest.mark.smoke

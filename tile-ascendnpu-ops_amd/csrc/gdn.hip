@@ -27,10 +27,17 @@
 //             2 .. N-1 from segment 0's end state through the maps;
 //   launch 2: segments 1 .. N-1 run exactly from their start states
 //             (outputs; the last segment writes hT).
-// The composition uses split-bf16 products (hi*hi + hi*lo + lo*hi): launch 1
-// stores each Phi already split, as a bf16 hi image and a bf16 lo image, so
-// the composition loads them straight into LDS.  With N = 1 a single launch
-// runs every chunk from h0.
+// Phi = gam I + E, where gam is the segment's whole decay and E what its keys
+// write: the composition keeps gam S in fp32, as a chunk step keeps
+// exp(gamma) S, and takes split-bf16 products (hi*hi + hi*lo + lo*hi) for E S
+// alone, whose factors come from bf16 products anyway.  With Phi itself split a
+// state that only decayed over 1000 tokens was off by 6.9e-6, relative, in four
+// segments and 1.0e-5 in eight; so it is off by 1.4e-7 in either, as in one
+// segment (1.5e-7), and with writes of any strength (beta x 0.001 to 1, decay x
+// 0.002 to 1) no further off than in one segment.
+// Launch 1 stores each E already split, as a bf16 hi image and a bf16 lo
+// image, so the composition loads them straight into LDS.  With N = 1 a
+// single launch runs every chunk from h0.
 //
 // Workgroup (one per (head, segment)): NCW chain wavefronts and 4 prep
 // wavefronts (launch 1: NCW = 8, three wavefronts per SIMD; launch 2 and
@@ -88,7 +95,8 @@ struct Args {
   const float* h0;
   bf16* o;
   float* hT;
-  float* ws;  // per head: segment 0's end state, then (Phi_j, Bseg_j), j = 1 .. N-2
+  float* ws;  // per head: segment 0's end state, then (E_j, Bseg_j), j = 1 .. N-2;
+              // after all heads, per head and segment its decay
   int B, T, H;
   float scale;
   int nseg;
@@ -486,11 +494,11 @@ __device__ __forceinline__ void split8(f32x4 a, f32x4 b, bf16x8& hi, bf16x8& lo)
   lo = pack8(ra, rb);
 }
 
-// A map's Phi stored already split: the [128][128] bf16 image of hi, then
-// that of lo (the values split8 forms from the fp32 entries).
+// A map's E = Phi - gam I stored already split: the [128][128] bf16 image of
+// hi, then that of lo (the values split8 forms from the fp32 entries).
 template <int NB>
-__device__ __forceinline__ void phi_store(const f32x4 (&s)[NB][8], float* slot, int col0, int g,
-                                          int ln) {
+__device__ __forceinline__ void phi_store(const f32x4 (&s)[NB][8], float gam, float* slot,
+                                          int col0, int g, int ln) {
   bf16* hi = reinterpret_cast<bf16*>(slot);
   bf16* lo = hi + DK * DV;
 #pragma unroll
@@ -499,9 +507,10 @@ __device__ __forceinline__ void phi_store(const f32x4 (&s)[NB][8], float* slot, 
     for (int kb = 0; kb < 8; ++kb)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float x = s[nb][kb][r];
+        const int row = acc_row(kb, g, r), col = col0 + 16 * nb + ln;
+        const float x = row == col ? s[nb][kb][r] - gam : s[nb][kb][r];
         const bf16 xh = (bf16)x;
-        const int idx = acc_row(kb, g, r) * DV + col0 + 16 * nb + ln;
+        const int idx = row * DV + col;
         hi[idx] = xh;
         lo[idx] = (bf16)(x - (float)xh);
       }
@@ -770,6 +779,10 @@ __device__ __forceinline__ float* ws_slot(const Args& A, int bh, int idx) {
   const int nslot = 2 * A.nseg - 3;
   return A.ws + ((size_t)bh * nslot + idx) * kStateFloats;
 }
+// The decay of segment seg, behind every head's slots.
+__device__ __forceinline__ float* ws_decay(const Args& A, int bh, int seg) {
+  return ws_slot(A, A.B * A.H, 0) + (size_t)bh * A.nseg + seg;
+}
 
 // Chain wavefront program.  Every wavefront of the workgroup passes the same
 // barrier sequence: 4 in the prologue, 2 per chunk.
@@ -783,6 +796,7 @@ __device__ void run_chain(const Args& A, Smem& sm, const Seg& sg, int wave, bool
   const int col0 = OUT ? 16 * NB * wave : 32 * (wave & 3);
   f32x4 s[NB][8];
   ChainTmp<NB> tmp;
+  float gam = 1.0f;  // Phi columns: the segment's decay, rounded as the state's is
   if (!idle) {
     if (OUT) {
       // segment 0 starts from h0, segment 1 from segment 0's end state, a
@@ -835,6 +849,9 @@ __device__ void run_chain(const Args& A, Smem& sm, const Seg& sg, int wave, bool
           A.o + ((int64_t)sg.b * A.T + (int64_t)cg * C) * tok_stride + (int64_t)sg.h * DV;
       chain_part2<NB, OUT, DEEP>(s, tmp, kimg, sm.tu[0], sm.tu[1], sm.l21[c & 1], sm.aqk, fc,
                                  orow0, tok_stride, n, col0, l2 >> 4, l2 & 15);
+      if constexpr (!OUT)
+        gam = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(
+                                            __builtin_bit_cast(int, gam * fc[kFacEG])));
     }
     lds_barrier();
   }
@@ -850,7 +867,8 @@ __device__ void run_chain(const Args& A, Smem& sm, const Seg& sg, int wave, bool
   } else if (usev) {
     dst = ws_slot(A, sg.bh, 2 + 2 * (sg.seg - 1));
   } else {
-    phi_store<NB>(s, ws_slot(A, sg.bh, 1 + 2 * (sg.seg - 1)), col0, g, ln);
+    phi_store<NB>(s, gam, ws_slot(A, sg.bh, 1 + 2 * (sg.seg - 1)), col0, g, ln);
+    if (wave == 4 && lane == 0) *ws_decay(A, sg.bh, sg.seg) = gam;
     return;
   }
   state_store<NB>(s, dst, col0, g, ln);
@@ -984,12 +1002,12 @@ __global__ __launch_bounds__(64 * (NCW + 4)) void gdn_fused_kernel(Args A) {
 }
 
 // Start states of the exact segments 2 .. N-1 (between the two launches):
-// S_start(j + 1) = Phi_j S_start(j) + Bseg_j from S_start(1) = segment 0's end
-// state.  The composition is independent per state column, so each head's
+// S_start(j + 1) = gam_j S_start(j) + E_j S_start(j) + Bseg_j from S_start(1)
+// = segment 0's end state.  The composition is independent per state column, so each head's
 // 128 columns are split over 8 / NW workgroups of NW wavefronts (the
-// workgroups of one head on one XCD, so that its Phi images are read from
+// workgroups of one head on one XCD, so that its E images are read from
 // HBM once): wavefront w keeps 16 columns of the state in registers, the
-// workgroup loads each Phi_j (as its hi and lo bf16 images) into LDS by
+// workgroup loads each E_j (as its hi and lo bf16 images) into LDS by
 // direct-to-LDS loads while the product with the previous one runs, and
 // each composition is written over the columns of Bseg_j it read.  LDS holds an image row r as 16 granules of 16 bytes,
 // granule p at position p ^ phi_swz(r): the 16 rows one operand read
@@ -1016,7 +1034,7 @@ __global__ __launch_bounds__(64 * NW) void gdn_compose_kernel(Args A) {
   const int nseg = A.nseg;
   float* const ws_head = A.ws + (size_t)bh * (2 * nseg - 3) * kStateFloats;
   auto slot = [&](int idx) { return ws_head + (size_t)idx * kStateFloats; };
-  // Phi_j into image buf: 64 windows of 1 KB (four rows each; 0-31 hi,
+  // E_j into image buf: 64 windows of 1 KB (four rows each; 0-31 hi,
   // 32-63 lo), wavefront w issuing windows w, w + NW, ..
   auto fetch = [&](int j, int buf) {
     const float* src = slot(1 + 2 * (j - 1));
@@ -1046,7 +1064,7 @@ __global__ __launch_bounds__(64 * NW) void gdn_compose_kernel(Args A) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) dst[acc_row(kb, g, r) * DV + col0 + ln] = src[kb][r];
   };
-  const int last = nseg - 2;  // maps Phi_1 .. Phi_last
+  const int last = nseg - 2;  // maps 1 .. last
   f32x4 s[8], bn[8];
 #pragma unroll
   for (int kb = 0; kb < 8; ++kb)
@@ -1054,15 +1072,19 @@ __global__ __launch_bounds__(64 * NW) void gdn_compose_kernel(Args A) {
     for (int r = 0; r < 4; ++r) s[kb][r] = slot(0)[acc_row(kb, g, r) * DV + col0 + ln];
   fetch(1, 0);
   load_b(bn, 1);
+  float gam = *ws_decay(A, bh, 1), gam_next = 0.0f;
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
   __syncthreads();
   for (int j = 1; j <= last; ++j) {
     f32x4 acc[8];
 #pragma unroll
-    for (int kb = 0; kb < 8; ++kb) acc[kb] = bn[kb];
+    for (int kb = 0; kb < 8; ++kb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[kb][r] = fmaf(gam, s[kb][r], bn[kb][r]);
     if (j + 1 <= last) {
       fetch(j + 1, j & 1);
       load_b(bn, j + 1);
+      gam_next = *ws_decay(A, bh, j + 1);
     }
     if (j > 1) store_s(s, j - 1);
     const bf16* phi_hi = phi_s[(j - 1) & 1];
@@ -1087,7 +1109,8 @@ __global__ __launch_bounds__(64 * NW) void gdn_compose_kernel(Args A) {
     }
 #pragma unroll
     for (int kb = 0; kb < 8; ++kb) s[kb] = acc[kb];
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the next Phi and B have landed
+    gam = gam_next;
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the next E, B and decay have landed
     __syncthreads();
   }
   store_s(s, last);
@@ -1130,7 +1153,9 @@ static int plan_segments(int64_t BH, int64_t nc, int requested) {
 }
 
 inline size_t ws_bytes_for(int64_t BH, int nseg) {
-  return nseg <= 1 ? 0 : (size_t)BH * (size_t)(2 * nseg - 3) * kStateFloats * sizeof(float);
+  if (nseg <= 1) return 0;
+  const size_t floats = (size_t)(2 * nseg - 3) * kStateFloats + (nseg > 2 ? nseg : 0);
+  return (size_t)BH * floats * sizeof(float);
 }
 
 // Argument checks shared by the entry points (0 when the call may proceed).
@@ -1213,7 +1238,8 @@ static int run(const bf16* q, const bf16* k, const bf16* v, const float* g, cons
 
 // Scratch of the allocation-free entry point: one array per GPU, holding
 // the segment maps of the call in flight.  kScratchBytes bounds the
-// segments: B * H * (2 N - 3) states of 64 KiB must fit (N = 1 needs none).
+// segments: B * H * (2 N - 3) states of 64 KiB and B * H * N decays must fit
+// (N = 1 needs none).
 constexpr size_t kScratchBytes = (size_t)32 << 20;
 __device__ __align__(256) uint8_t scratch[kScratchBytes];
 
