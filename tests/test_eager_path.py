@@ -24,6 +24,38 @@ def test_plain_calls():
         assert _seen(x)
 
 
+@pytest.mark.parametrize("make", [
+    lambda: torch.full((1, 1), 2 + 3j).conj().imag,  # negative bit, contiguous
+    lambda: torch._neg_view(torch.ones(4, 64)),
+    lambda: torch._efficientzerotensor((3,)),
+], ids=["conj_imag", "neg_view", "zerotensor"])
+def test_lazy_tensors_take_the_custom_op(make):
+    # the storage does not hold the values: the dispatcher materialises them
+    # for the custom op, a raw pointer would be read as it lies
+    x = make()
+    assert x.is_contiguous()
+    assert not _seen(x) and not _seen(torch.ones(3), x)
+    got = []
+
+    @torch.library.custom_op("tileops_test::eager_probe", mutates_args=())
+    def probe(t: torch.Tensor) -> torch.Tensor:
+        got.append((t.is_neg(), t._is_zerotensor()))
+        return t.clone()
+
+    assert torch.equal(probe(x), x + 0) and got == [(False, False)]
+
+
+@pytest.mark.gpu
+def test_negative_views_on_the_gpu():
+    from tileops.ops.reduction import ArgmaxFwdOp, LogSumExpFwdOp
+
+    x = torch.randn(5, 64, generator=torch.Generator().manual_seed(3)).cuda()
+    neg = torch._neg_view(x)
+    assert torch.equal(LogSumExpFwdOp(dtype=torch.float32)(neg),
+                       LogSumExpFwdOp(dtype=torch.float32)(-x))
+    assert torch.equal(ArgmaxFwdOp(dtype=torch.float32, dim=-1)(neg), torch.argmin(x, dim=-1))
+
+
 class _Sub(torch.Tensor):
     pass
 

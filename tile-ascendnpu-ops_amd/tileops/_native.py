@@ -210,9 +210,11 @@ def eager(*tensors: torch.Tensor) -> bool:
     The custom op exists for everything that must see one opaque operator:
     compilation and tracing, dispatch and function modes (fake tensors among
     them), tensor subclasses, functorch transforms, forward-mode and
-    reverse-mode autograd.  A plain eager call is none of these and gets the
-    same result from the launch function; the dispatcher's Python round trip
-    costs it about 7 us (Argmax [4, 128]: 17.0 -> 9.8 us per call).
+    reverse-mode autograd, and lazy negations and zeros, whose storage does not
+    hold the values until the dispatcher resolves them.  A plain eager call is
+    none of these and gets the same result from the launch function; the
+    dispatcher's Python round trip costs it about 7 us (Argmax [4, 128]: 17.0 ->
+    9.8 us per call).
     """
     if (
         torch.compiler.is_compiling()
@@ -225,7 +227,7 @@ def eager(*tensors: torch.Tensor) -> bool:
         return False
     grad = torch.is_grad_enabled()
     for t in tensors:
-        if type(t) not in _PLAIN or (grad and t.requires_grad):
+        if type(t) not in _PLAIN or (grad and t.requires_grad) or t.is_neg() or t._is_zerotensor():
             return False
     return True
 
