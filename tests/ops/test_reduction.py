@@ -368,3 +368,21 @@ def test_logsumexp_over_several_dims(shape, dims, dtype):
     y = LogSumExpFwdOp(dtype=dtype, dim=dims)(x)
     atol, rtol = ref_tolerance(dtype)
     assert_close_np(to_np(y), torch.logsumexp(x.double(), dims).cpu().numpy(), atol, rtol, "lse")
+
+
+def test_strided_form_leaves_large_sizes_to_the_general_path():
+    # a size past the entry point's 31 bits, wherever it stands; the largest
+    # sizes below it are taken
+    from tileops.ops._multidim import strided_form
+
+    def form(shape, dims):
+        return strided_form(torch.empty(shape, device="meta"), dims)
+
+    big = 2**31
+    for shape, dims in (((2, big), [0]), ((big, 2, 64), [1]), ((2, big, 64), [1]),
+                        ((2, 3, big), [0, 1]), ((2, big, 64), [0, 2]), ((2, 3, big // 2), [0, 2])):
+        assert form(shape, dims) is None, (shape, dims)
+    assert form((2, big - 1), [0]) == (1, 2, big - 1, False)
+    assert form((big - 1, 2, 64), [1]) == (big - 1, 2, 64, False)
+    assert form((2, big - 1, 64), [0, 2]) == (2, big - 1, 64, True)
+    assert form((2, 3, big // 2 - 1), [0, 2]) == (2, 3, big // 2 - 1, True)

@@ -63,21 +63,23 @@ def strided_form(x: torch.Tensor, dims: list[int]) -> "tuple[int, int, int, bool
 
     Below 64 neighbouring columns (or, for ``ends``, rows of 64 elements) the
     strided reads leave most of a wavefront idle and the copy is kept; ``ends``
-    merges ``outer`` partials per output on one wavefront, which bounds it.
+    merges ``outer`` partials per output on one wavefront, which bounds it.  As
+    on the general path at most 2^31 - 1 elements are reduced to one, and the
+    entry point takes each of the three sizes below 2^31.
     """
     if not x.is_contiguous() or x.numel() == 0 or not dims:
         return None
     shape, lo, hi = x.shape, dims[0], dims[-1]
     if hi - lo + 1 == len(dims):  # one run of reduced dims
         outer, n, inner = prod(shape[:lo]), prod(shape[lo:hi + 1]), prod(shape[hi + 1:])
-        if inner < 64 or n >= 2**31 or outer * ((inner + 15) // 16) >= 2**31:
+        if inner < 64 or max(outer, n, inner) >= 2**31:
             return None
         return outer, n, inner, False
     kept = [i for i in range(lo, hi + 1) if i not in dims]
     if lo == 0 and hi == x.ndim - 1 and kept[-1] - kept[0] + 1 == len(kept):
         outer, n = prod(shape[:kept[0]]), prod(shape[kept[0]:kept[-1] + 1])
         inner = prod(shape[kept[-1] + 1:])
-        if inner < 64 or inner >= 2**31 or outer > 16384:
+        if inner < 64 or max(n, outer * inner) >= 2**31 or outer > 16384:
             return None
         return outer, n, inner, True
     return None
