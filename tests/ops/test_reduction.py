@@ -386,3 +386,33 @@ def test_strided_form_leaves_large_sizes_to_the_general_path():
     assert form((big - 1, 2, 64), [1]) == (big - 1, 2, 64, False)
     assert form((2, big - 1, 64), [0, 2]) == (2, big - 1, 64, True)
     assert form((2, 3, big // 2 - 1), [0, 2]) == (2, 3, big // 2 - 1, True)
+
+
+def _windows(n):
+    """The ends, and around multiples of 2^24 workgroups of 4 to 64 rows."""
+    at = [0, n - 100] + [k for e in (24, 26, 28, 30) for k in (2**e - 50,) if k + 100 < n]
+    return [slice(i, i + 100) for i in at]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape, dim, dtype", [
+    ((2**28 + 40, 5), -1, torch.float16),     # short rows, sixteen to a workgroup
+    ((2, 2**31 + 64), 0, torch.bfloat16),     # copied, short rows past 2^31
+    ((2**24 + 3, 2, 64), 1, torch.bfloat16),  # a column workgroup per outer slice
+    ((2, 2**26 + 9, 64), [0, 2], torch.float16),  # merged from partials
+])
+def test_reductions_of_more_rows_than_one_launch_holds(shape, dim, dtype):
+    # 2^32 threads and more: each launch goes in slices
+    if torch.cuda.mem_get_info()[0] < 40 << 30:
+        pytest.skip("needs 40 GB of device memory")
+    x = torch.empty(shape, device="cuda", dtype=dtype).normal_()
+    y = LogSumExpFwdOp(dtype=dtype, dim=dim)(x)
+    i = ArgmaxFwdOp(dtype=dtype, dim=dim)(x) if isinstance(dim, int) else None
+    kept = 1 if dim == 0 or not isinstance(dim, int) else 0
+    atol, rtol = ref_tolerance(dtype)
+    for w in _windows(x.shape[kept]):
+        part = x[:, w] if kept == 1 else x[w]
+        ref = torch.logsumexp(part.double(), dim).cpu().numpy()
+        assert_close_np(to_np(y[w]), ref, atol, rtol, f"lse {w}")
+        if i is not None:
+            assert torch.equal(i[w].cpu(), torch.argmax(part.cpu(), dim=dim))

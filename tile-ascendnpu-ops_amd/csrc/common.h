@@ -109,6 +109,19 @@ inline int launch_status() {
   return e == hipSuccess ? 0 : (int)e;
 }
 
+// A one-shot grid of `blocks` workgroups: HIP refuses 2^32 threads and more in
+// one dimension of a launch, so that larger grids go in slices,
+// launch(first workgroup, workgroups).
+template <typename F>
+inline int launch_slices(int64_t blocks, int threads, F&& launch) {
+  const int64_t most = (int64_t)UINT32_MAX / threads;
+  for (int64_t b0 = 0; b0 < blocks; b0 += most) {
+    launch(b0, dim3((unsigned)(blocks - b0 < most ? blocks - b0 : most)));
+    if (int e = launch_status()) return e;
+  }
+  return 0;
+}
+
 }  // namespace tileops
 
 namespace tileops {

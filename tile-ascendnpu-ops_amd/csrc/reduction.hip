@@ -282,10 +282,10 @@ __global__ __launch_bounds__(WPR > 4 ? 64 * WPR : 256) void row_reduce_kernel(
 template <typename T, int OP, int G, bool PACKS, bool ALIGNED>
 __global__ __launch_bounds__(256) void short_row_kernel(const T* __restrict__ x,
                                                         void* __restrict__ out, int64_t M, int N,
-                                                        PartMap pm) {
+                                                        PartMap pm, int64_t block0) {
   constexpr int V = PACKS ? Elem<T>::kVec : 1, EDGE = PACKS && !ALIGNED ? 2 : 0;
   static_assert(EDGE == 0 || G >= Elem<T>::kVec, "a lane per edge element");
-  const int64_t row = (int64_t)blockIdx.x * (256 / G) + threadIdx.x / G;
+  const int64_t row = (block0 + blockIdx.x) * (256 / G) + threadIdx.x / G;
   const int lane = threadIdx.x % G;
   typename RowState<OP>::S st = row_init<OP>();
   if (row < M) {
@@ -340,14 +340,22 @@ __global__ __launch_bounds__(256) void short_row_kernel(const T* __restrict__ x,
 template <typename T, int OP>
 __global__ __launch_bounds__(256) void merge_partials_kernel(
     const typename RowState<OP>::S* __restrict__ part, void* __restrict__ out, int64_t M,
-    int nsplit) {
+    int nsplit, int64_t block0) {
   const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int64_t row = (block0 + blockIdx.x) * 4 + (threadIdx.x >> 6);
   if (row >= M) return;
   typename RowState<OP>::S st = row_init<OP>();
   for (int i = lane; i < nsplit; i += 64) st = row_merge<OP>(st, part[row * nsplit + i]);
   st = row_wave<OP>(st);
   if (lane == 0) row_store<T, OP>(out, row, st);
+}
+
+template <typename T, int OP>
+static int launch_merge(const void* ws, void* out, int64_t M, int nsplit, hipStream_t s) {
+  return launch_slices((M + 3) / 4, 256, [&](int64_t block0, dim3 grid) {
+    merge_partials_kernel<T, OP><<<grid, dim3(256), 0, s>>>(
+        static_cast<const typename RowState<OP>::S*>(ws), out, M, nsplit, block0);
+  });
 }
 
 // How a [M, N] row reduction is laid out.  One wavefront per row from 3072
@@ -403,29 +411,31 @@ static void launch_rows_u(const T* x, void* out, int64_t M, int64_t N, const Row
   else launch_rows<T, OP, WPR, 4>(x, out, M, N, p, pm, s);
 }
 
-// The short-row kernel where it applies: rows of at most 64 packs.  Ragged
-// rows of up to 16 elements go element by element.
+// The short-row kernel takes rows of at most 64 packs; ragged rows of up to 16
+// elements go element by element.
+static bool short_rows(int64_t N, int vec) { return N / vec <= 64; }
+
 template <typename T, int OP>
-static bool try_short(const T* x, void* out, int64_t M, int64_t N, PartMap pm, hipStream_t s) {
+static int launch_short(const T* x, void* out, int64_t M, int64_t N, PartMap pm, hipStream_t s) {
   constexpr int V = Elem<T>::kVec;
-  if (N / V > 64 || M > (int64_t)INT32_MAX) return false;  // four rows per workgroup at worst
   const int n = (int)N, np = n / V;
-  const dim3 block(256);
-  auto grid = [&](int G) { return dim3((unsigned)((M + 256 / G - 1) / (256 / G))); };
+  auto go = [&](auto kernel, int G) {
+    const int64_t rows = 256 / G;
+    return launch_slices((M + rows - 1) / rows, 256, [&](int64_t block0, dim3 grid) {
+      kernel<<<grid, dim3(256), 0, s>>>(x, out, M, n, pm, block0);
+    });
+  };
   if (host_aligned16(x) && n % V == 0) {
-    if (np <= 4) short_row_kernel<T, OP, 4, true, true><<<grid(4), block, 0, s>>>(x, out, M, n, pm);
-    else if (np <= 16) short_row_kernel<T, OP, 16, true, true><<<grid(16), block, 0, s>>>(x, out, M, n, pm);
-    else if (np <= 32) short_row_kernel<T, OP, 32, true, true><<<grid(32), block, 0, s>>>(x, out, M, n, pm);
-    else short_row_kernel<T, OP, 64, true, true><<<grid(64), block, 0, s>>>(x, out, M, n, pm);
-  } else if (n <= 16) {
-    if (n <= 4) short_row_kernel<T, OP, 4, false, false><<<grid(4), block, 0, s>>>(x, out, M, n, pm);
-    else short_row_kernel<T, OP, 16, false, false><<<grid(16), block, 0, s>>>(x, out, M, n, pm);
-  } else {
-    if (np <= 16) short_row_kernel<T, OP, 16, true, false><<<grid(16), block, 0, s>>>(x, out, M, n, pm);
-    else if (np <= 32) short_row_kernel<T, OP, 32, true, false><<<grid(32), block, 0, s>>>(x, out, M, n, pm);
-    else short_row_kernel<T, OP, 64, true, false><<<grid(64), block, 0, s>>>(x, out, M, n, pm);
+    if (np <= 4) return go(short_row_kernel<T, OP, 4, true, true>, 4);
+    if (np <= 16) return go(short_row_kernel<T, OP, 16, true, true>, 16);
+    if (np <= 32) return go(short_row_kernel<T, OP, 32, true, true>, 32);
+    return go(short_row_kernel<T, OP, 64, true, true>, 64);
   }
-  return true;
+  if (n <= 4) return go(short_row_kernel<T, OP, 4, false, false>, 4);
+  if (n <= 16) return go(short_row_kernel<T, OP, 16, false, false>, 16);
+  if (np <= 16) return go(short_row_kernel<T, OP, 16, true, false>, 16);
+  if (np <= 32) return go(short_row_kernel<T, OP, 32, true, false>, 32);
+  return go(short_row_kernel<T, OP, 64, true, false>, 64);
 }
 
 // Rows of x[M, N]; with keep > 0 rows r, r + keep, .. belong to output r
@@ -441,20 +451,16 @@ static int launch_row_reduce(const void* xv, void* out, int64_t M, int64_t N, in
   if (folds == 1 && p.nsplit > 1 && ws_bytes < (size_t)M * p.nsplit * sizeof(S))
     p = plan_rows(M, N, Elem<T>::kVec, false);  // no scratch
   PartMap pm{nout, 0};
-  const bool is_short = N / Elem<T>::kVec <= 64 && M <= (int64_t)INT32_MAX;
+  const bool is_short = short_rows(N, Elem<T>::kVec);
   if (folds > 1 || (p.nsplit > 1 && !is_short)) pm.per = (int)folds * (is_short ? 1 : p.nsplit);
   void* dst = pm.per > 0 ? ws : out;
-  if (!try_short<T, OP>(x, dst, M, N, pm, s)) {
-    if (p.wpr == 1) launch_rows_u<T, OP, 1>(x, dst, M, N, p, pm, s);
-    else if (p.wpr == 4) launch_rows_u<T, OP, 4>(x, dst, M, N, p, pm, s);
-    else launch_rows<T, OP, 16, 4>(x, dst, M, N, p, pm, s);
-  }
-  if (pm.per > 0) {
-    if (int e = launch_status()) return e;
-    merge_partials_kernel<T, OP><<<dim3((unsigned)((nout + 3) / 4)), dim3(256), 0, s>>>(
-        static_cast<const S*>(ws), out, nout, pm.per);
-  }
-  return launch_status();
+  int e = 0;
+  if (is_short) e = launch_short<T, OP>(x, dst, M, N, pm, s);
+  else if (p.wpr == 1) launch_rows_u<T, OP, 1>(x, dst, M, N, p, pm, s);
+  else if (p.wpr == 4) launch_rows_u<T, OP, 4>(x, dst, M, N, p, pm, s);
+  else launch_rows<T, OP, 16, 4>(x, dst, M, N, p, pm, s);
+  if (e || (e = launch_status())) return e;
+  return pm.per > 0 ? launch_merge<T, OP>(ws, out, nout, pm.per, s) : 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -470,12 +476,14 @@ static int launch_row_reduce(const void* xv, void* out, int64_t M, int64_t N, in
 template <typename T, int OP, int V, int TX>
 __global__ __launch_bounds__(256) void col_reduce_kernel(const T* __restrict__ x,
                                                          void* __restrict__ out, int64_t N,
-                                                         int64_t inner, int64_t ntile, int nsplit) {
+                                                         int64_t inner, int64_t ntile, int nsplit,
+                                                         int64_t block0) {
   typedef typename RowState<OP>::S S;
   constexpr int TY = 256 / TX, U = 4;
   const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
-  const int64_t tile = blockIdx.x % ntile;
-  const int64_t rest = blockIdx.x / ntile;
+  const int64_t block = block0 + blockIdx.x;
+  const int64_t tile = block % ntile;
+  const int64_t rest = block / ntile;
   const int split = (int)(rest % nsplit);
   const int64_t o = rest / nsplit;
   const int64_t c0 = (tile * TX + tx) * V;
@@ -570,39 +578,32 @@ static ColPlan plan_cols(int64_t outer, int64_t N, int64_t inner, int vec, bool 
 }
 
 template <typename T, int OP, int V>
-static void launch_cols(const T* x, void* out, int64_t outer, int64_t N, int64_t inner,
-                        const ColPlan& p, hipStream_t s) {
-  const dim3 grid((unsigned)(p.ntile * p.nsplit * outer)), block(256);
-  if (p.tx == 256)
-    col_reduce_kernel<T, OP, V, 256><<<grid, block, 0, s>>>(x, out, N, inner, p.ntile, p.nsplit);
-  else if (p.tx == 64)
-    col_reduce_kernel<T, OP, V, 64><<<grid, block, 0, s>>>(x, out, N, inner, p.ntile, p.nsplit);
-  else
-    col_reduce_kernel<T, OP, V, 16><<<grid, block, 0, s>>>(x, out, N, inner, p.ntile, p.nsplit);
+static int launch_cols(const T* x, void* out, int64_t outer, int64_t N, int64_t inner,
+                       const ColPlan& p, hipStream_t s) {
+  auto go = [&](auto kernel) {
+    return launch_slices(p.ntile * p.nsplit * outer, 256, [&](int64_t block0, dim3 grid) {
+      kernel<<<grid, dim3(256), 0, s>>>(x, out, N, inner, p.ntile, p.nsplit, block0);
+    });
+  };
+  if (p.tx == 256) return go(col_reduce_kernel<T, OP, V, 256>);
+  if (p.tx == 64) return go(col_reduce_kernel<T, OP, V, 64>);
+  return go(col_reduce_kernel<T, OP, V, 16>);
 }
 
 template <typename T, int OP>
 static int launch_col_reduce(const void* xv, void* out, int64_t outer, int64_t N, int64_t inner,
                              void* ws, hipStream_t s) {
-  typedef typename RowState<OP>::S S;
   const T* x = static_cast<const T*>(xv);
   ColPlan p = plan_cols(outer, N, inner, Elem<T>::kVec, OP != 0);
-  if (p.ntile * p.nsplit * outer > (int64_t)INT32_MAX) return TILEOPS_ESHAPE;
-  if (p.v > 1 && !host_aligned16(x)) {  // same grid, one column per thread
+  if (p.v > 1 && !host_aligned16(x)) {  // one column per thread
     p.v = 1;
     p.ntile = (inner + p.tx - 1) / p.tx;
-    if (p.ntile * p.nsplit * outer > (int64_t)INT32_MAX) return TILEOPS_ESHAPE;
   }
   void* dst = p.nsplit > 1 ? ws : out;
-  if (p.v > 1) launch_cols<T, OP, Elem<T>::kVec>(x, dst, outer, N, inner, p, s);
-  else launch_cols<T, OP, 1>(x, dst, outer, N, inner, p, s);
-  if (p.nsplit > 1) {
-    if (int e = launch_status()) return e;
-    const int64_t nout = outer * inner;
-    merge_partials_kernel<T, OP><<<dim3((unsigned)((nout + 3) / 4)), dim3(256), 0, s>>>(
-        static_cast<const S*>(ws), out, nout, p.nsplit);
-  }
-  return launch_status();
+  const int e = p.v > 1 ? launch_cols<T, OP, Elem<T>::kVec>(x, dst, outer, N, inner, p, s)
+                        : launch_cols<T, OP, 1>(x, dst, outer, N, inner, p, s);
+  if (e || p.nsplit == 1) return e;
+  return launch_merge<T, OP>(ws, out, outer * inner, p.nsplit, s);
 }
 
 // One call: x[outer, n, inner].  kRows: rows of `inner` (outer 1); kAxis: over
@@ -659,8 +660,7 @@ static int reduce_rows(int op, const void* x, void* y, int64_t M, int64_t N, int
 
 static size_t rows_bytes(int64_t M, int64_t N, int vec, int64_t folds) {
   static_assert(sizeof(LseState) == 8 && sizeof(ArgState) == 8, "partials of 8 bytes");
-  const bool is_short = N / vec <= 64 && M <= (int64_t)INT32_MAX;
-  const int nsplit = is_short ? 1 : plan_rows(M, N, vec).nsplit;
+  const int nsplit = short_rows(N, vec) ? 1 : plan_rows(M, N, vec).nsplit;
   return folds > 1 || nsplit > 1 ? (size_t)M * nsplit * 8 : 0;
 }
 
