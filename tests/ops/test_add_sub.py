@@ -87,3 +87,18 @@ def test_add_sub_storage_offset_operands(op_cls, sign, dtype):
     y = op_cls(input=(96 * 64,), other=(96 * 64,), dtype=dtype)(
         torch.randn(96 * 64, device="cuda").to(dtype), base[1:])
     assert y.shape == (96 * 64,)
+
+
+@pytest.mark.gpu
+def test_broadcast_of_more_packs_than_one_launch_holds():
+    # 2^33 packs, two to a thread: the launch goes in slices
+    rows, cols = 2**18 + 8, 2**18
+    if torch.cuda.mem_get_info()[0] < 140 << 30:
+        pytest.skip("needs 140 GB of device memory")
+    a = torch.randn(rows, 1, device="cuda", dtype=torch.bfloat16)
+    b = torch.randn(1, cols, device="cuda", dtype=torch.bfloat16)
+    y = AddFwdOp(input=(rows, 1), other=(1, cols), dtype=torch.bfloat16)(a, b)
+    for i in (0, 1, 2**17 - 1, 2**17, 2**18 - 1, 2**18, rows - 1):
+        assert torch.equal(y[i], a[i] + b[0]), i
+    del y
+    torch.cuda.empty_cache()

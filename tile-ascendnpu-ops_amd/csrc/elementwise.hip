@@ -569,13 +569,14 @@ __global__ __launch_bounds__(256) void bcast_inner_kernel(const T* __restrict__ 
                                                           T* __restrict__ y, I npack,
                                                           I row_packs, float p, BcastDesc d,
                                                           int vec_mask, int bc_mask,
-                                                          int flat_mask, BcastDivs dv) {
+                                                          int flat_mask, BcastDivs dv,
+                                                          I block0) {
   constexpr int V = Elem<T>::kVec;
   constexpr int NOP = BcastArity<OP>::n;
   const T* src[3] = {a, b, w};
   const int nd = d.ndim;  // >= 1; dimension nd - 1 is the row
   constexpr int U = kInnerPacks;
-  const I pk0 = (I)blockIdx.x * (256 * U) + threadIdx.x;
+  const I pk0 = (block0 + (I)blockIdx.x) * (256 * U) + threadIdx.x;
   Pack<T> in[U][3];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
@@ -743,10 +744,11 @@ static void coalesce_dims(BcastDesc& d, int nop) {
 
 // The pack kernel applies when the row length is a whole number of packs,
 // each operand's row is unit-stride (16-byte aligned base and row offsets) or
-// broadcast, and the output is 16-byte aligned.  Returns false otherwise.
+// broadcast, and the output is 16-byte aligned.  Returns false otherwise, else
+// the launch's status in `status`.
 template <typename T, int OP>
 static bool launch_bcast_inner(const T* const (&src)[3], T* y, const BcastDesc& d, int64_t n,
-                               float p, hipStream_t s) {
+                               float p, hipStream_t s, int& status) {
   constexpr int V = Elem<T>::kVec;
   constexpr int NOP = BcastArity<OP>::n;
   const int nd = d.ndim;
@@ -770,16 +772,19 @@ static bool launch_bcast_inner(const T* const (&src)[3], T* y, const BcastDesc& 
     }
   }
   const int64_t npack = n / V, row_packs = d.shape[nd - 1] / V;
-  const unsigned grid = (unsigned)((npack + 256 * kInnerPacks - 1) / (256 * kInnerPacks));
+  const int64_t blocks = (npack + 256 * kInnerPacks - 1) / (256 * kInnerPacks);
   const int flat = flat_operands<T>(src, d, NOP);
   const BcastDivs dv = divisors(d, row_packs);
-  if (fits32 && npack <= (int64_t)INT32_MAX - 256 * kInnerPacks)
-    bcast_inner_kernel<T, OP, uint32_t><<<dim3(grid), dim3(256), 0, s>>>(
-        src[0], src[1], src[2], y, (uint32_t)npack, (uint32_t)row_packs, p, d, vec_mask, bc_mask,
-        flat, dv);
-  else
-    bcast_inner_kernel<T, OP, int64_t><<<dim3(grid), dim3(256), 0, s>>>(
-        src[0], src[1], src[2], y, npack, row_packs, p, d, vec_mask, bc_mask, flat, dv);
+  const bool narrow = fits32 && npack <= (int64_t)INT32_MAX - 256 * kInnerPacks;
+  status = launch_slices(blocks, 256, [&](int64_t block0, dim3 grid) {
+    if (narrow)
+      bcast_inner_kernel<T, OP, uint32_t><<<grid, dim3(256), 0, s>>>(
+          src[0], src[1], src[2], y, (uint32_t)npack, (uint32_t)row_packs, p, d, vec_mask,
+          bc_mask, flat, dv, (uint32_t)block0);
+    else
+      bcast_inner_kernel<T, OP, int64_t><<<grid, dim3(256), 0, s>>>(
+          src[0], src[1], src[2], y, npack, row_packs, p, d, vec_mask, bc_mask, flat, dv, block0);
+  });
   return true;
 }
 
@@ -831,7 +836,8 @@ static int launch_bcast(const void* av, const void* bv, const void* wv, void* yv
     }
     aligned &= host_aligned16(src[o]);
   }
-  if (!flat && launch_bcast_inner<T, OP>(src, y, d, n, p, s)) return launch_status();
+  int status = 0;
+  if (!flat && launch_bcast_inner<T, OP>(src, y, d, n, p, s, status)) return status;
   int64_t npack = 0;
   if (flat && aligned) {
     npack = n / V;
