@@ -384,7 +384,11 @@ static size_t plan_bytes(const Problem& p, const SplitPlan& s) {
 
 static bool plan_wins(const Problem& p, const SplitPlan& s) {
   if (!(p.scale > 0.0f)) return false;  // the running max is of raw scores
-  if ((int64_t)p.B * p.Hkv * s.ntile * s.nsplit > (int64_t)INT32_MAX) return false;
+  // at most 2^32 - 1 threads a launch: this kernel's and the combining one's
+  // (mha_fwd_kernel takes eight row tiles in 512 threads)
+  const int64_t wgs = (int64_t)p.B * p.Hkv * s.ntile * s.nsplit, rows = (int64_t)p.B * p.Sq * p.H;
+  if (wgs * (p.D > 128 ? 128 : 256) > (int64_t)UINT32_MAX) return false;
+  if (s.nsplit > 1 && (rows + 3) / 4 * 256 > (int64_t)UINT32_MAX) return false;
   if ((int64_t)p.Sq * (p.H / p.Hkv) > (int64_t)INT32_MAX) return false;
   if ((int64_t)p.Hkv * p.D * 2 * 32 > (int64_t)UINT32_MAX) return false;
   const double main = main_cycles(p);
