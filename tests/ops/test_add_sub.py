@@ -9,6 +9,9 @@ the kernel reads broadcast operands through zero strides, so no copy is
 made.
 """
 
+import copy
+import pickle
+
 import pytest
 import torch
 
@@ -87,6 +90,21 @@ def test_add_sub_storage_offset_operands(op_cls, sign, dtype):
     y = op_cls(input=(96 * 64,), other=(96 * 64,), dtype=dtype)(
         torch.randn(96 * 64, device="cuda").to(dtype), base[1:])
     assert y.shape == (96 * 64,)
+
+
+@pytest.mark.smoke
+def test_used_broadcast_ops_pickle_and_copy():
+    # the plans kept from earlier calls hold ctypes arrays
+    a, b = torch.randn(3, 4), torch.randn(4)
+    op = AddFwdOp(input=(3, 4), other=(4,), dtype=torch.float32)
+    op.kernel._plans["kept"] = op.kernel._plan((a, b))
+    for again in (pickle.loads(pickle.dumps(op)), copy.deepcopy(op)):
+        kernel = again.kernel
+        assert kernel.N_total == 12 and kernel.alpha == 1 and kernel._plans == {}
+        out_shape, nd, shape, strides = kernel._plan((a, b))
+        assert out_shape == (3, 4) and list(shape) == [3, 4]
+        assert [list(s) for s in strides] == [[4, 1], [0, 1]]
+    assert "kept" in op.kernel._plans
 
 
 @pytest.mark.gpu

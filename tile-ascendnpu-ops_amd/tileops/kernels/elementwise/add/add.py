@@ -54,10 +54,17 @@ class BroadcastFwdKernel(Kernel):
         self._plans: dict = {}
         self.init_config(config)
 
+    # The kept host arrays cannot be pickled and are made again on use.
+    def __getstate__(self) -> dict:
+        return {k: v for k, v in self.__dict__.items() if k != "_plans"}
+
+    def __setstate__(self, state: dict) -> None:
+        self.__dict__.update(state, _plans={})
+
     @property
     def default_config(self) -> dict:
-        # bcast_vec_kernel / bcast_inner_kernel: 256-thread workgroups, one
-        # 16-byte pack per thread; operands of up to 8 broadcast dimensions
+        # bcast_vec_kernel / bcast_inner_kernel: 256-thread workgroups, one or
+        # two 16-byte packs per thread; operands of up to 8 broadcast dimensions
         return {"threads": 256, "vector_bytes": 16, "max_dims": MAX_DIMS}
 
     def _operands(self, names: Sequence[str], tensors: Sequence[torch.Tensor]):
