@@ -12,6 +12,7 @@ import torch
 
 from oracle import tileops_oracle as orc
 from tests._util import NAMES, assert_close_np, from_np, ref_tolerance, to_np
+from tileops import _native
 from tileops.kernels.reduction.argmax import ArgreduceKernel
 from tileops.kernels.reduction.logsumexp import LogSumExpKernel
 from tileops.ops.reduction.argmax import ArgmaxFwdOp
@@ -416,3 +417,112 @@ def test_reductions_of_more_rows_than_one_launch_holds(shape, dim, dtype):
         assert_close_np(to_np(y[w]), ref, atol, rtol, f"lse {w}")
         if i is not None:
             assert torch.equal(i[w].cpu(), torch.argmax(part.cpu(), dim=dim))
+
+
+# -- the C functions with and without scratch ----------------------------------------------
+def _reduce(op, x, room):
+    """tileops_reduce_fwd of the rows of x with ``room(need)`` bytes of scratch."""
+    lib, (M, N) = _native.lib(), x.shape
+    code = _native.dtype_code(x.dtype)
+    need = lib.tileops_reduce_workspace_bytes(M, N, code)
+    room = room(need)
+    ws = torch.empty(max(room, 1), dtype=torch.uint8, device=x.device)
+    y = torch.empty(M, dtype=x.dtype if op == _native.LOGSUMEXP else torch.int64, device=x.device)
+    _native.check(lib.tileops_reduce_fwd(op, x.data_ptr(), y.data_ptr(), M, N, code,
+                                         ws.data_ptr() if room else None, room,
+                                         _native.stream_of(x)), "tileops_reduce_fwd")
+    return y, need
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M, N, dtype", [
+    (1, 600000, torch.float32),
+    (4, 131072, torch.bfloat16),   # the shortest rows that split
+    (128, 131073, torch.float16),  # the most rows, ragged
+])
+def test_rows_with_and_without_scratch(M, N, dtype):
+    x = torch.randn(M, N, device="cuda").to(dtype)
+    x[:, N // 3] = x[:, N - 2] = 30.0  # a tie: the first wins
+    atol, rtol = ref_tolerance(dtype)
+    ref = torch.logsumexp(x.double(), -1).cpu().numpy()
+    lib = _native.lib()
+    code = _native.dtype_code(dtype)
+    for room in (lambda need: 0, lambda need: need - 1, lambda need: need):
+        i, need = _reduce(_native.ARGMAX, x, room)
+        assert need > 0 and torch.equal(i.cpu(), torch.full((M,), N // 3))
+        assert torch.equal(_reduce(_native.ARGMIN, -x, room)[0], i)
+        assert_close_np(to_np(_reduce(_native.LOGSUMEXP, x, room)[0]), ref, atol, rtol, "lse")
+    i = torch.empty(M, dtype=torch.int64, device="cuda")
+    y = torch.empty(M, dtype=dtype, device="cuda")
+    s = _native.stream_of(x)
+    assert lib.tileops_argreduce_fwd(x.data_ptr(), i.data_ptr(), M, N, code, 0, s) == 0
+    assert lib.tileops_logsumexp_fwd(x.data_ptr(), y.data_ptr(), M, N, code, s) == 0
+    assert torch.equal(i.cpu(), torch.full((M,), N // 3))
+    assert_close_np(to_np(y), ref, atol, rtol, "lse without scratch")
+
+
+@pytest.mark.smoke
+def test_reduce_entry_points_reject_bad_scratch():
+    lib, p = _native.lib(), 4096  # non-null host values: refused before any launch
+    need = lib.tileops_reduce_axis_workspace_bytes(1, 1, 20000, 64, 0, 0)  # columns split
+    assert need > 0
+    axis = lib.tileops_reduce_axis_fwd
+    assert axis(1, p, p, 1, 20000, 64, 0, 0, None, 0, None) == -4
+    assert axis(1, p, p, 1, 20000, 64, 0, 0, None, need, None) == -4
+    assert axis(1, p, p, 1, 20000, 64, 0, 0, p, need - 1, None) == -4
+    assert axis(1, p, p, 1, 20000, 64, 0, 0, p + 4, need, None) == -1
+    assert axis(0, p, p, 8, 4, 64, 1, 0, None, 0, None) == -4  # both ends: merged from partials
+    assert lib.tileops_reduce_axis_workspace_bytes(0, 8, 4, 64, 1, 0) == 8 * 4 * 8
+    assert axis(1, p, p, 8, 4, 64, 1, 0, p, 1 << 20, None) == -1  # no index over both ends
+    assert axis(3, p, p, 8, 4, 64, 0, 0, None, 0, None) == -1
+    assert axis(0, p, p, 8, 0, 64, 0, 0, None, 0, None) == -2
+    assert axis(0, p, p, 8, 4, 2**31, 0, 0, None, 0, None) == -2
+    assert axis(0, None, p, 8, 4, 64, 0, 0, None, 0, None) == -3
+    rows = lib.tileops_reduce_fwd
+    assert rows(0, p, p, 4, 131072, 2, p + 8, 1 << 20, None) == -1
+    assert rows(3, p, p, 4, 64, 2, None, 0, None) == -1
+    assert rows(0, p, p, 4, 0, 2, None, 0, None) == -2
+    assert rows(0, None, None, 0, 64, 2, None, 0, None) == 0
+    # which rows split: at most 128, of 256 chunks of 64 packs and more
+    ask = lib.tileops_reduce_workspace_bytes
+    assert ask(4, 131072, 2) > 0 and ask(128, 131072, 2) > 0
+    assert ask(129, 131072, 2) == 0 and ask(4, 130560, 2) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape, dim, dtype", [
+    ((6, 131080), 1, torch.bfloat16),    # rows split over workgroups, merged
+    ((6, 600001), 1, torch.float32),     # ragged
+    ((6, 4, 128), 1, torch.float16),     # columns, few rows
+    ((2, 1000, 128), 1, torch.bfloat16),  # 16 row groups per column
+    ((20000, 128), 0, torch.float32),    # columns split, merged
+    ((20001, 65), 0, torch.float16),
+    ((70, 6, 203), [0, 2], torch.bfloat16),  # partials of short ragged rows
+    ((2, 6, 600000), [0, 2], torch.float32),  # partials of split rows
+])
+def test_special_values_in_every_plan(shape, dim, dtype):
+    # one output of each kind: all -inf, one +inf, a NaN, all the type's lowest
+    # value, the lowest with one zero, the largest value (kept finite)
+    x = torch.randn(shape, device="cuda").to(dtype)
+    dims = [dim] if isinstance(dim, int) else dim
+    kept = [d for d in range(len(shape)) if d not in dims][-1]
+    info = torch.finfo(dtype)
+
+    def put(i, all_, last=None):
+        sel = x.select(kept, i)
+        if all_ is not None:
+            sel.fill_(all_)
+        if last is not None:
+            sel.movedim([d - (d > kept) for d in dims], list(range(-len(dims), 0)))[
+                (...,) + (-1,) * len(dims)] = last
+
+    for i, (all_, last) in enumerate([(float("-inf"), None), (None, float("inf")),
+                                      (None, float("nan")), (info.min, None), (info.min, 0.0),
+                                      (0.0, info.max)]):
+        put(i, all_, last)
+    y = to_np(LogSumExpFwdOp(dtype=dtype, dim=dim)(x))
+    ref = torch.logsumexp(x.double(), dim).to(dtype).float().cpu().numpy()
+    atol, rtol = ref_tolerance(dtype)
+    assert_close_np(y, ref, atol, rtol, "lse")
+    if isinstance(dim, int):
+        assert torch.equal(ArgmaxFwdOp(dtype=dtype, dim=dim)(x).cpu(), torch.argmax(x.cpu(), dim))
