@@ -251,6 +251,20 @@ int tileops_mha_fwd_ws(const void* q, const void* k, const void* v, void* o, flo
                        void* stream);
 
 /*
+ * tileops_mha_fwd_ws with the kernel chosen by the caller: `splits` 0 as
+ * planned, -1 the kernel of 256 query rows per workgroup, 1 .. 64 the one that
+ * splits the keys, in that many splits (TILEOPS_EINVAL unless scale > 0;
+ * scratch of tileops_mha_workspace_bytes_ex with the same `splits`, 0 for one
+ * split, is required).
+ */
+size_t tileops_mha_workspace_bytes_ex(int64_t B, int64_t Sq, int64_t Skv, int64_t H, int64_t Hkv,
+                                      int64_t D, int causal, float scale, int64_t splits);
+int tileops_mha_fwd_ex(const void* q, const void* k, const void* v, void* o, float* lse, int64_t B,
+                       int64_t Sq, int64_t Skv, int64_t H, int64_t Hkv, int64_t D, int causal,
+                       float scale, float softcap, int dtype, int64_t splits, void* ws,
+                       size_t ws_bytes, void* stream);
+
+/*
  * Chunked gated delta rule (gated DeltaNet) prefill, per (b, h):
  *   S_t = exp(g_t) S_{t-1} + beta_t k_t (v_t - k_t^T exp(g_t) S_{t-1})^T
  *   o_t = scale * q_t^T S_t

@@ -12,6 +12,7 @@ import torch
 
 from oracle import tileops_oracle as orc
 from tests._util import NAMES, assert_close_np, to_np
+from tileops import _native
 from tileops.kernels.attention.multi_head_attention import GQAPrefillFwdKernel
 from tileops.ops.attention.multi_head_attention import MultiHeadAttentionFwdOp
 from tileops.workloads.attention import MhaFwdWorkload
@@ -126,6 +127,120 @@ def test_gqa_few_queries_many_keys(causal, D, dtype, B, H, Hkv, sq, skv, softcap
     kern = GQAPrefillFwdKernel(B, H, Hkv, sq, skv, D, causal, dtype, softcap=softcap)
     o, lse = kern(q, k, v)
     _check(q, k, v, o, lse, causal, softcap=softcap, rtol=CAUSAL_RTOL)
+
+
+def _forced(q, k, v, causal, splits, softcap=0.0, room=None):
+    """tileops_mha_fwd_ex: splits -1 mha_fwd_kernel, 1 .. 64 the key-split kernel,
+    0 as planned with ``room`` bytes of scratch (default: what is asked for)."""
+    lib, dev = _native.lib(), q.device
+    B, sq, H, D = q.shape
+    skv, hkv = k.shape[1], k.shape[2]
+    size = (B, sq, skv, H, hkv, D, int(causal), D**-0.5)
+    need = lib.tileops_mha_workspace_bytes_ex(*size, splits)
+    room = need if room is None else room(need)
+    ws = torch.empty(max(room, 1), dtype=torch.uint8, device=dev)
+    o = torch.full_like(q, float("nan"))
+    lse = torch.full((B, H, sq), float("nan"), device=dev)
+    code = lib.tileops_mha_fwd_ex(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(), *size, softcap,
+        _native.dtype_code(q.dtype), splits, ws.data_ptr() if room else None, room,
+        _native.stream_of(q))
+    _native.check(code, "tileops_mha_fwd_ex")
+    return o, lse, need
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("splits", [-1, 1, 3])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("D, dtype, B, H, Hkv, sq, skv, softcap", [
+    (128, torch.bfloat16, 2, 8, 2, 200, 333, 0.0),   # grouped heads, ragged
+    (128, torch.bfloat16, 1, 4, 4, 700, 700, 0.0),   # several query blocks
+    (128, torch.float16, 2, 2, 2, 1, 1000, 0.0),     # a decode step
+    (128, torch.bfloat16, 1, 4, 2, 300, 437, 2.0),   # soft-capped
+    (64, torch.float16, 1, 6, 2, 77, 300, 0.0),
+    (64, torch.bfloat16, 1, 2, 1, 513, 1100, 5.0),
+    (96, torch.bfloat16, 1, 4, 2, 300, 437, 0.0),
+    (192, torch.float16, 1, 4, 2, 300, 437, 0.0),
+    (192, torch.bfloat16, 1, 2, 2, 260, 260, 2.0),
+    (256, torch.bfloat16, 1, 4, 2, 300, 437, 0.0),
+    (256, torch.float16, 1, 2, 1, 5, 1500, 2.0),
+])
+def test_both_kernels_whichever_is_planned(splits, causal, D, dtype, B, H, Hkv, sq, skv, softcap):
+    q = torch.randn(B, sq, H, D, device="cuda", dtype=dtype) * (2 if softcap else 1)
+    k = torch.randn(B, skv, Hkv, D, device="cuda", dtype=dtype)
+    v = torch.randn(B, skv, Hkv, D, device="cuda", dtype=dtype)
+    o, lse, need = _forced(q, k, v, causal, splits, softcap)
+    assert need == (splits * B * sq * H * (D + 2) * 4 if splits > 1 else 0)
+    _check(q, k, v, o, lse, causal, _sample_pairs(B, H), softcap=softcap, rtol=CAUSAL_RTOL)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("splits", [-1, 1, 5])
+@pytest.mark.parametrize("where", ["q", "k", "v"])
+def test_nan_reaches_the_rows_that_see_it(where, splits):
+    B, H, Hkv, sq, skv, D = 1, 4, 2, 3, 900, 128
+    q, k, v = (torch.randn(B, n, h, D, device="cuda", dtype=torch.bfloat16)
+               for n, h in ((sq, H), (skv, Hkv), (skv, Hkv)))
+    # token 1 of head 0 alone; the last key of head pair 0: only token 2 sees it
+    x, at = {"q": (q, (0, 1, 0, 5)), "k": (k, (0, skv - 1, 0, 5)),
+             "v": (v, (0, skv - 1, 0, 5))}[where]
+    x[at] = float("nan")
+    o, lse, _ = _forced(q, k, v, True, splits)
+    nan = torch.zeros(o.shape, dtype=torch.bool)
+    if where == "q":
+        nan[0, 1, 0] = True
+    elif where == "k":
+        nan[0, 2, :2] = True
+    else:
+        nan[0, 2, :2, 5] = True
+    if where == "v":  # a probability of 0 times NaN: the masked rows may hold it too
+        assert o.isnan().cpu()[nan].all() and not o.isnan()[..., :5].any()
+        assert not o[:, :, 2:].isnan().any()
+    else:
+        assert torch.equal(o.isnan().cpu(), nan)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("room", [lambda need: 0, lambda need: need - 1], ids=["none", "short"])
+def test_without_scratch_no_call_is_split(room):
+    B, H, Hkv, sq, skv, D = 2, 8, 2, 1, 4000, 128
+    q, k, v = (torch.randn(B, n, h, D, device="cuda", dtype=torch.bfloat16)
+               for n, h in ((sq, H), (skv, Hkv), (skv, Hkv)))
+    o, lse, need = _forced(q, k, v, True, 0, room=room)
+    assert need > 0  # a split is planned
+    o1, lse1, _ = _forced(q, k, v, True, -1)
+    assert torch.equal(o, o1) and torch.equal(lse, lse1)
+    _check(q, k, v, o, lse, True)
+    op = GQAPrefillFwdKernel(B, H, Hkv, sq, skv, D, True, torch.bfloat16)
+    o2, lse2, _ = _forced(q, k, v, True, 0)
+    for got in (op(q, k, v), op(q, k, v)):  # the same bits each time
+        assert torch.equal(got[0], o2) and torch.equal(got[1], lse2)
+
+
+@pytest.mark.smoke
+def test_key_split_plan():
+    # which kernel a shape gets (256 compute units): decode steps and short
+    # chunks against a cache are split, prefill is not
+    ask = _native.lib().tileops_mha_workspace_bytes
+
+    def splits(B, sq, skv, H, Hkv, D, causal=1, scale=0.1):
+        need = ask(B, sq, skv, H, Hkv, D, causal, scale)
+        assert need % (B * sq * H * (D + 2) * 4) == 0
+        return need // (B * sq * H * (D + 2) * 4)
+
+    assert splits(8, 1, 8191, 32, 8, 128) > 1
+    assert splits(1, 1, 32768, 32, 8, 128) > 1
+    assert splits(1, 128, 8192, 32, 8, 128) > 1
+    assert splits(8, 1, 8191, 32, 8, 128, scale=-0.1) == 0  # the maximum is of raw scores
+    assert splits(8, 4096, 4096, 32, 32, 128) == 0
+    assert splits(4, 512, 512, 32, 32, 128) == 0
+    for bad in ((-2, 0), (65, 0), (2, 0)):  # out of range; two splits without scratch
+        p = 4096
+        code = _native.lib().tileops_mha_fwd_ex(
+            p, p, p, p, p, 1, 1, 64, 2, 2, 128, 0, 1.0, 0.0, 2, bad[0], None, 0, None)
+        assert code == (-4 if bad[0] == 2 else -2)
+    assert _native.lib().tileops_mha_fwd_ex(p, p, p, p, p, 1, 1, 64, 2, 2, 128, 0, -1.0, 0.0, 2, 1,
+                                            None, 0, None) == -1
 
 
 @pytest.mark.gpu

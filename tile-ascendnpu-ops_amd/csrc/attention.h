@@ -92,12 +92,19 @@ struct Problem {
   int dtype;
 };
 
-// The key-split kernel (attention_split.hip): whether it is planned for these
-// sizes with `ws_bytes` of scratch (SIZE_MAX: any amount), the scratch its
-// plan uses, and the launch.
-bool split_planned(const Problem& p, size_t ws_bytes);
-size_t split_workspace_bytes(const Problem& p);
-int split_launch(const Problem& p, void* ws, size_t ws_bytes, hipStream_t s);
+// The key-split kernel (attention_split.hip): its best layout for these sizes
+// (or the one with `nsplit` splits), whether it takes them, whether that layout
+// beats mha_fwd_kernel, the scratch it uses, and the launch.
+constexpr int kMaxSplit = 64;
+struct SplitPlan {
+  int ntile, nsplit;
+  double cycles;
+};
+SplitPlan split_plan(const Problem& p, int nsplit = 0);
+bool split_fits(const Problem& p, const SplitPlan& plan);
+bool split_wins(const Problem& p, const SplitPlan& plan);
+size_t split_bytes(const Problem& p, const SplitPlan& plan);
+int split_launch(const Problem& p, const SplitPlan& plan, void* ws, hipStream_t s);
 
 }  // namespace mha
 }  // namespace tileops

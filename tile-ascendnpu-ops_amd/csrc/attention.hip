@@ -783,7 +783,9 @@ static int check(const Problem& p, int64_t B, int64_t Sq, int64_t Skv, int64_t H
   return 0;
 }
 
-static int run(const Problem& p, void* ws, size_t ws_bytes, hipStream_t s) {
+// splits: 0 as planned, -1 mha_fwd_kernel, else that many key splits.
+static int run(const Problem& p, int64_t splits, void* ws, size_t ws_bytes, hipStream_t s) {
+  if (splits < -1 || splits > kMaxSplit) return TILEOPS_ESHAPE;
   if (p.B == 0 || p.Sq == 0) return 0;
   if (p.Skv == 0) return TILEOPS_ESHAPE;
   if (!p.q || !p.k || !p.v || !p.o || !p.lse) return TILEOPS_ENULL;
@@ -793,7 +795,13 @@ static int run(const Problem& p, void* ws, size_t ws_bytes, hipStream_t s) {
   // grid: (Sq / 256) query blocks x H x B (x 2 for D = 192, 256), indexed in int
   if (((p.Sq + 255LL) / 256) * p.H * p.B * (p.D >= 192 ? 2 : 1) > (int64_t)INT32_MAX)
     return TILEOPS_ESHAPE;
-  if (split_planned(p, ws ? ws_bytes : 0)) return split_launch(p, ws, ws ? ws_bytes : 0, s);
+  if (splits >= 0) {
+    const SplitPlan split = split_plan(p, (int)splits);
+    const bool room = split_bytes(p, split) <= (ws ? ws_bytes : 0);
+    if (splits > 0 && !split_fits(p, split)) return TILEOPS_EINVAL;
+    if (splits > 0 && !room) return TILEOPS_EWORKSPACE;
+    if (splits > 0 || (room && split_wins(p, split))) return split_launch(p, split, ws, s);
+  }
   if (p.dtype == TILEOPS_BF16)
     return dispatch_d<bf16>(p.D, p.q, p.k, p.v, p.o, p.lse, p.B, p.Sq, p.Skv, p.H, p.Hkv,
                             p.causal, p.scale, p.softcap, s);
@@ -804,23 +812,38 @@ static int run(const Problem& p, void* ws, size_t ws_bytes, hipStream_t s) {
 }  // namespace mha
 }  // namespace tileops
 
-extern "C" size_t tileops_mha_workspace_bytes(int64_t B, int64_t Sq, int64_t Skv, int64_t H,
-                                              int64_t Hkv, int64_t D, int causal, float scale) {
+extern "C" size_t tileops_mha_workspace_bytes_ex(int64_t B, int64_t Sq, int64_t Skv, int64_t H,
+                                                 int64_t Hkv, int64_t D, int causal, float scale,
+                                                 int64_t splits) {
   const mha::Problem p{nullptr, nullptr, nullptr, nullptr, nullptr, (int)B, (int)Sq, (int)Skv,
                        (int)H, (int)Hkv, (int)D, causal != 0, scale, 0.0f, TILEOPS_BF16};
   if (mha::check(p, B, Sq, Skv, H, Hkv, D, causal, 0.0f, TILEOPS_BF16)) return 0;
-  if (B == 0 || Sq == 0 || Skv == 0) return 0;
-  return mha::split_workspace_bytes(p);
+  if (B == 0 || Sq == 0 || Skv == 0 || splits < 0 || splits > mha::kMaxSplit) return 0;
+  const mha::SplitPlan split = mha::split_plan(p, (int)splits);
+  return splits > 0 || mha::split_wins(p, split) ? mha::split_bytes(p, split) : 0;
+}
+
+extern "C" size_t tileops_mha_workspace_bytes(int64_t B, int64_t Sq, int64_t Skv, int64_t H,
+                                              int64_t Hkv, int64_t D, int causal, float scale) {
+  return tileops_mha_workspace_bytes_ex(B, Sq, Skv, H, Hkv, D, causal, scale, 0);
+}
+
+extern "C" int tileops_mha_fwd_ex(const void* q, const void* k, const void* v, void* o, float* lse,
+                                  int64_t B, int64_t Sq, int64_t Skv, int64_t H, int64_t Hkv,
+                                  int64_t D, int causal, float scale, float softcap, int dtype,
+                                  int64_t splits, void* ws, size_t ws_bytes, void* stream) {
+  const mha::Problem p{q, k, v, o, lse, (int)B, (int)Sq, (int)Skv, (int)H, (int)Hkv, (int)D,
+                       causal != 0, scale, softcap, dtype};
+  if (int e = mha::check(p, B, Sq, Skv, H, Hkv, D, causal, softcap, dtype)) return e;
+  return mha::run(p, splits, ws, ws_bytes, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int tileops_mha_fwd_ws(const void* q, const void* k, const void* v, void* o, float* lse,
                                   int64_t B, int64_t Sq, int64_t Skv, int64_t H, int64_t Hkv,
                                   int64_t D, int causal, float scale, float softcap, int dtype,
                                   void* ws, size_t ws_bytes, void* stream) {
-  const mha::Problem p{q, k, v, o, lse, (int)B, (int)Sq, (int)Skv, (int)H, (int)Hkv, (int)D,
-                       causal != 0, scale, softcap, dtype};
-  if (int e = mha::check(p, B, Sq, Skv, H, Hkv, D, causal, softcap, dtype)) return e;
-  return mha::run(p, ws, ws_bytes, static_cast<hipStream_t>(stream));
+  return tileops_mha_fwd_ex(q, k, v, o, lse, B, Sq, Skv, H, Hkv, D, causal, scale, softcap, dtype,
+                            0, ws, ws_bytes, stream);
 }
 
 extern "C" int tileops_mha_fwd(const void* q, const void* k, const void* v, void* o, float* lse,

@@ -329,13 +329,6 @@ __global__ __launch_bounds__(256) void mha_combine_kernel(SplitArgs A) {
 // 36 measured shapes of 4 to 660 us).  The split kernel is taken where it is
 // expected to be at least 10 % faster; on none of those shapes it was slower.
 // ---------------------------------------------------------------------------
-struct SplitPlan {
-  int ntile, nsplit;
-  double cycles;
-};
-
-constexpr int kMaxSplit = 64;
-
 // What an eager call of `cycles` on the GPU costs: it is no shorter than its
 // host path, ~10.4 us with one launch and ~14.5 with two and scratch.  Equal
 // costs go by the GPU time.
@@ -358,31 +351,37 @@ static double main_cycles(const Problem& p) {
 // mha_split_kernel: a step is one 32-key block per wavefront, bound by its
 // share of HBM (2600 bytes a cycle over the chip, a block read once for all
 // row tiles) or of L2 (16 bytes a cycle per CU).
-static SplitPlan split_plan(const Problem& p) {
+SplitPlan split_plan(const Problem& p, int nsplit) {
   const int64_t R = (int64_t)p.Sq * (p.H / p.Hkv);
   SplitPlan best{(int)((R + 31) / 32), 1, 1e30};
+  if (nsplit > 0) {
+    best.nsplit = nsplit;
+    return best;
+  }
   const int64_t base = (int64_t)p.B * p.Hkv * best.ntile;
   const int nb = (p.Skv + 31) / 32;
   const int nw = p.D > 128 ? 2 : 4, wgs = p.D <= 64 ? 2 : 1;
   const int64_t cus = device_cu_count(), slots = cus * wgs;
   const double bytes = 32.0 * (p.D <= 64 ? 64 : p.D <= 128 ? 128 : 256) * 4 * nw;
+  const double l2 = bytes * wgs / 16.0, hbm = bytes / 2600.0 / best.ntile;
+  double least = 0.0;  // call_cost of `best`
   for (int ns = 1; ns <= kMaxSplit && ns <= (nb + nw - 1) / nw; ++ns) {
     const int64_t wg = base * ns, rounds = (wg + slots - 1) / slots;
     const int steps = ((nb + ns - 1) / ns + nw - 1) / nw;
-    const double step = std::max(bytes * wgs / 16.0, bytes * std::min(wg, slots) / 2600.0 / best.ntile);
+    const double step = std::max(l2, hbm * std::min(wg, slots));
     const double c = rounds * (6000.0 + steps * step) + (ns > 1 ? 6000.0 + 200.0 * ns : 0.0);
-    if (ns == 1 || call_cost(c, ns > 1) < call_cost(best.cycles, best.nsplit > 1))
-      best.nsplit = ns, best.cycles = c;
+    const double cost = call_cost(c, ns > 1);
+    if (ns == 1 || cost < least) best.nsplit = ns, best.cycles = c, least = cost;
   }
   return best;
 }
 
-static size_t plan_bytes(const Problem& p, const SplitPlan& s) {
+size_t split_bytes(const Problem& p, const SplitPlan& s) {
   if (s.nsplit == 1) return 0;
   return (size_t)s.nsplit * p.B * p.Sq * p.H * (size_t)(p.D + 2) * sizeof(float);
 }
 
-static bool plan_wins(const Problem& p, const SplitPlan& s) {
+bool split_fits(const Problem& p, const SplitPlan& s) {
   if (!(p.scale > 0.0f)) return false;  // the running max is of raw scores
   // at most 2^32 - 1 threads a launch: this kernel's and the combining one's
   // (mha_fwd_kernel takes eight row tiles in 512 threads)
@@ -391,18 +390,12 @@ static bool plan_wins(const Problem& p, const SplitPlan& s) {
   if (s.nsplit > 1 && (rows + 3) / 4 * 256 > (int64_t)UINT32_MAX) return false;
   if ((int64_t)p.Sq * (p.H / p.Hkv) > (int64_t)INT32_MAX) return false;
   if ((int64_t)p.Hkv * p.D * 2 * 32 > (int64_t)UINT32_MAX) return false;
+  return true;
+}
+
+bool split_wins(const Problem& p, const SplitPlan& s) {
   const double main = main_cycles(p);
-  return s.cycles < 0.9 * main && call_cost(s.cycles, s.nsplit > 1) < call_cost(main, false);
-}
-
-bool split_planned(const Problem& p, size_t ws_bytes) {
-  const SplitPlan s = split_plan(p);
-  return plan_wins(p, s) && plan_bytes(p, s) <= ws_bytes;
-}
-
-size_t split_workspace_bytes(const Problem& p) {
-  const SplitPlan s = split_plan(p);
-  return plan_wins(p, s) ? plan_bytes(p, s) : 0;
+  return split_fits(p, s) && s.cycles < 0.9 * main && call_cost(s.cycles, s.nsplit > 1) < call_cost(main, false);
 }
 
 template <typename T, int D>
@@ -431,9 +424,8 @@ static int launch_d(int D, const SplitArgs& a, const SplitPlan& s, hipStream_t s
   return TILEOPS_ESHAPE;
 }
 
-int split_launch(const Problem& p, void* ws, size_t ws_bytes, hipStream_t st) {
+int split_launch(const Problem& p, const SplitPlan& s, void* ws, hipStream_t st) {
   constexpr float kLog2e = 1.4426950408889634f;
-  const SplitPlan s = split_plan(p);
   SplitArgs a{p.q, p.k, p.v, p.o, p.lse, static_cast<float*>(ws), p.B, p.Sq, p.Skv, p.H, p.Hkv,
               p.causal ? 1 : 0, p.scale * kLog2e, 0.0f, 0.0f, s.ntile, s.nsplit};
   if (p.softcap > 0.0f) {  // scores in log2 units from the cap on
