@@ -217,6 +217,30 @@ def test_without_scratch_no_call_is_split(room):
         assert torch.equal(got[0], o2) and torch.equal(got[1], lse2)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("B, sq, skv, H, Hkv, D, causal, splits", [
+    (4, 94, 94, 64, 8, 192, False, -1),    # many short sequences of wide heads
+    (1, 512, 512, 8, 8, 256, True, -1),
+    (16, 64, 64, 32, 32, 256, True, -1),
+    (64, 64, 64, 32, 32, 96, True, -1),
+    (1, 1, 128, 8, 8, 256, True, -1),
+    (2, 256, 256, 16, 16, 64, True, 1),    # one split, no scratch
+    (64, 8, 512, 16, 4, 256, True, 1),
+])
+def test_planned_kernel(B, sq, skv, H, Hkv, D, causal, splits):
+    # where mha_fwd_kernel is the faster one (by 1.1 to 2.8 times) it is taken
+    q = torch.randn(B, sq, H, D, device="cuda", dtype=torch.bfloat16)
+    k = torch.randn(B, skv, Hkv, D, device="cuda", dtype=torch.bfloat16)
+    v = torch.randn(B, skv, Hkv, D, device="cuda", dtype=torch.bfloat16)
+    o, lse, need = _forced(q, k, v, causal, 0)
+    assert need == 0
+    o1, lse1, _ = _forced(q, k, v, causal, splits)
+    assert torch.equal(o, o1) and torch.equal(lse, lse1)
+    o2, _, _ = _forced(q, k, v, causal, -splits)
+    # from two 32-key blocks on the running maxima differ and P rounds another way
+    assert not torch.equal(o, o2)
+
+
 @pytest.mark.smoke
 def test_key_split_plan():
     # which kernel a shape gets (256 compute units): decode steps and short

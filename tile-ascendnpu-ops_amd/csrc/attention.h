@@ -98,7 +98,7 @@ struct Problem {
 constexpr int kMaxSplit = 64;
 struct SplitPlan {
   int ntile, nsplit;
-  double cycles;
+  double us;
 };
 SplitPlan split_plan(const Problem& p, int nsplit = 0);
 bool split_fits(const Problem& p, const SplitPlan& plan);

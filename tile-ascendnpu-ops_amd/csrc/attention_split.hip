@@ -325,32 +325,61 @@ __global__ __launch_bounds__(256) void mha_combine_kernel(SplitArgs A) {
 }
 
 // ---------------------------------------------------------------------------
-// When and how far to split, from estimated cycles of one CU (rates fitted to
-// 36 measured shapes of 4 to 660 us).  The split kernel is taken where it is
-// expected to be at least 10 % faster; on none of those shapes it was slower.
+// When and how far to split, from estimated times in us.  The rates are fitted
+// to 1350 random shapes timed with mha_fwd_kernel and with up to twelve split
+// counts (every head dimension, 1 to 1024 queries, 16 to 32768 keys, 1 to 64
+// heads; the estimates are off by 11 and 8 %).  The split kernel is taken where
+// it is expected to be at least a tenth faster, a fifth at head dimensions 192
+// and 256.  One of those shapes is then slower than with mha_fwd_kernel (6 %);
+// over all, calls are 1.58 times faster (geometric mean), and would be 1.60
+// with the faster kernel every time.  On 700 others: one slower (15 %), 1.60
+// times.  (Rates from 36 shapes of head dimensions 64 and 128, one fixed cost
+// for all, made 100 of 900 shapes slower: B34 S94 H64/8 D192 took 375 us where
+// mha_fwd_kernel takes 134, B64 S64 H32 D128 115 where it takes 77.)
 // ---------------------------------------------------------------------------
-// What an eager call of `cycles` on the GPU costs: it is no shorter than its
-// host path, ~10.4 us with one launch and ~14.5 with two and scratch.  Equal
-// costs go by the GPU time.
-static double call_cost(double cycles, bool two_launches) {
-  return std::max(cycles, two_launches ? 35000.0 : 25000.0) + 1e-3 * cycles;
+struct Rates {
+  int D;
+  double main_fixed, main_tile;             // mha_fwd_kernel: a workgroup, and a key tile of it
+  double split_fixed, split_rows, split_step;  // a workgroup, its 32 rows' outputs, a step
+};
+static const Rates& rates_of(int D) {
+  static const Rates rates[] = {{64, 5.1, 0.93, 0.9, 1.9, 1.15},
+                                {96, 7.2, 1.97, 1.7, 3.1, 1.4},
+                                {128, 7.5, 2.22, 2.2, 3.0, 1.45},
+                                {192, 5.9, 1.43, 2.4, 6.6, 1.95},
+                                {256, 6.0, 1.83, 3.4, 6.5, 2.35}};
+  for (const Rates& r : rates)
+    if (r.D >= D) return r;
+  return rates[4];
 }
 
-// mha_fwd_kernel: a workgroup's fixed cost and 128 keys; the longest block
-// where every block is resident at once, else the mean one.  Its loads of a
-// decode step's keys are HBM traffic it does not hide (2300 bytes a cycle).
-static double main_cycles(const Problem& p) {
-  const double blocks = (double)((p.Sq + 255) / 256) * p.H * p.B * (p.D >= 192 ? 2 : 1);
-  const double rounds = std::max(1.0, blocks / device_cu_count());
-  const double keys = p.causal && rounds > 1.0 ? p.Skv - 0.5 * std::max(p.Sq - 256, 0) : p.Skv;
-  const double tile = p.D <= 64 ? 4200.0 : p.D <= 128 ? 4800.0 : 9600.0;
-  const double hbm = (double)p.B * p.Hkv * p.Skv * p.D * 4.0 / 2300.0;
-  return 22400.0 * rounds + std::max(rounds * tile * keys / 128.0, hbm);
+// What an eager call of `us` on the GPU costs: it is no shorter than its host
+// path, ~10.4 us with one launch and ~14.5 with two and scratch.  Equal costs
+// go by the GPU time.
+static double call_cost(double us, bool two_launches) {
+  return std::max(us, two_launches ? 14.5 : 10.4) + 1e-3 * us;
 }
 
-// mha_split_kernel: a step is one 32-key block per wavefront, bound by its
-// share of HBM (2600 bytes a cycle over the chip, a block read once for all
-// row tiles) or of L2 (16 bytes a cycle per CU).
+// mha_fwd_kernel: a workgroup per CU and round; the longest block where every
+// block is resident at once, else the mean one.  Its loads of a decode step's
+// keys are HBM traffic it does not hide (3.9 TB/s).
+static double main_us(const Problem& p) {
+  const Rates& r = rates_of(p.D);
+  const int64_t cus = device_cu_count();
+  const int64_t blocks = ((int64_t)p.Sq + 255) / 256 * p.H * p.B * (p.D >= 192 ? 2 : 1);
+  const double whole = (double)((blocks + cus - 1) / cus);
+  const double rounds = blocks <= 3 * cus ? whole : std::min(whole, (double)blocks / cus + 0.5);
+  const int keys = p.causal && rounds > 1.0 ? p.Skv - std::max(p.Sq - 256, 0) / 2 : p.Skv;
+  const int bn = p.D == 96 || p.D == 128 ? 128 : 64;
+  const double hbm = (double)p.B * p.Hkv * p.Skv * p.D * 4.0 / 3.9e6;
+  return 0.8 + r.main_fixed * rounds + std::max(rounds * r.main_tile * ((keys + bn - 1) / bn), hbm);
+}
+
+// mha_split_kernel: a step is one 32-key block per wavefront, bound by its own
+// chain of loads and products or its share of HBM (7.9 TB/s of blocks, each
+// read once for all row tiles; where two workgroups share some CUs those set the
+// time, as if all did); then the combination, with its launch, a few loads per
+// split and row, and the partial outputs' bytes.
 SplitPlan split_plan(const Problem& p, int nsplit) {
   const int64_t R = (int64_t)p.Sq * (p.H / p.Hkv);
   SplitPlan best{(int)((R + 31) / 32), 1, 1e30};
@@ -358,20 +387,23 @@ SplitPlan split_plan(const Problem& p, int nsplit) {
     best.nsplit = nsplit;
     return best;
   }
+  const Rates& r = rates_of(p.D);
   const int64_t base = (int64_t)p.B * p.Hkv * best.ntile;
   const int nb = (p.Skv + 31) / 32;
   const int nw = p.D > 128 ? 2 : 4, wgs = p.D <= 64 ? 2 : 1;
   const int64_t cus = device_cu_count(), slots = cus * wgs;
   const double bytes = 32.0 * (p.D <= 64 ? 64 : p.D <= 128 ? 128 : 256) * 4 * nw;
-  const double l2 = bytes * wgs / 16.0, hbm = bytes / 2600.0 / best.ntile;
+  const double hbm = bytes / 7.9e6 / best.ntile;
+  const double fixed = r.split_fixed + r.split_rows * std::min<int64_t>(R, 32) / 32.0;
+  const double part = 0.25 + (double)p.B * p.Sq * p.H * p.D * 4.0 / 3.7e6;
   double least = 0.0;  // call_cost of `best`
   for (int ns = 1; ns <= kMaxSplit && ns <= (nb + nw - 1) / nw; ++ns) {
     const int64_t wg = base * ns, rounds = (wg + slots - 1) / slots;
     const int steps = ((nb + ns - 1) / ns + nw - 1) / nw;
-    const double step = std::max(l2, hbm * std::min(wg, slots));
-    const double c = rounds * (6000.0 + steps * step) + (ns > 1 ? 6000.0 + 200.0 * ns : 0.0);
-    const double cost = call_cost(c, ns > 1);
-    if (ns == 1 || cost < least) best.nsplit = ns, best.cycles = c, least = cost;
+    const double step = std::max(r.split_step, hbm * (wg <= cus ? wg : slots));
+    const double us = 2.6 + rounds * (fixed + steps * step) + (ns > 1 ? 3.2 + part * ns : 0.0);
+    const double cost = call_cost(us, ns > 1);
+    if (ns == 1 || cost < least) best.nsplit = ns, best.us = us, least = cost;
   }
   return best;
 }
@@ -394,8 +426,9 @@ bool split_fits(const Problem& p, const SplitPlan& s) {
 }
 
 bool split_wins(const Problem& p, const SplitPlan& s) {
-  const double main = main_cycles(p);
-  return split_fits(p, s) && s.cycles < 0.9 * main && call_cost(s.cycles, s.nsplit > 1) < call_cost(main, false);
+  const double main = main_us(p);
+  return split_fits(p, s) && s.us < (p.D > 128 ? 0.8 : 0.9) * main &&
+         call_cost(s.us, s.nsplit > 1) < call_cost(main, false);
 }
 
 template <typename T, int D>
