@@ -168,15 +168,21 @@ __device__ __forceinline__ void row_store(void* out, int64_t row, typename RowSt
 // and those after them in its last, one per lane,
 // so that an odd row length costs no more loads than an even one (LogSumExp
 // bf16 16384 x 4097: 73.9 us with one element per lane and load, 34.8 so).
-// With PartMap::per > 0 `out` holds partials: `per` for each of the `keep`
-// outputs, of which rows r, r + keep, .. give nsplit each.
+// PARTS: `out` holds partials, `per` for each of the `keep` outputs, of which
+// rows r, r + keep, .. give nsplit each; else nsplit is 1 (as a parameter its
+// divisions and products cost every row: Argmax fp32 100000 x 500 44.2 us and
+// 41.7).  All U loads of a step are issued before their uses, past-the-end ones
+// clamped onto the row's last pack: a load under a branch of its own was waited
+// for there (then, us: that shape 36.9, Argmax bf16 32768 x 4096 61.5 -> 42.2,
+// 1024 x 32768 18.4 -> 12.9; LogSumExp bf16 32768 x 4096 48.7 -> 43.1, 700 x
+// 16384 8.5 -> 6.2).
 struct PartMap {
   int64_t keep;
   int per;
 };
-template <typename T, int OP, int WPR, int U, bool ALIGNED>
+template <typename T, int OP, int WPR, int U, bool ALIGNED, bool PARTS>
 __global__ __launch_bounds__(WPR > 4 ? 64 * WPR : 256) void row_reduce_kernel(
-    const T* __restrict__ x, void* __restrict__ out, int64_t M, int64_t N, int nstep, int nsplit,
+    const T* __restrict__ x, void* __restrict__ out, int64_t M, int64_t N, int nstep, int splits,
     PartMap pm) {
   typedef typename RowState<OP>::S S;
   constexpr int V = Elem<T>::kVec;
@@ -185,6 +191,7 @@ __global__ __launch_bounds__(WPR > 4 ? 64 * WPR : 256) void row_reduce_kernel(
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wave_in_row = wave % WPR;
+  const int nsplit = PARTS ? splits : 1;
   const int64_t ngroup = (M + ROWS_PER_BLOCK - 1) / ROWS_PER_BLOCK * nsplit;
 
   __shared__ S part[WPB];
@@ -195,35 +202,43 @@ __global__ __launch_bounds__(WPR > 4 ? 64 * WPR : 256) void row_reduce_kernel(
     S st = row_init<OP>();
     if (row < M) {
       const T* xr = x + row * N;
-      int64_t head = 0;
+      int head = 0;
       if constexpr (!ALIGNED) {
         const uint32_t mis = (uint32_t)(reinterpret_cast<uintptr_t>(xr) & 15u);
-        head = min((int64_t)((16u - mis) & 15u) / (int64_t)sizeof(T), N);
+        head = (int)min((int64_t)((16u - mis) & 15u) / (int64_t)sizeof(T), N);
       }
-      const int64_t np = (N - head) / V;
+      const int np = (int)((N - head) / V);  // at least 64: shorter rows are short_row_kernel's
       const T* xb = xr + head;
       const int gw = split * WPR + wave_in_row, nw = nsplit * WPR;
+      // what a slot past the row reads as: exp(-inf) adds 0 to a sum, and the
+      // worst value with an index past every other never wins
+      constexpr float kPast = OP == 2 ? INFINITY : -INFINITY;
       for (int k = 0; k < nstep; ++k) {
-        // Slots past the row read as -inf: they add exp(-inf) = 0 to a sum
-        // and are skipped by the arg-reduction below.
         constexpr int EDGE = ALIGNED ? 0 : 2;
         float vals[U * V + EDGE];
-        int64_t base[U];
+        const int c0 = (k * U * nw + gw) * 64;
+        if (c0 >= np && gw > 0) break;  // the first wavefront has the row's end to fold
+        Pack<T> p[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          p[u] = load_pack_nt(xb + (int64_t)min(c0 + u * nw * 64 + lane, np - 1) * V);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          base[u] = ((int64_t)(k * U + u) * nw + gw) * 64 + lane;
 #pragma unroll
-          for (int e = 0; e < V; ++e) vals[u * V + e] = -INFINITY;
-          if (base[u] < np) {
-            const Pack<T> p = load_pack_nt(xb + base[u] * V);
+          for (int e = 0; e < V; ++e) vals[u * V + e] = Elem<T>::to_f32(p[u].v[e]);
+        }
+        if (c0 + ((U - 1) * nw + 1) * 64 > np) {  // the row ends in this step
 #pragma unroll
-            for (int e = 0; e < V; ++e) vals[u * V + e] = Elem<T>::to_f32(p.v[e]);
+          for (int u = 0; u < U; ++u) {
+            const bool in = c0 + u * nw * 64 + lane < np;
+#pragma unroll
+            for (int e = 0; e < V; ++e) vals[u * V + e] = in ? vals[u * V + e] : kPast;
           }
         }
         bool first = false, last = false;
-        const int64_t t = head + np * V + lane;
+        const int64_t t = head + (int64_t)np * V + lane;
         if constexpr (!ALIGNED) {
-          first = gw == 0 && k == 0 && lane < (int)head;
+          first = gw == 0 && k == 0 && lane < head;
           last = gw == 0 && k == nstep - 1 && t < N;
           vals[U * V] = vals[U * V + 1] = -INFINITY;
           if (first) vals[U * V] = Elem<T>::to_f32(xr[lane]);
@@ -237,11 +252,9 @@ __global__ __launch_bounds__(WPR > 4 ? 64 * WPR : 256) void row_reduce_kernel(
           }
 #pragma unroll
           for (int u = 0; u < U; ++u) {
-            if (base[u] < np) {
+            const uint32_t i0 = (uint32_t)head + (uint32_t)(c0 + u * nw * 64 + lane) * V;
 #pragma unroll
-              for (int e = 0; e < V; ++e)
-                arg_step<OP == 2>(st, vals[u * V + e], (int)(head + base[u] * V + e));
-            }
+            for (int e = 0; e < V; ++e) arg_step<OP == 2>(st, vals[u * V + e], (int)(i0 + e));
           }
           if constexpr (!ALIGNED) {
             if (last) arg_step<OP == 2>(st, vals[U * V + 1], (int)t);
@@ -265,7 +278,7 @@ __global__ __launch_bounds__(WPR > 4 ? 64 * WPR : 256) void row_reduce_kernel(
       __syncthreads();
     }
     if (lane == 0 && wave_in_row == 0 && row < M) {
-      if (pm.per > 0)
+      if constexpr (PARTS)
         static_cast<S*>(out)[row % pm.keep * pm.per + row / pm.keep * nsplit + split] = st;
       else
         row_store<T, OP>(out, row, st);
@@ -279,7 +292,7 @@ __global__ __launch_bounds__(WPR > 4 ? 64 * WPR : 256) void row_reduce_kernel(
 // LogSumExp bf16 88000 x 128: 50 -> 8.9).  PACKS: a lane takes one pack;
 // ragged rows as in row_reduce_kernel (G >= 16 lanes hold the elements before
 // and after the packs).  Otherwise a lane takes one element.
-template <typename T, int OP, int G, bool PACKS, bool ALIGNED>
+template <typename T, int OP, int G, bool PACKS, bool ALIGNED, bool PARTS>
 __global__ __launch_bounds__(256) void short_row_kernel(const T* __restrict__ x,
                                                         void* __restrict__ out, int64_t M, int N,
                                                         PartMap pm, int64_t block0) {
@@ -329,7 +342,7 @@ __global__ __launch_bounds__(256) void short_row_kernel(const T* __restrict__ x,
   }
   st = row_wave<OP, G>(st);
   if (row < M && lane == 0) {
-    if (pm.per > 0)
+    if constexpr (PARTS)
       static_cast<typename RowState<OP>::S*>(out)[row % pm.keep * pm.per + row / pm.keep] = st;
     else
       row_store<T, OP>(out, row, st);
@@ -389,7 +402,7 @@ static RowPlan plan_rows(int64_t M, int64_t N, int vec, bool split = true) {
   return p;
 }
 
-template <typename T, int OP, int WPR, int U>
+template <typename T, int OP, int WPR, int U, bool PARTS>
 static void launch_rows(const T* x, void* out, int64_t M, int64_t N, const RowPlan& p,
                         PartMap pm, hipStream_t s) {
   const bool aligned = host_aligned16(x) && (N % Elem<T>::kVec) == 0;
@@ -397,25 +410,36 @@ static void launch_rows(const T* x, void* out, int64_t M, int64_t N, const RowPl
   const int64_t blocks = (M + rows_per_block - 1) / rows_per_block * p.nsplit;
   const dim3 grid((unsigned)std::min<int64_t>(blocks, 256 * 32)), block(WPR > 4 ? 64 * WPR : 256);
   if (aligned)
-    row_reduce_kernel<T, OP, WPR, U, true><<<grid, block, 0, s>>>(x, out, M, N, p.nstep, p.nsplit, pm);
+    row_reduce_kernel<T, OP, WPR, U, true, PARTS><<<grid, block, 0, s>>>(x, out, M, N, p.nstep, p.nsplit, pm);
   else
-    row_reduce_kernel<T, OP, WPR, U, false><<<grid, block, 0, s>>>(x, out, M, N, p.nstep, p.nsplit, pm);
+    row_reduce_kernel<T, OP, WPR, U, false, PARTS><<<grid, block, 0, s>>>(x, out, M, N, p.nstep, p.nsplit, pm);
 }
 
-template <typename T, int OP, int WPR>
+template <typename T, int OP, int WPR, bool PARTS>
 static void launch_rows_u(const T* x, void* out, int64_t M, int64_t N, const RowPlan& p,
                           PartMap pm, hipStream_t s) {
-  if (p.u == 1) launch_rows<T, OP, WPR, 1>(x, out, M, N, p, pm, s);
-  else if (p.u == 2) launch_rows<T, OP, WPR, 2>(x, out, M, N, p, pm, s);
-  else if (p.u == 3) launch_rows<T, OP, WPR, 3>(x, out, M, N, p, pm, s);
-  else launch_rows<T, OP, WPR, 4>(x, out, M, N, p, pm, s);
+  if (p.u == 1) launch_rows<T, OP, WPR, 1, PARTS>(x, out, M, N, p, pm, s);
+  else if (p.u == 2) launch_rows<T, OP, WPR, 2, PARTS>(x, out, M, N, p, pm, s);
+  else if (p.u == 3) launch_rows<T, OP, WPR, 3, PARTS>(x, out, M, N, p, pm, s);
+  else launch_rows<T, OP, WPR, 4, PARTS>(x, out, M, N, p, pm, s);
+}
+
+template <typename T, int OP, bool PARTS>
+static int launch_long(const T* x, void* out, int64_t M, int64_t N, const RowPlan& p, PartMap pm,
+                       hipStream_t s) {
+  if constexpr (PARTS && OP != 0)  // an index has partials of split rows alone (plan_rows)
+    launch_rows<T, OP, 4, 4, true>(x, out, M, N, p, pm, s);
+  else if (p.wpr == 1) launch_rows_u<T, OP, 1, PARTS>(x, out, M, N, p, pm, s);
+  else if (p.wpr == 4) launch_rows_u<T, OP, 4, PARTS>(x, out, M, N, p, pm, s);
+  else launch_rows<T, OP, 16, 4, PARTS>(x, out, M, N, p, pm, s);
+  return launch_status();
 }
 
 // The short-row kernel takes rows of at most 64 packs; ragged rows of up to 16
 // elements go element by element.
 static bool short_rows(int64_t N, int vec) { return N / vec <= 64; }
 
-template <typename T, int OP>
+template <typename T, int OP, bool PARTS>
 static int launch_short(const T* x, void* out, int64_t M, int64_t N, PartMap pm, hipStream_t s) {
   constexpr int V = Elem<T>::kVec;
   const int n = (int)N, np = n / V;
@@ -426,16 +450,16 @@ static int launch_short(const T* x, void* out, int64_t M, int64_t N, PartMap pm,
     });
   };
   if (host_aligned16(x) && n % V == 0) {
-    if (np <= 4) return go(short_row_kernel<T, OP, 4, true, true>, 4);
-    if (np <= 16) return go(short_row_kernel<T, OP, 16, true, true>, 16);
-    if (np <= 32) return go(short_row_kernel<T, OP, 32, true, true>, 32);
-    return go(short_row_kernel<T, OP, 64, true, true>, 64);
+    if (np <= 4) return go(short_row_kernel<T, OP, 4, true, true, PARTS>, 4);
+    if (np <= 16) return go(short_row_kernel<T, OP, 16, true, true, PARTS>, 16);
+    if (np <= 32) return go(short_row_kernel<T, OP, 32, true, true, PARTS>, 32);
+    return go(short_row_kernel<T, OP, 64, true, true, PARTS>, 64);
   }
-  if (n <= 4) return go(short_row_kernel<T, OP, 4, false, false>, 4);
-  if (n <= 16) return go(short_row_kernel<T, OP, 16, false, false>, 16);
-  if (np <= 16) return go(short_row_kernel<T, OP, 16, true, false>, 16);
-  if (np <= 32) return go(short_row_kernel<T, OP, 32, true, false>, 32);
-  return go(short_row_kernel<T, OP, 64, true, false>, 64);
+  if (n <= 4) return go(short_row_kernel<T, OP, 4, false, false, PARTS>, 4);
+  if (n <= 16) return go(short_row_kernel<T, OP, 16, false, false, PARTS>, 16);
+  if (np <= 16) return go(short_row_kernel<T, OP, 16, true, false, PARTS>, 16);
+  if (np <= 32) return go(short_row_kernel<T, OP, 32, true, false, PARTS>, 32);
+  return go(short_row_kernel<T, OP, 64, true, false, PARTS>, 64);
 }
 
 // Rows of x[M, N]; with keep > 0 rows r, r + keep, .. belong to output r
@@ -453,14 +477,16 @@ static int launch_row_reduce(const void* xv, void* out, int64_t M, int64_t N, in
   PartMap pm{nout, 0};
   const bool is_short = short_rows(N, Elem<T>::kVec);
   if (folds > 1 || (p.nsplit > 1 && !is_short)) pm.per = (int)folds * (is_short ? 1 : p.nsplit);
-  void* dst = pm.per > 0 ? ws : out;
-  int e = 0;
-  if (is_short) e = launch_short<T, OP>(x, dst, M, N, pm, s);
-  else if (p.wpr == 1) launch_rows_u<T, OP, 1>(x, dst, M, N, p, pm, s);
-  else if (p.wpr == 4) launch_rows_u<T, OP, 4>(x, dst, M, N, p, pm, s);
-  else launch_rows<T, OP, 16, 4>(x, dst, M, N, p, pm, s);
-  if (e || (e = launch_status())) return e;
-  return pm.per > 0 ? launch_merge<T, OP>(ws, out, nout, pm.per, s) : 0;
+  if (pm.per == 0)
+    return is_short ? launch_short<T, OP, false>(x, out, M, N, pm, s)
+                    : launch_long<T, OP, false>(x, out, M, N, p, pm, s);
+  int e;
+  if constexpr (OP == 0)
+    e = is_short ? launch_short<T, OP, true>(x, ws, M, N, pm, s)
+                 : launch_long<T, OP, true>(x, ws, M, N, p, pm, s);
+  else
+    e = launch_long<T, OP, true>(x, ws, M, N, p, pm, s);
+  return e ? e : launch_merge<T, OP>(ws, out, nout, pm.per, s);
 }
 
 // ---------------------------------------------------------------------------
