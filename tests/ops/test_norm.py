@@ -167,3 +167,29 @@ def test_fused_add_layer_norm_ragged_rows(m, n, dtype, param_dtype):
     # the bound of the test above: one rounding of y, fp32 statistics
     atol, rtol = ref_tolerance(dtype)
     assert_close_np(to_np(y), y_ref, atol, rtol, "y")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("param_dtype", [None, torch.float32])
+@pytest.mark.parametrize("n, dtype, per_cu", [
+    (3328, torch.float32, (2,)),                 # 13 packs per lane
+    (6656, torch.bfloat16, (2, 3)),
+    (1280, torch.float32, (3, 4)),               # 5
+    (4096, torch.bfloat16, (3, 4)),              # 8
+    (6144, torch.float16, (3, 4, 5, 6, 10, 32)),  # 12
+])
+def test_fused_add_layer_norm_at_the_lines_of_the_dispatch(n, dtype, per_cu, param_dtype):
+    # a wavefront or a workgroup per row, by the rows per compute unit: the last
+    # row count on one side of each line and the first on the other
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    op = FusedAddLayerNormFwdOp(dtype=dtype)
+    for m in (k * cus + d for k in per_cu for d in (0, 1)):
+        test = FusedAddLayerNormTest(m, n, dtype, param_dtype=param_dtype)
+        x, r, w, b = test.gen_inputs()
+        y, r_out = op(x, r, w, b)
+        assert torch.equal(r_out, (x.float() + r.float()).to(dtype))
+        rows = torch.cat([torch.arange(0, m, 61), torch.tensor([m - 2, m - 1])]).cuda()
+        y_ref, _ = test.ref_program(x[rows], r[rows], w, b)
+        # one rounding of y, fp32 statistics, as above
+        atol, rtol = ref_tolerance(dtype)
+        torch.testing.assert_close(y[rows], y_ref.to(y.device), atol=atol, rtol=rtol)

@@ -411,14 +411,33 @@ static int launch_fused_add_ln(const void* xv, const void* rv, const void* wv, c
   const bool packable = aligned && N % V == 0;
   const int64_t lane_packs = (N / V + 63) / 64;
   const int n = (int)N;
-  // One wavefront per row where rows are short and many; a workgroup per row
-  // else (1 x 8192 bf16: 7.8 -> 4.3 us, 64 x 4096 5.5 -> 4.0, 1000 x 2048 5.3
-  // -> 4.7, 4096 x 5120 34.1 -> 32.3; the wavefront stays where it is the
-  // faster: 16384 x 768 21.3 against 27.1, 32768 x 4096 181 against 183, and at
-  // 13 to 16 packs per lane 2048 x 8192 23.7 against 27.3).  Ragged rows of two packs and more have at least one aligned pack
-  // (2048 x 4097 bf16: 26.0 us three-pass, 17.4 so).
+  // One wavefront per row where rows are many, a workgroup per row else (bf16 1 x
+  // 8192 7.8 -> 4.3 us, 64 x 4096 5.5 -> 4.0).  From four rows per CU on the
+  // wavefronts' four-row workgroups fill the chip (16384 x 768 21.3 us against
+  // 27.1, 2048 x 8192 23.7 against 27.3); longer rows and fp32 parameters, which
+  // the workgroups read again for every row, leave a CU with three workgroups at
+  // a time, or two: then the fourth or third row of a CU waits (wavefront,
+  // workgroup, us: bf16 832 x 6656 10.7 and 11.8, 832 x 8192 11.7 and 13.5; fp32
+  // 896 x 2048 5.7 and 6.5, 768 x 3328 8.8 and 9.7, 512 x 3328 8.6 and 7.5; fp32
+  // parameters 832 x 6656 10.6 and 12.4; bf16 1000 x 2048 5.3 and 4.7).
+  // At 9 to 12 packs per lane the wavefronts win where two of their workgroups
+  // fill each CU evenly and where rows are very many, and from five rows per CU
+  // on with fp32 parameters for 16-bit rows (bf16 1300 x 6144 16.6 and 14.5, 2048
+  // x 6144 18.7 and 20.5, 3000 x 6144 31.2 and 29.3, 4096 x 5120 33.8 and 32.1,
+  // 16384 x 5120 113 and 118, fp32 2048 x 2304 15.1 and 16.4; fp32 parameters
+  // 1025 x 5120 13.3 and 11.4, 2048 x 6144 18.9 and 22.8, 4096 x 5120 33.1 and
+  // 34.7).
+  // Ragged rows of two packs and more have at least one aligned pack (2048 x
+  // 4097 bf16: 26.0 us three-pass, 17.4 so).
   // grid x dimension times block size stays within 32 bits on both fast paths
-  const bool wave = M > 1024 && (lane_packs <= 8 || (lane_packs > 12 && lane_packs <= 16));
+  const int64_t cus = device_cu_count();
+  const bool wide = sizeof(W) == 4;
+  const int rows = wide && lane_packs > 12 ? 2 : lane_packs > (wide ? 4 : 8) ? 3 : 4;
+  bool wave = lane_packs <= 16 && M > rows * cus;
+  if (wave && M > 4 * cus && lane_packs > 8 && lane_packs <= 12) {
+    if (sizeof(W) > sizeof(T)) wave = M > 5 * cus;
+    else wave = (M > 6 * cus && M < 10 * cus) || M > 32 * cus;
+  }
   if (packable && wave && M <= (int64_t)(UINT32_MAX / 64)) {
     if (lane_packs <= 1) launch_wave<T, W, 1>(x, r, w, b, y, ro, M, n, eps, s);
     else if (lane_packs <= 2) launch_wave<T, W, 2>(x, r, w, b, y, ro, M, n, eps, s);

@@ -214,6 +214,14 @@ def stream_of(t: torch.Tensor) -> int:
 
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
 
+# looked up once: a call of `eager` is 0.65 us of a 10 us host path
+_is_compiling = torch.compiler.is_compiling
+_tracing_state = torch._C._get_tracing_state
+_dispatch_modes = torch._C._len_torch_dispatch_stack
+_function_modes = torch._C._len_torch_function_stack
+_functorch_level = torch._C._functorch.peek_interpreter_stack
+_forward_ad = torch.autograd.forward_ad
+
 
 def eager(*tensors: torch.Tensor) -> bool:
     """True when a call on ``tensors`` may run its launch function directly
@@ -229,12 +237,12 @@ def eager(*tensors: torch.Tensor) -> bool:
     9.8 us per call).
     """
     if (
-        torch.compiler.is_compiling()
-        or torch._C._get_tracing_state() is not None
-        or torch._C._len_torch_dispatch_stack()
-        or torch._C._len_torch_function_stack()
-        or torch._C._functorch.peek_interpreter_stack() is not None
-        or torch.autograd.forward_ad._current_level >= 0
+        _is_compiling()
+        or _tracing_state() is not None
+        or _dispatch_modes()
+        or _function_modes()
+        or _functorch_level() is not None
+        or _forward_ad._current_level >= 0
     ):
         return False
     grad = torch.is_grad_enabled()

@@ -65,7 +65,7 @@ class FusedAddLayerNormKernel(Kernel):
     def default_config(self) -> dict:
         # fused_add_ln_wave_kernel: one wavefront per row with the row held in
         # registers, four rows per 256-thread workgroup, weight / bias staged
-        # in LDS as fp32 (longer rows: one 256-thread workgroup per row)
+        # in LDS as fp32 (few or longer rows: one 256-thread workgroup per row)
         return {"rows_per_wave": 1, "rows_per_workgroup": 4}
 
     def forward(
