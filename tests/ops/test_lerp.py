@@ -195,3 +195,36 @@ def test_broadcast_ragged_rows_match_the_materialised_broadcast(dtype, sa, sb, s
     off.copy_(full[1])
     y = LerpTensorFwdOp(input=shape, end=shape, weight=shape, dtype=dtype)(full[0], off, full[2])
     assert torch.equal(y, ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("sa, sb, sw", [
+    ((17, 7710), (17, 1), (17, 7710)),            # 131,070 elements: one below the line
+    ((17, 7711), (17, 1), (17, 7711)),            # above it, whole packs and 7 elements (3 in fp32)
+    ((7, 67, 21, 21), (67, 1, 1), (7, 1, 1, 1)),  # packs across rows, channels and images
+    ((8, 67, 22, 22), (67, 1, 1), (8, 1, 1, 1)),  # whole packs
+    ((1, 1), (131, 1009), (131, 1)),              # only the second operand is laid out like y
+    ((1100, 1001), (1, 1001), (1100, 1)),         # an operand read element by element
+    ((30001, 9), (30001, 1), (1, 1)),             # rows of a pack and one element
+])
+def test_broadcast_packs_across_ragged_rows(dtype, sa, sb, sw):
+    # the sizes from which the outputs go as flat packs; the same arithmetic on
+    # materialised operands: equal bit for bit
+    a, b, w = (torch.randn(s, device="cuda").to(dtype) for s in (sa, sb, sw))
+    shape = torch.broadcast_shapes(sa, sb, sw)
+    full = [t.expand(shape).contiguous() for t in (a, b, w)]
+    y = LerpTensorFwdOp(input=sa, end=sb, weight=sw, dtype=dtype)(a, b, w)
+    ref = LerpTensorFwdOp(input=shape, end=shape, weight=shape, dtype=dtype)(*full)
+    assert torch.equal(y, ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_broadcast_packs_beside_transposed_and_misaligned_operands(dtype):
+    m, n = 1100, 1009
+    a = torch.randn(m, n, device="cuda").to(dtype)
+    b = torch.randn(n, m, device="cuda").to(dtype).t()
+    w = torch.randn(m * n + 1, device="cuda").to(dtype)[1:].view(m, n)
+    op = LerpTensorFwdOp(input=(m, n), end=(m, n), weight=(m, n), dtype=dtype)
+    assert torch.equal(op(a, b, w), op(a, b.contiguous(), w.clone()))

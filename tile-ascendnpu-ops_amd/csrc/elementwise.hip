@@ -636,24 +636,43 @@ __global__ __launch_bounds__(256) void bcast_inner_kernel(const T* __restrict__ 
 // least V elements), so the multi-index is divided out twice, and an operand
 // that is broadcast along the row is two scalars; others are read element by
 // element.  Element by element for everything, two divisions each, measured
-// 25.6 us for a channel bias fp16 32x1024x14x14; this 7.6.
+// 25.6 us for a channel bias fp16 32x1024x14x14; this 7.6.  Where the output is
+// not whole packs, a thread each takes the elements that remain (in a launch of
+// their own they cost ~1.6 us: a column added to bf16 370 x 1001 4.3 us, element
+// by element 2.9, so 2.7).
 template <typename T, int OP>
 __global__ __launch_bounds__(256) void bcast_flat_kernel(const T* __restrict__ a,
                                                          const T* __restrict__ b,
                                                          const T* __restrict__ w,
-                                                         T* __restrict__ y, uint32_t npack, float p,
+                                                         T* __restrict__ y, uint32_t n, float p,
                                                          BcastDesc d, int flat_mask, BcastDivs dv) {
   constexpr int V = Elem<T>::kVec;
   constexpr int NOP = BcastArity<OP>::n;
   const T* src[3] = {a, b, w};
   const uint32_t pk = blockIdx.x * 256u + threadIdx.x;
-  if (pk >= npack) return;
+  const int last = d.ndim - 1;
+  const uint32_t row = (uint32_t)d.shape[last];
+  if (pk >= n / V) {  // an element of the last, less than a pack
+    const uint32_t i = n / V * V + (pk - n / V);
+    if (i >= n) return;
+    uint32_t r = div_by(i, dv.row), off[3];
+#pragma unroll
+    for (int o = 0; o < NOP; ++o) off[o] = (i - r * row) * (uint32_t)d.st[o][last];
+    for (int k = last - 1; k >= 0; --k) {
+      const uint32_t sh = (uint32_t)d.shape[k], q = div_by(r, dv.dim[k]), idx = r - q * sh;
+      r = q;
+#pragma unroll
+      for (int o = 0; o < NOP; ++o) off[o] += idx * (uint32_t)d.st[o][k];
+    }
+    const float we = NOP == 3 ? Elem<T>::to_f32(src[2][off[2]]) : 0.0f;
+    y[i] = Elem<T>::from_f32(bc_apply<OP>(Elem<T>::to_f32(src[0][off[0]]),
+                                          Elem<T>::to_f32(src[1][off[1]]), we, p));
+    return;
+  }
   Pack<T> in[3];
 #pragma unroll
   for (int o = 0; o < NOP; ++o)
     if ((flat_mask >> o) & 1) in[o] = load_pack_nt(src[o] + (int64_t)pk * V);
-  const int last = d.ndim - 1;
-  const uint32_t row = (uint32_t)d.shape[last];
   const uint32_t r0 = div_by(pk * V, dv.row), c0 = pk * V - r0 * row;
   uint32_t base[2][3];  // offsets of the rows the pack starts and ends in
 #pragma unroll
@@ -792,29 +811,28 @@ static bool launch_bcast_inner(const T* const (&src)[3], T* y, const BcastDesc& 
 // has at least a pack's elements and 32-bit offsets reach every one, from
 // kFlatMin elements on (an element per thread is as fast below: channel bias
 // bf16 of 94,080 elements 2.7 us against 3.1; row bias of 300,300 3.0 against
-// 4.8, hence its higher line); returns the packs it took (the rest of the
-// output, less than a pack, is the caller's).
+// 4.8, hence its higher line); returns whether it took the call.
 constexpr int64_t kFlatMin = 1 << 17;
 template <typename T, int OP>
-static int64_t launch_bcast_flat(const T* const (&src)[3], T* y, const BcastDesc& d, int64_t n,
-                                 float p, hipStream_t s) {
+static bool launch_bcast_flat(const T* const (&src)[3], T* y, const BcastDesc& d, int64_t n,
+                              float p, hipStream_t s) {
   constexpr int V = Elem<T>::kVec;
   constexpr int NOP = BcastArity<OP>::n;
-  if (n < kFlatMin || n > (int64_t)INT32_MAX - 256 * V || !host_aligned16(y)) return 0;
-  if (d.shape[d.ndim - 1] < V) return 0;
+  if (n < kFlatMin || n > (int64_t)INT32_MAX - 256 * V || !host_aligned16(y)) return false;
+  if (d.shape[d.ndim - 1] < V) return false;
   const int flat_mask = flat_operands<T>(src, d, NOP);
-  if (flat_mask == 0) return 0;
+  if (flat_mask == 0) return false;
   for (int o = 0; o < NOP; ++o) {
     // element-wise operands: the crossover lies higher
-    if (!((flat_mask >> o) & 1) && d.st[o][d.ndim - 1] != 0 && n < 8 * kFlatMin) return 0;
+    if (!((flat_mask >> o) & 1) && d.st[o][d.ndim - 1] != 0 && n < 8 * kFlatMin) return false;
     int64_t omax = 0;
     for (int k = 0; k < d.ndim; ++k) omax += (d.shape[k] - 1) * d.st[o][k];
-    if (omax >= (int64_t)UINT32_MAX) return 0;
+    if (omax >= (int64_t)UINT32_MAX) return false;
   }
-  const int64_t npack = n / V;
-  bcast_flat_kernel<T, OP><<<dim3((unsigned)((npack + 255) / 256)), dim3(256), 0, s>>>(
-      src[0], src[1], src[2], y, (uint32_t)npack, p, d, flat_mask, divisors(d, d.shape[d.ndim - 1]));
-  return npack;
+  const int64_t threads = n / V + n % V;
+  bcast_flat_kernel<T, OP><<<dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s>>>(
+      src[0], src[1], src[2], y, (uint32_t)n, p, d, flat_mask, divisors(d, d.shape[d.ndim - 1]));
+  return true;
 }
 
 template <typename T, int OP>
@@ -844,8 +862,8 @@ static int launch_bcast(const void* av, const void* bv, const void* wv, void* yv
     if (npack > 0)
       bcast_vec_kernel<T, OP><<<dim3((unsigned)((npack + 255) / 256)), dim3(256), 0, s>>>(
           src[0], src[1], src[2], y, npack, p);
-  } else {
-    npack = launch_bcast_flat<T, OP>(src, y, d, n, p, s);
+  } else if (launch_bcast_flat<T, OP>(src, y, d, n, p, s)) {
+    return launch_status();
   }
   const int64_t done = npack * V;
   if (done < n)
