@@ -1072,19 +1072,18 @@ __global__ __launch_bounds__(64 * NW) void gdn_compose_kernel(Args A) {
     for (int r = 0; r < 4; ++r) s[kb][r] = slot(0)[acc_row(kb, g, r) * DV + col0 + ln];
   fetch(1, 0);
   load_b(bn, 1);
-  float gam = *ws_decay(A, bh, 1), gam_next = 0.0f;
+  const float gams = *ws_decay(A, bh, min(lane, last));  // lane j: the decay of segment j
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
   __syncthreads();
   for (int j = 1; j <= last; ++j) {
+    const float gam = __builtin_bit_cast(
+        float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, gams), j));
     f32x4 acc[8];
 #pragma unroll
-    for (int kb = 0; kb < 8; ++kb)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc[kb][r] = fmaf(gam, s[kb][r], bn[kb][r]);
+    for (int kb = 0; kb < 8; ++kb) acc[kb] = bn[kb];
     if (j + 1 <= last) {
       fetch(j + 1, j & 1);
       load_b(bn, j + 1);
-      gam_next = *ws_decay(A, bh, j + 1);
     }
     if (j > 1) store_s(s, j - 1);
     const bf16* phi_hi = phi_s[(j - 1) & 1];
@@ -1108,9 +1107,10 @@ __global__ __launch_bounds__(64 * NW) void gdn_compose_kernel(Args A) {
       }
     }
 #pragma unroll
-    for (int kb = 0; kb < 8; ++kb) s[kb] = acc[kb];
-    gam = gam_next;
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the next E, B and decay have landed
+    for (int kb = 0; kb < 8; ++kb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) s[kb][r] = fmaf(gam, s[kb][r], acc[kb][r]);
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the next E and B have landed
     __syncthreads();
   }
   store_s(s, last);
