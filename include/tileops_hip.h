@@ -241,7 +241,7 @@ int tileops_mha_fwd(const void* q, const void* k, const void* v, void* o, float*
  * the fp32 partial outputs and row statistics of the splits
  * (tileops_mha_workspace_bytes, 0 where no split is planned) go to `ws`
  * (16-byte aligned) and are combined by a second launch.  With `ws` NULL or
- * smaller than that no call is split.
+ * smaller than that such a call takes the kernel of tileops_mha_fwd's prefill.
  */
 size_t tileops_mha_workspace_bytes(int64_t B, int64_t Sq, int64_t Skv, int64_t H, int64_t Hkv,
                                    int64_t D, int causal, float scale);
@@ -315,12 +315,12 @@ size_t tileops_gdn_prefill_workspace_bytes_ex(int64_t B, int64_t T, int64_t H, i
  * allocating routine.  No counterpart in the reference.  The segment maps
  * live in a 32 MiB device array of the library (one per GPU, held until
  * the process ends): a call uses as many segments N as the array holds
- * (B * H * (2 N - 3) maps of 64 KiB), down to one segment, which needs no
- * array, so every B, T and H is accepted.  Calls that use the array run one
- * after another on the device: each waits for the previous such call's
- * completion event, whatever stream it ran on (once per device, at the
- * first call, the library creates that event and looks up the array's
- * address).  Under stream capture the event is not used, and captured calls
+ * (B * H * (2 N - 3) maps of 64 KiB and B * H * N floats), down to one
+ * segment, which needs no array, so every B, T and H is accepted.  Calls
+ * that use the array run one after another on the device: each waits for
+ * the previous such call's completion event, whatever stream it ran on
+ * (once per device, at the first call, the library creates that event and
+ * looks up the array's address).  Under stream capture the event is not used, and captured calls
  * on parallel branches of one graph race on the array.  Results equal
  * tileops_gdn_prefill_fwd_ex's with the same segment count bit for bit.
  */

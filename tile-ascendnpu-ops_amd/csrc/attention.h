@@ -46,7 +46,7 @@ template <int D> struct Swz {
 // `base + off` (base uniform, in SGPRs; off a per-lane byte offset) and they
 // land at LDS byte address lds + 16 l.  Issued as inline assembly so that the
 // compiler does not track the LDS write: every wait for these loads is
-// explicit (vmcnt) and followed by a workgroup barrier before any wavefront
+// explicit (vmcnt) and followed by a workgroup barrier before another wavefront
 // reads the data.  The compiler's hazard checks do not look into inline
 // assembly: the load starts with the one wait state the ISA requires after
 // the SALU write of M0 that precedes it (its base comes from SALU

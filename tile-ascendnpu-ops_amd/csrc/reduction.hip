@@ -2,13 +2,13 @@
 // of a row-major [M, N] tensor, over the middle dimension of [outer, N, inner]
 // (column kernel, below) or over the outer two of [R, M, L].
 //
-// Rows.// A wavefront streams its share of a row in 16-byte packs, UNROLL packs per
+// Rows.  A wavefront streams its share of a row in 16-byte packs, U packs per
 // lane in flight, folds them into a per-lane partial, and the 64 partials meet
 // in a shuffle butterfly.  What bounds the kernel is HBM where the rows fill
 // the chip, and the latency of one wavefront's chain of loads where they do
 // not, so the number of wavefronts per row follows the row count (plan_rows):
 // 1 (four rows per workgroup), 4, 16 (a 1024-thread workgroup), or several
-// 16-wavefront workgroups per row whose partials a second launch merges.
+// 4-wavefront workgroups per row whose partials a second launch merges.
 #include <algorithm>
 
 #include <float.h>
@@ -167,7 +167,7 @@ __device__ __forceinline__ void row_store(void* out, int64_t row, typename RowSt
 // the row's first wavefront folds the elements before them in its first step
 // and those after them in its last, one per lane,
 // so that an odd row length costs no more loads than an even one (LogSumExp
-// bf16 16384 x 4097: 73.9 us with one element per lane and load, 34.8 so).
+// bf16 16384 x 4097: 73.9 us with one element per lane and load, 28.9 so).
 // PARTS: `out` holds partials, `per` for each of the `keep` outputs, of which
 // rows r, r + keep, .. give nsplit each; else nsplit is 1 (as a parameter its
 // divisions and products cost every row: Argmax fp32 100000 x 500 44.2 us and
@@ -372,16 +372,18 @@ static int launch_merge(const void* ws, void* out, int64_t M, int nsplit, hipStr
 }
 
 // How a [M, N] row reduction is laid out.  One wavefront per row from 3072
-// rows up (a dozen wavefronts per CU), four below, sixteen where at most 512
-// rows leave each of those work (LogSumExp bf16 512 x 32768: 14.2 us with
-// four, 11.1 with sixteen; 1024 rows: 18.6 and 19.5).  At most 128 rows (two
-// CUs each) of 256 chunks or more (sixteen wavefronts would take four steps
-// and more, ~2 us each) are split over workgroups of four wavefronts, one
-// step each up to 1024 workgroups; the merge launch and its scratch cost ~2.5
-// us on the GPU and ~4 us of an eager call's host time, so shorter rows stay
-// whole (LogSumExp bf16 4 x 102400: 17.5 us with four wavefronts per row,
-// 10.7 with sixteen, 6.3 split, but 10.7 and 14.6 us per eager call; Argmax of 2^21
-// fp16 elements 682 -> 9.7 us, of 2^25 fp32 9222 -> 32).
+// rows up (a dozen wavefronts per CU; LogSumExp bf16 3072 x 4096 7.9 us, 9.3 with
+// four), four below, sixteen where at most 512 rows leave each of those work
+// (512 x 32768: LogSumExp bf16 9.9 us with four and 9.6 with sixteen, Argmax 11.4
+// and 10.3; 1024 rows: 14.9 and 16.6; 512 x 8192: 5.5 and 8.4).  At most 128 rows
+// (two CUs each) of 256 chunks or more (sixteen wavefronts would take four steps
+// and more, ~2 us each) are split over workgroups of four wavefronts, one step
+// each up to 1024 workgroups; the merge launch and its scratch cost ~2.5 us on
+// the GPU and ~4 us of an eager call's host time, so shorter rows stay whole
+// (LogSumExp bf16 4 x 102400: 15.3 us with four wavefronts per row, 9.4 with
+// sixteen, 6.3 split, but 10.4 and ~14 us per eager call; 4 x 131072 10.0 whole
+// and 6.1 split; Argmax of 2^21 fp16 elements 143 with sixteen, 9.1 split, of
+// 2^25 fp32 33.7 split).
 // A wavefront keeps 4 packs per lane in flight, fewer where its whole share of
 // the row is less (slots past the row still cost their exponentials).
 struct RowPlan {

@@ -11,7 +11,8 @@ segments (config ``segments``: 0 lets the library choose from the head
 count and the device's compute units): one launch runs segment 0 exactly
 and the state maps of the inner segments, a second composes each later
 segment's start state and runs it exactly.  The workspace holds the maps
-(64 KiB per map and head).  Device code: gdn_fused_kernel in csrc/gdn.hip.
+(64 KiB per map and head) and the segments' decays.  Device code:
+gdn_fused_kernel and gdn_compose_kernel in csrc/gdn.hip.
 """
 
 from typing import Optional, Tuple

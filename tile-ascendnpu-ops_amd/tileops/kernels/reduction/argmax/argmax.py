@@ -4,7 +4,8 @@ Reference class: examples/TileOPs/tileops/kernels/reduction/argmax/argmax.py:89-
 Semantics are torch.argmax / torch.argmin: first occurrence among equal
 values, NaN counts as the extreme value.  The launch is wrapped in the
 ``tileops::argreduce_fwd`` custom op (reference: ``npub::argreduce_fwd``).
-Device code: row_reduce_kernel<T, 1|2, ...> in csrc/reduction.hip.
+Device code in csrc/reduction.hip: row_reduce_kernel, short_row_kernel and
+merge_partials_kernel<T, 1|2, ...>, col_reduce_kernel over other dims.
 """
 
 from typing import Optional
@@ -94,7 +95,7 @@ class ArgreduceKernel(Kernel):
                 "Reduction dimension is empty (N=0). "
                 "argmax/argmin over an empty dimension is undefined."
             )
-        # row_reduce_kernel: as LogSumExpKernel
+        # as LogSumExpKernel: what rows of middling number and length run with
         return {"wavefronts_per_row": 1 if self.M >= 3072 else 4, "packs_in_flight": 4}
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:

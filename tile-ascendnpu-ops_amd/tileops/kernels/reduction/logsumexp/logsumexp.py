@@ -2,11 +2,13 @@
 
 Reference class: examples/TileOPs/tileops/kernels/reduction/logsumexp/logsumexp.py:150-336.
 y[i] = max_i + log(sum_j exp(x[i, j] - max_i)) in fp32, rounded to the input
-dtype.  One wavefront folds each row with an online (max, scaled-sum) pair, so
-any N works without host padding.  The launch is wrapped in the
+dtype.  Lanes fold a row with online (max, scaled-sum) pairs, in a few lanes of
+a wavefront or in several workgroups by the shape, so any N works without host
+padding.  The launch is wrapped in the
 ``tileops::logsumexp_fwd`` custom op (with a fake impl) so ``torch.compile``
 can trace through it, as the reference's ``npub::logsumexp_fwd`` did.
-Device code: row_reduce_kernel<T, 0, ...> in csrc/reduction.hip.
+Device code in csrc/reduction.hip: row_reduce_kernel, short_row_kernel and
+merge_partials_kernel<T, 0, ...>, col_reduce_kernel over other dims.
 """
 
 from typing import Optional
@@ -86,9 +88,9 @@ class LogSumExpKernel(Kernel):
 
     @property
     def default_config(self) -> dict:
-        # row_reduce_kernel: one wavefront per row (four rows per workgroup)
-        # from 3072 rows up, else at least four wavefronts per row (few long
-        # rows: sixteen, or several workgroups); 4 packs in flight per lane
+        # what rows of middling number and length run with; the library goes by
+        # the shape (plan_rows in csrc/reduction.hip): few long rows take sixteen
+        # wavefronts or several workgroups each, short rows part of a wavefront
         return {"wavefronts_per_row": 1 if self.M >= 3072 else 4, "packs_in_flight": 4}
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
