@@ -384,9 +384,15 @@ def test_strided_form_leaves_large_sizes_to_the_general_path():
                         ((2, 3, big), [0, 1]), ((2, big, 64), [0, 2]), ((2, 3, big // 2), [0, 2])):
         assert form(shape, dims) is None, (shape, dims)
     assert form((2, big - 1), [0]) == (1, 2, big - 1, False)
-    assert form((big - 1, 2, 64), [1]) == (big - 1, 2, 64, False)
+    assert form((big - 1, 4, 64), [1]) == (big - 1, 4, 64, False)
     assert form((2, big - 1, 64), [0, 2]) == (2, big - 1, 64, True)
     assert form((2, 3, big // 2 - 1), [0, 2]) == (2, 3, big // 2 - 1, True)
+    # many small slices are copied: from 16384 on, below 64 packs of 16 bytes
+    assert strided_form(torch.empty((16384, 3, 84), device="meta"), [1]) is None
+    assert form((16384, 4, 64), [1]) == (16384, 4, 64, False)
+    assert form((16383, 3, 84), [1]) == (16383, 3, 84, False)
+    half = torch.empty((16384, 4, 64), device="meta", dtype=torch.float16)
+    assert strided_form(half, [1]) is None
 
 
 def _windows(n):
@@ -399,7 +405,8 @@ def _windows(n):
 @pytest.mark.parametrize("shape, dim, dtype", [
     ((2**28 + 40, 5), -1, torch.float16),     # short rows, sixteen to a workgroup
     ((2, 2**31 + 64), 0, torch.bfloat16),     # copied, short rows past 2^31
-    ((2**24 + 3, 2, 64), 1, torch.bfloat16),  # a column workgroup per outer slice
+    ((2**24 + 3, 8, 64), 1, torch.bfloat16),  # a column workgroup per outer slice
+    ((2**24 + 3, 2, 64), 1, torch.bfloat16),  # copied
     ((2, 2**26 + 9, 64), [0, 2], torch.float16),  # merged from partials
 ])
 def test_reductions_of_more_rows_than_one_launch_holds(shape, dim, dtype):

@@ -581,9 +581,10 @@ __global__ __launch_bounds__(256) void col_reduce_kernel(const T* __restrict__ x
 
 // Threads across the columns: 256 where that alone fills the chip, and for a
 // few rows from half a workgroup per CU on (LogSumExp bf16 [4, 128, 4096] over
-// dimension 0: 5.3 us with 256, 6.7 with 64 and their merge) except where a
-// thread would store eight scattered indices (Argmax fp16 of that shape: 7.8
-// and 6.6); else 64, else 16.  With less than a workgroup per CU and six steps
+// dimension 0: 5.3 us with 256, 6.7 with 64 and their merge; bf16 [8, 2^20] 8.9
+// and 12.4, fp32 [2, 2^19] 4.7 and 6.8) except where a thread would store eight
+// scattered indices (Argmax fp16 of that shape: 7.8 and 6.6; bf16 [8, 2^20] 13.4
+// and 10.8); else 64, else 16.  With less than a workgroup per CU and six steps
 // of ~2 us or more the rows are split, one step each up to two workgroups per
 // CU (Argmax bf16 [3, 1000, 64]: 32 us whole, 9.7 split; 300 rows: 9.4 either
 // way, and whole is one launch).  Rows past the end of a thread's last step

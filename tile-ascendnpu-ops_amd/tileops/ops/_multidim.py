@@ -63,7 +63,11 @@ def strided_form(x: torch.Tensor, dims: list[int]) -> "tuple[int, int, int, bool
 
     Below 64 neighbouring columns (or, for ``ends``, rows of 64 elements) the
     strided reads leave most of a wavefront idle and the copy is kept; ``ends``
-    merges ``outer`` partials per output on one wavefront, which bounds it.  As
+    merges ``outer`` partials per output on one wavefront, which bounds it.  A
+    column workgroup has a slice to itself, so that many small slices, of less
+    than 64 packs, are copied too (us, as they lie and copied: LogSumExp bf16
+    [131072, 4, 64] 240 and 122, [16384, 4, 64] 36.7 and 24.0, [2048, 4, 64] 6.9 and
+    8.3, [16384, 16, 64] 55.5 and 53.5, [16384, 8, 128] 48.8 and 55.0).  As
     on the general path at most 2^31 - 1 elements are reduced to one, and the
     entry point takes each of the three sizes below 2^31.
     """
@@ -73,6 +77,8 @@ def strided_form(x: torch.Tensor, dims: list[int]) -> "tuple[int, int, int, bool
     if hi - lo + 1 == len(dims):  # one run of reduced dims
         outer, n, inner = prod(shape[:lo]), prod(shape[lo:hi + 1]), prod(shape[hi + 1:])
         if inner < 64 or max(outer, n, inner) >= 2**31:
+            return None
+        if outer >= 16384 and n * inner * x.dtype.itemsize < 64 * 16:
             return None
         return outer, n, inner, False
     kept = [i for i in range(lo, hi + 1) if i not in dims]
