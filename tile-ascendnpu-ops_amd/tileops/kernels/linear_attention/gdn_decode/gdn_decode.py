@@ -117,7 +117,8 @@ class GDNDecodeKernel(Kernel):
                 raise ValueError(f"Expected {name}.shape {shape}, got {tuple(t.shape)}")
             if t.dtype != dt:
                 raise ValueError(f"Expected {name}.dtype {dt}, got {t.dtype}")
-        q, k, v, g, beta, state = (t.contiguous() for t in (q, k, v, g, beta, state))
+        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+        g, beta, state = g.contiguous(), beta.contiguous(), state.contiguous()
         fwd = (_gdn_decode_fwd_launch if _native.eager(q, k, v, g, beta, state)
                else _gdn_decode_fwd)
         return fwd(B, H, K, V, self.scale, q, k, v, g, beta, state)

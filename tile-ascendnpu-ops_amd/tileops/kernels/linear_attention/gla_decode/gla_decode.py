@@ -104,6 +104,7 @@ class GLADecodeKernel(Kernel):
                 raise ValueError(f"Expected {name}.shape {shape}, got {tuple(t.shape)}")
             if t.dtype != self.dtype:
                 raise ValueError(f"Expected {name}.dtype {self.dtype}, got {t.dtype}")
-        q, k, v, gk, state = (t.contiguous() for t in (q, k, v, gk, state))
+        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+        gk, state = gk.contiguous(), state.contiguous()
         fwd = _gla_decode_fwd_launch if _native.eager(q, k, v, gk, state) else _gla_decode_fwd
         return fwd(B, H, DK, DV, self.scale, q, k, v, gk, state)
