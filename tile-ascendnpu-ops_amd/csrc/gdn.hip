@@ -672,7 +672,8 @@ template <int NB, bool OUT, bool DEEP>
 __device__ __forceinline__ void chain_part2(f32x4 (&s)[NB][8], ChainTmp<NB>& t, const bf16* kimg,
                                             const bf16* tu11, const bf16* tu22, const bf16* l21,
                                             const bf16* aqkimg, const float* fc, bf16* orow0,
-                                            int64_t otok, int n, int col0, int g, int ln) {
+                                            int64_t otok, int n, int col0, int g, int ln,
+                                            float& gam) {
   bf16x8 wa[2], wl[2], wz[2];
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
@@ -748,6 +749,7 @@ __device__ __forceinline__ void chain_part2(f32x4 (&s)[NB][8], ChainTmp<NB>& t, 
     }
   }
   const float eg = fc[kFacEG];
+  if constexpr (!OUT) gam *= eg;
 #pragma unroll
   for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
@@ -796,7 +798,7 @@ __device__ void run_chain(const Args& A, Smem& sm, const Seg& sg, int wave, bool
   const int col0 = OUT ? 16 * NB * wave : 32 * (wave & 3);
   f32x4 s[NB][8];
   ChainTmp<NB> tmp;
-  float gam = 1.0f;  // Phi columns: the segment's decay, rounded as the state's is
+  float gam = 1.0f;  // map segments: the decay so far, rounded as the state's is
   if (!idle) {
     if (OUT) {
       // segment 0 starts from h0, segment 1 from segment 0's end state, a
@@ -848,10 +850,7 @@ __device__ void run_chain(const Args& A, Smem& sm, const Seg& sg, int wave, bool
       bf16* orow0 =
           A.o + ((int64_t)sg.b * A.T + (int64_t)cg * C) * tok_stride + (int64_t)sg.h * DV;
       chain_part2<NB, OUT, DEEP>(s, tmp, kimg, sm.tu[0], sm.tu[1], sm.l21[c & 1], sm.aqk, fc,
-                                 orow0, tok_stride, n, col0, l2 >> 4, l2 & 15);
-      if constexpr (!OUT)
-        gam = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(
-                                            __builtin_bit_cast(int, gam * fc[kFacEG])));
+                                 orow0, tok_stride, n, col0, l2 >> 4, l2 & 15, gam);
     }
     lds_barrier();
   }
